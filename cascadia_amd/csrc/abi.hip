@@ -16,7 +16,6 @@
 #include "ov.hpp"
 #include "gemv.hpp"
 #include "grouped.hpp"
-#include "prefill.hpp"
 #include "quant.hpp"
 #include "skinny.hpp"
 #include "sparse.hpp"
@@ -821,59 +820,38 @@ void expert_blob_sections(uint32_t hidden, uint32_t inter, uint32_t group, uint3
   }
 }
 
-// Which prefill kernel: prefill.hip's (K and G multiples of 128), or the
-// MFMA-tile GEMM of grouped.hip (any G of 32, 64, 128k; CASCADIA_INT4_PREFILL_TILES=1
-// takes it for every shape).
-bool prefill_tiles(const cascadia_int4_layout *L) {
-  return cai4::tuning_env("CASCADIA_INT4_PREFILL_TILES", 0) > 0 || L->group_size % 128 != 0;
-}
-
 // Prefill GEMM (M >= 64 tokens, MFMA-tiled weights).
 int run_prefill(const cascadia_int4_layout *L, const uint8_t *packed, const uint8_t *scales,
                 const uint16_t *x, uint32_t M, void *y, bool out_f32, hipStream_t st) {
   int dev;
   if (int rc = current_device(&dev)) return rc;
   if ((size_t)M * L->k_cols * 2 >= 0x7FFFFFFFu) return CASCADIA_INT4_ERR_ARG;
-  if (prefill_tiles(L)) {
-    const int cus = device_props(dev).num_cus;
-    void *ws = nullptr;
-    if (int rc = lib_workspace(
-            dev,
-            cai4::gg_dense_workspace((int)M, (int)L->n_rows, (int)L->k_cols, (int)L->group_size,
-                                     cai4::GG_A_BF16, out_f32 ? cai4::GG_F32 : cai4::GG_BF16, cus),
-            &ws, st))
-      return rc;
-    cai4::GgArgs a{};
-    a.w0 = packed;
-    a.s0 = scales;
-    a.x = x;
-    a.y = y;
-    a.M = (int)M;
-    a.N = (int)L->n_rows;
-    a.K = (int)L->k_cols;
-    a.G = (int)L->group_size;
-    a.sdt = (int)L->scale_dtype;
-    a.ldy = (int)L->n_rows;
-    a.epi = out_f32 ? cai4::GG_F32 : cai4::GG_BF16;
-    return hip_status(cai4::gg_dense(a, cai4::GG_A_BF16, ws, cus, st));
-  }
+  const int cus = device_props(dev).num_cus;
   void *ws = nullptr;
-  if (int rc = lib_workspace(dev,
-                             cai4::prefill_workspace_bytes((int)M, (int)L->n_rows, (int)L->k_cols,
-                                                           device_props(dev).num_cus),
-                             &ws, st))
+  if (int rc = lib_workspace(
+          dev,
+          cai4::gg_dense_workspace((int)M, (int)L->n_rows, (int)L->k_cols, (int)L->group_size,
+                                   cai4::GG_A_BF16, out_f32 ? cai4::GG_F32 : cai4::GG_BF16, cus),
+          &ws, st))
     return rc;
-  return hip_status(cai4::prefill_gemm(packed, scales, x, y, (int)M, (int)L->n_rows,
-                                       (int)L->k_cols, (int)L->group_size, (int)L->scale_dtype,
-                                       out_f32 ? 1 : 0, ws, device_props(dev).num_cus, st));
+  cai4::GgArgs a{};
+  a.w0 = packed;
+  a.s0 = scales;
+  a.x = x;
+  a.y = y;
+  a.M = (int)M;
+  a.N = (int)L->n_rows;
+  a.K = (int)L->k_cols;
+  a.G = (int)L->group_size;
+  a.sdt = (int)L->scale_dtype;
+  a.ldy = (int)L->n_rows;
+  a.epi = out_f32 ? cai4::GG_F32 : cai4::GG_BF16;
+  return hip_status(cai4::gg_dense(a, cai4::GG_A_BF16, ws, cus, st));
 }
 
-// Many tokens over MFMA-tiled weights: one of the prefill GEMMs.
+// Many tokens over MFMA-tiled weights: the tile GEMM (grouped.hip).
 bool prefill_shape(const cascadia_int4_layout *L, uint32_t seq) {
   if (!L->tiling || seq < 64 || L->n_rows < 16) return false;
-  if (L->group_size % 128 == 0 && !prefill_tiles(L))
-    return cai4::prefill_supported((int)seq, (int)L->n_rows, (int)L->k_cols, (int)L->group_size,
-                                   (int)L->tiling);
   return cai4::gg_supported((int)L->k_cols, (int)L->group_size, 1);
 }
 

@@ -7,34 +7,53 @@
 // element is the same sum, y = sum_g s_g * sum_{c in g} (nibble - 8) x_c, with
 // exact products and f32 accumulation.
 //
-// Arithmetic (as in prefill.hip): weights enter v_mfma_f32_16x16x32_bf16 as
-// the exact bf16 value 128 + nibble; each group's partial starts from the
-// seed -136 * sum(x) over the group's columns (computed once per row and
-// group by gg_prep) and is scaled in f32 when the group ends, acc += s * p.
-// A group of 32 or 64 columns spans one or two 32-column MFMA steps: the
-// tiled layout stores those matrices' fragments with their four dwords (one
-// 32-column segment of the 128-column k-block each, per 16-lane row)
-// transposed across the lane rows (layout.hip), so that step s holds columns
-// 32 s .. 32 s + 31 as loaded, and the activation fragment of lane row c in
-// step s is chunk 4 s + c.  Groups of 128 or more keep the untransposed order
-// (step s = chunk 4 c + s).
+// Arithmetic: weights enter v_mfma_f32_32x32x16_bf16 as the exact bf16 value
+// 128 + nibble; each group's partial starts from the seed -136 * sum(x) over
+// the group's columns (computed once per row and group by gg_prep) and is
+// scaled in f32 when the group ends, acc += s * p.  A k-block of 128 columns is
+// four sub-steps of 32: a sub-step is dword s of every weight fragment.  Groups
+// of 32 or 64 columns end with a sub-step: the tiled layout stores those
+// matrices' fragments with their four dwords transposed across the lane rows
+// (layout.hip), so that dword s holds columns 32 s .. 32 s + 31.
 //
-// Two-plane activations (hilo): the A operand is hi + lo (two bf16 planes
+// Two-plane activations (PL = 2): the A operand is hi + lo (two bf16 planes
 // whose sum carries an f32 value to 2^-16: the SwiGLU intermediate, or an f32
-// input); each step runs the MFMA on both planes with the same decoded weights.
+// input); both planes run with the same decoded weights.
 //
-// SwiGLU: a workgroup holds gate and up tiles of the same columns; each wave
-// has NT / 2 of each, and the epilogue writes hi / lo of silu(g) * u.
+// SwiGLU: each wave has 32 gate and the same 32 up columns, and the epilogue
+// writes hi / lo of silu(g) * u and, for the down projection, their seeds.
 //
 // Grouped mode: workgroup row y takes chunk y of a table written by the MoE
 // grouping -- (expert, first grouped row, rows) -- and reads expert e's
 // matrices at + e * estride.  A tile's rows past its count read zeros and are
-// not stored; M-tiles wholly past the count skip their MFMAs, so an expert
-// with few rows costs little more than streaming its weights.
+// not stored; a wave whose rows are all past it only loads and waits.
 //
-// Pipeline (as in prefill.hip): three LDS stages; every stage's activations,
-// weight tiles, scales and seeds go global -> LDS by buffer loads with an LDS
-// destination, two k-blocks ahead, issued in eight parts over the steps.
+// Bound: matrix-core and VALU issue.  Measured on the card: a 32x32x16 MFMA
+// takes 32 cycles of its SIMD's matrix core and, with two waves, about 10 of
+// the issue slots the VALU also needs (two 16x16x32 ones take 15), a VALU
+// instruction 4; so V VALU instructions per MFMA cost max(32, 10 + 4 V).  V is
+// the nibble decode (7 per fragment, shared by the NT MFMAs that use it: 3.5)
+// and the scaled adds (16 per MFMA and group: 2 at G 128, 8 at G 32), nothing
+// else: load offsets step in scalar registers, LDS offsets are immediates.  On
+// data like the weights' the power limit holds the clock at 1.9-2.1 GHz.
+//
+// Schedule: one slot per MFMA (a scheduling barrier ends it) holding that
+// MFMA's share of everything else -- half a fragment's decode, an LDS read for
+// the next sub-step, a stage load, eight scaled adds of the group before -- so
+// that a wave keeps the matrix core fed by itself and its VALU work runs in
+// the MFMAs' shadow.  Written as decode / MFMA / add blocks, the two waves of
+// a SIMD, held together by the stage barriers, ran the same phase at once.
+//
+// Pipeline: three LDS stages of one k-block; activations, weight tiles, scales
+// and seeds go global -> LDS by buffer loads with an LDS destination.  The
+// barrier that publishes stage k + 1 stands before the last sub-step of k, when
+// no wave reads stage k any more: its buffer takes the loads of k + 3, and the
+// first fragments of k + 1 are read while the last MFMAs of k run.
+//
+// Measured (M 2048, N 14336, K 4096, G 128): 264 -> 230 us against the
+// 16x16x32 kernel with block phases (3600 -> 2900 cycles per k-block; the tile
+// through LDS in 16-byte stores, 14.5k cycles of 2-byte stores before); 1024
+// tokens over 384 experts, G 32: 2.50 -> 2.07 ms a layer.
 #include "grouped.hpp"
 #include "int4_common.hpp"
 
@@ -44,251 +63,143 @@ namespace {
 
 typedef __amdgpu_buffer_rsrc_t rsrc_t;
 typedef __attribute__((address_space(3))) void lds_void;
+typedef float f32x16_t __attribute__((ext_vector_type(16)));
 
 CAI4_DEV rsrc_t rsrc(const void *base, size_t bytes) {
   const int n = bytes > 0x7FFFFFFFu ? 0x7FFFFFFF : (int)bytes;
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(base), (short)0, n, 0x00020000);
 }
 
-template <int n>
-CAI4_DEV void gg_wait_barrier() {
-  asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(n) : "memory");
+// The same with the (wave-uniform) base and size forced into scalar registers.
+CAI4_DEV rsrc_t rsrc_scalar(const void *base, size_t bytes) {
+  const uint64_t b = (uint64_t)base;
+  // (readfirstlane returns int: without the cast its sign would fill the high half)
+  const uint64_t u = (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)b) |
+                     (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)(b >> 32)) << 32;
+  const int n = __builtin_amdgcn_readfirstlane(bytes > 0x7FFFFFFFu ? 0x7FFFFFFF : (int)bytes);
+  return __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<void *>(u), (short)0, n, 0x00020000);
 }
 
-CAI4_DEV uint32_t lds_addr(const uint8_t *p) {
-  return __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(const lds_void *)p);
+// Wait until at most n of this wave's vector-memory loads are outstanding and
+// its LDS reads have returned, then barrier.  Inline asm with a memory
+// clobber: neither LDS reads nor the LDS-destination loads move across it.
+template <int n>
+CAI4_DEV void gg_wait_barrier() {
+  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(n) : "memory");
 }
 
 // One global -> LDS buffer load (16 or 4 bytes per lane, lane i at M0 +
-// bytes * i).  Inline asm: the compiler cannot tell the stage buffers apart
-// and would make LDS reads of any stage wait for the newest prefetch.
+// bytes * i) from byte voff + soff.  Inline asm: the compiler cannot tell the
+// stage buffers apart and would make LDS reads of any stage wait for the
+// newest prefetch.  A lane's row limit is in voff (soff only steps along K).
 template <int bytes>
-CAI4_DEV void gg_dma(rsrc_t r, uint32_t lds, uint32_t voff) {
+CAI4_DEV void gg_dma(rsrc_t r, uint32_t lds, uint32_t voff, uint32_t soff) {
   if constexpr (bytes == 16)
-    asm volatile("buffer_load_dwordx4 %1, %2, 0 offen lds" ::"{m0}"(lds), "v"(voff), "s"(r)
+    asm volatile("buffer_load_dwordx4 %1, %2, %3 offen lds" ::"{m0}"(lds), "v"(voff), "s"(r),
+                 "s"(soff)
                  : "memory");
   else
-    asm volatile("buffer_load_dword %1, %2, 0 offen lds" ::"{m0}"(lds), "v"(voff), "s"(r)
+    asm volatile("buffer_load_dword %1, %2, %3 offen lds" ::"{m0}"(lds), "v"(voff), "s"(r),
+                 "s"(soff)
                  : "memory");
 }
 
-// Workgroup geometry and the LDS of one stage: activations [PL][BM][256 B]
-// (XOR-swizzled 16-byte chunks), weight tiles [NT16][1 KB], scales
-// [NT16][GPK][16] u16, seeds [GPK][BM] f32.
-template <int MS, int NT, int WM, int WN, int GPK, bool HILO, bool SW>
+CAI4_DEV f32x16_t mfma32_bf16(u32x4_t a, u32x4_t b, f32x16_t c) {
+  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, a),
+                                                 __builtin_bit_cast(bf16x8_t, b), c, 0, 0, 0);
+}
+
+// Workgroup geometry (WM x WN waves of 32 MT rows x 64 columns, PL activation
+// planes, GPK scale groups per 128-column k-block) and the LDS of one stage:
+// activations [PL][BM][256 B] (16-byte chunk c of row r at slot c ^ (r & 15)),
+// weight tiles [NT16][1 KB], then 256-byte pieces of scales [NT16][GPK][16] u16
+// and seeds [GPK][BM] f32, MPW pieces per wave (the last ones spare: every
+// wave issues the same number of loads, the stage waits count them).
+template <int MT, int WM, int WN, int GPK, int PL, bool SW>
 struct Gg {
   static constexpr int W = WM * WN;
-  static constexpr int PL = HILO ? 2 : 1;
-  static constexpr int BM = 16 * MS * WM, BN = 16 * NT * WN;
-  static constexpr int RM = 16 * MS;
-  static constexpr int NT16 = NT * WN;                 // weight tiles per stage
+  static constexpr int RM = 32 * MT, BM = RM * WM, BN = 64 * WN;
+  static constexpr int NT16 = BN / 16;                 // weight tiles per stage
   static constexpr int OUTC = SW ? BN / 2 : BN;        // output columns per workgroup
-  static constexpr int A = 0, B = PL * BM * 256, S = B + NT16 * 1024, X = S + NT16 * 32 * GPK,
-                       BYTES = X + BM * 4 * GPK;
+  static constexpr int SLD = NT16 * GPK / 8, XLD = GPK * BM / 64;  // 256-byte pieces
+  static constexpr int MPW = (SLD + XLD + W - 1) / W;
+  static constexpr int A = 0, B = PL * BM * 256, S = B + NT16 * 1024, X = S + SLD * 256,
+                       BYTES = S + MPW * W * 256;
   static constexpr int AL = PL * BM / (4 * W);         // 1 KB activation loads per wave
   static constexpr int BL = NT16 / W;                  // weight tiles per wave
-  static constexpr int SLANES = NT16 * 8 * GPK / W;    // 4-byte scale lanes per wave
-  static constexpr int SLD = (SLANES + 63) / 64;
-  static constexpr int XLANES = GPK * BM / (4 * W);    // 16-byte seed lanes per wave
-  static constexpr int LOADS = AL + BL + SLD + 1;
-  static_assert(AL >= 1 && BL >= 1 && XLANES >= 1 && XLANES <= 64, "workgroup shape");
-  static_assert(SLANES < 64 || SLANES % 64 == 0, "scale lanes");
-  static_assert(!SW || (W % 2 == 0 && NT % 2 == 0 && (NT16 / 2) % BL == 0), "SwiGLU shape");
+  static constexpr int LOADS = AL + BL + MPW;
+  static constexpr int NT = MT * PL;                   // A fragments per 16-column step
+  static constexpr int SLOTS = 4 * NT;                 // MFMAs per 32-column sub-step
+  static_assert(AL >= 1 && BL >= 1 && SLD >= 1 && XLD >= 1, "workgroup shape");
+  static_assert(NT == 1 || NT == 2, "fragments per step");
+  static_assert(!SW || (W % 2 == 0 && SLD % 2 == 0), "SwiGLU shape");
   static_assert(3 * BYTES <= 160 * 1024, "LDS");
 };
 
+// Keeps these values' computation in its slot: the instruction selector orders
+// arithmetic freely between scheduling barriers unless something there uses it.
+CAI4_DEV void gg_pin(float &a, float &b, float &c, float &d, float &e, float &f, float &g,
+                     float &h) {
+#ifdef __HIP_DEVICE_COMPILE__
+  asm volatile("" : "+v"(a), "+v"(b), "+v"(c), "+v"(d), "+v"(e), "+v"(f), "+v"(g), "+v"(h));
+#endif
+}
+
+// A read of LDS at byte address at + off.  The constant off is a pointer step,
+// not integer arithmetic, so that it becomes the instruction's offset.
+template <class T>
+CAI4_DEV T lds_at(uint32_t at, int off) {
+  typedef const __attribute__((address_space(3))) uint8_t *bytes_t;
+  return *reinterpret_cast<const __attribute__((address_space(3))) T *>(
+      reinterpret_cast<bytes_t>(at) + off);
+}
+
 constexpr uint32_t kGgOOB = 0x80000000u;  // an offset past every range: no data moves
 
-// What a wave's loads of a k-block read: its rsrcs (the weight / scale ones
-// are the wave's own matrix in SwiGLU mode) and geometry.
-struct GgLd {
-  rsrc_t xr0, xr1, wr, sr, qr;
-  int K, KB, NG, G, Rp, wave, lane, half;  // half: SwiGLU, the wave loads up tiles
-  int mrows;  // live rows of the tile
-  // rows through a row map (GgArgs::row_map): each A load's byte offset at
-  // k-block 0 (its x row and chunk; kGgOOB for a row past the count) and the
-  // seed lane's (one x row and group per lane, 4 bytes)
-  int ind;
-  uint32_t aoff[4], soff;
-};
+struct GgTrue { static constexpr bool value = true; };
+struct GgFalse { static constexpr bool value = false; };
 
-template <class P, int GPK, bool SW>
-CAI4_DEV void gg_load(int l, uint8_t *buf, const GgLd &d, int kb) {
-  const int lane = d.lane;
-  if (l < P::AL) {
-    const int blk = d.wave * P::AL + l;
-    const int pl = blk / (P::BM / 4), rb = blk - pl * (P::BM / 4);
-    const int row = 4 * rb + (lane >> 4);
-    const int q = (lane & 15) ^ (row & 15);
-    if (4 * rb < d.mrows)
-      gg_dma<16>(P::PL > 1 && pl ? d.xr1 : d.xr0, lds_addr(buf + P::A + blk * 1024),
-                 d.ind ? d.aoff[l < 4 ? l : 0] + (uint32_t)kb * 256
-                       : (uint32_t)(row * d.K + kb * 128 + 8 * q) * 2);
-    else if (lane == 0)
-      // a block of dead rows (past the tile's count, never stored): one 4-byte
-      // load instead, so that every stage issues the same number of loads (the
-      // stage waits count them)
-      gg_dma<4>(d.xr0, lds_addr(buf + P::A + blk * 1024), 0);
-  } else if (l < P::AL + P::BL) {
-    const int tile = d.wave * P::BL + (l - P::AL);
-    const int mt = SW && d.half ? tile - P::NT16 / 2 : tile;  // tile within its matrix
-    gg_dma<16>(d.wr, lds_addr(buf + P::B + tile * 1024),
-               (uint32_t)(mt * d.KB + kb) * 1024 + 16 * lane);
-  } else if (l < P::AL + P::BL + P::SLD) {
-    // scales: the wave's BL tiles, 32 GPK bytes each, 4 bytes per lane; lanes
-    // past SLANES must not run (they would write the next wave's slots)
-    const int i = (l - P::AL - P::BL) * 64 + lane;
-    const int tile = d.wave * P::BL + i / (8 * GPK), j = i % (8 * GPK);
-    const int mt = SW && d.half ? tile - P::NT16 / 2 : tile;
-    const int g0 = (kb * 128) / d.G;
-    if (i < P::SLANES)
-      gg_dma<4>(d.sr, lds_addr(buf + P::S + (d.wave * P::SLANES + (i & ~63)) * 4),
-                (uint32_t)((mt * d.NG + g0) * 32 + 4 * j));
-  } else if (d.ind) {
-    // seeds through the row map: one row of one group per lane
-    constexpr int XL4 = GPK * P::BM / P::W;
-    if (lane < XL4)
-      gg_dma<4>(d.qr, lds_addr(buf + P::X + d.wave * XL4 * 4),
-                d.soff + (uint32_t)(kb * GPK * d.Rp) * 4);
-  } else {
-    // seeds: 4 rows of one group per lane
-    if (lane < P::XLANES) {
-      const int idx = d.wave * P::XLANES + lane;
-      const int g = idx / (P::BM / 4), rq = idx - g * (P::BM / 4);
-      gg_dma<16>(d.qr, lds_addr(buf + P::X + d.wave * P::XLANES * 16),
-                 (uint32_t)((kb * GPK + g) * d.Rp + 4 * rq) * 4);
+// Sum over groups of L consecutive lanes (L = 4, 8, 16 within a DPP row):
+// quad sums, then a half-row mirror (lane i <- 7 - i of its 8 lanes: the other
+// quad of the same half), then a row mirror (the other half).
+template <int L>
+CAI4_DEV float lane_group_sum(float t) {
+  t += dpp_f32<0xB1>(t);                          // quad_perm 1,0,3,2
+  t += dpp_f32<0x4E>(t);                          // quad_perm 2,3,0,1
+  if constexpr (L >= 8) t += dpp_f32<0x141>(t);   // row_half_mirror
+  if constexpr (L >= 16) t += dpp_f32<0x140>(t);  // row_mirror
+  return t;
+}
+
+// A [BM][OUTC] u16 tile from LDS (row pitch `pitch` bytes) to rows row0.. of
+// dst [., ldy], columns col0..: 16 bytes per thread where dst allows it.
+template <int OUTC>
+CAI4_DEV void gg_store_tile(const uint8_t *lds, int pitch, uint16_t *dst, size_t row0, int mrows,
+                            int col0, int N, int ldy, int tid, int nth) {
+  const bool wide = (ldy & 7) == 0 && ((uintptr_t)dst & 15) == 0;
+  for (int c = tid; c < mrows * (OUTC / 8); c += nth) {
+    const int row = c / (OUTC / 8), col = 8 * (c - row * (OUTC / 8));
+    const u32x4_t v = *reinterpret_cast<const u32x4_t *>(lds + row * pitch + col * 2);
+    const int n = col0 + col;
+    if (n >= N) continue;
+    uint16_t *p = dst + (row0 + row) * (size_t)ldy + n;
+    if (wide && n + 8 <= N) {
+      *reinterpret_cast<u32x4_t *>(p) = v;
+    } else {
+#pragma unroll
+      for (int e = 0; e < 8; ++e)
+        if (n + e < N) p[e] = (uint16_t)(v[e >> 1] >> (16 * (e & 1)));
     }
   }
 }
 
-struct GgNext {
-  uint8_t *buf;
-  GgLd d;
-  int kb, KE;
-};
-
-template <class P, int GPK, bool SW>
-CAI4_DEV void gg_issue_part(const GgNext &n, int part) {
-  if (n.kb < n.KE) {
-#pragma unroll
-    for (int l = 0; l < P::LOADS; ++l)
-      if (l >= part * P::LOADS / 8 && l < (part + 1) * P::LOADS / 8)
-        gg_load<P, GPK, SW>(l, n.buf, n.d, n.kb);
-  }
-  __builtin_amdgcn_sched_barrier(0);
-}
-
-// Activation fragments of step s for the MS M-tiles (and the lo plane).
-template <class P, int MS, int GPK>
-CAI4_DEV void gg_read_a(const uint8_t *buf, int wm, int lane, int s, u32x4_t (&af)[P::PL][MS]) {
-  const int lr = lane & 15, lg = lane >> 4;
-  const int chunk = GPK > 1 ? 4 * s + lg : 4 * lg + s;
-#pragma unroll
-  for (int p = 0; p < P::PL; ++p)
-#pragma unroll
-    for (int i = 0; i < MS; ++i) {
-      const int row = wm * P::RM + 16 * i + lr;  // row & 15 == lr
-      af[p][i] = *reinterpret_cast<const u32x4_t *>(buf + P::A + p * P::BM * 256 + row * 256 +
-                                                    16 * (chunk ^ lr));
-    }
-}
-
-// LDS tile index of the wave's j-th weight tile.
-template <class P, int NT, bool SW>
-CAI4_DEV int gg_tile(int wn, int j) {
-  if constexpr (SW)
-    return j < NT / 2 ? wn * (NT / 2) + j : P::NT16 / 2 + wn * (NT / 2) + (j - NT / 2);
-  else
-    return NT * wn + j;
-}
-
-template <class P, int MS, int NT, int GPK, bool HILO, bool SW>
-CAI4_DEV void gg_compute(const uint8_t *buf, int wm, int wn, int lane, int sdt, int mt_live,
-                         const GgNext &nx, f32x4_t (&acc)[MS][NT]) {
-  constexpr int SPG = 4 / GPK;  // MFMA steps per group
-  const int lr = lane & 15, lg = lane >> 4;
-  u32x4_t b[NT];
-  float sc[GPK][NT];
-#pragma unroll
-  for (int j = 0; j < NT; ++j) {
-    const int tile = gg_tile<P, NT, SW>(wn, j);
-    b[j] = *reinterpret_cast<const u32x4_t *>(buf + P::B + tile * 1024 + 16 * lane);
-#pragma unroll
-    for (int g = 0; g < GPK; ++g) {
-      const uint32_t bits =
-          *reinterpret_cast<const uint16_t *>(buf + P::S + tile * 32 * GPK + g * 32 + 2 * lr);
-      sc[g][j] = scale_bits_f32(bits, sdt);
-    }
-  }
-  f32x4_t p[MS][NT];
-  u32x4_t af[P::PL][MS], an[P::PL][MS];
-  gg_read_a<P, MS, GPK>(buf, wm, lane, 0, af);
-  f32x4_t seed[MS];
-#pragma unroll
-  for (int s = 0; s < 4; ++s) {
-    const int g = s / SPG;
-    const bool first = s % SPG == 0, last = s % SPG == SPG - 1;
-    if (first) {
-#pragma unroll
-      for (int i = 0; i < MS; ++i)
-        // D layout: lane holds rows 4 (lane / 16) + v of the 16-row tile
-        seed[i] = *reinterpret_cast<const f32x4_t *>(
-            buf + P::X + 4 * (g * P::BM + wm * P::RM + 16 * i + 4 * lg));
-    }
-    if (s < 3) gg_read_a<P, MS, GPK>(buf, wm, lane, s + 1, an);
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      u32x4_t d[NT / 2];
-#pragma unroll
-      for (int j = 0; j < NT / 2; ++j) d[j] = decode8(b[h * NT / 2 + j][s]);
-      __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int j = 0; j < NT / 2; ++j)
-#pragma unroll
-        for (int i = 0; i < MS; ++i) {
-          if (i >= mt_live) continue;  // uniform: M-tile past the rows
-          f32x4_t c = first ? seed[i] : p[i][h * NT / 2 + j];  // NOLINT
-          c = mfma_bf16(af[0][i], d[j], c);
-          if constexpr (HILO) c = mfma_bf16(af[1][i], d[j], c);
-          p[i][h * NT / 2 + j] = c;
-        }
-      __builtin_amdgcn_sched_barrier(0);
-      gg_issue_part<P, GPK, SW>(nx, 2 * s + h);
-    }
-    if (last) {
-#pragma unroll
-      for (int i = 0; i < MS; ++i) {
-        if (i >= mt_live) continue;
-#pragma unroll
-        for (int j = 0; j < NT; ++j) acc[i][j] += sc[g][j] * p[i][j];
-      }
-    }
-#pragma unroll
-    for (int q = 0; q < P::PL; ++q)
-#pragma unroll
-      for (int i = 0; i < MS; ++i) af[q][i] = an[q][i];
-  }
-}
-
-template <class P, int MS, int NT, int GPK, bool HILO, bool SW>
-CAI4_DEV void gg_stage(uint8_t *cur, uint8_t *nxt2, const GgLd &d, int kb, int KE, int wm, int wn,
-                       int sdt, int mt_live, f32x4_t (&acc)[MS][NT]) {
-  if (kb >= KE) return;  // uniform
-  if (kb + 1 < KE)
-    gg_wait_barrier<P::LOADS>();
-  else
-    gg_wait_barrier<0>();
-  const GgNext nx{nxt2, d, kb + 2, KE};
-  gg_compute<P, MS, NT, GPK, HILO, SW>(cur, wm, wn, d.lane, sdt, mt_live, nx, acc);
-}
-
-// SDT: the scale dtype (a.sdt) as a constant, so that each scale's f32
-// conversion is one instruction in the k-loop.
-template <int MS, int NT, int WM, int WN, int GPK, bool HILO, bool SW, int SDT>
-__global__ __launch_bounds__(64 * WM * WN) void gg_kernel(GgArgs a) {
-  using P = Gg<MS, NT, WM, WN, GPK, HILO, SW>;
-  __shared__ __attribute__((aligned(16))) uint8_t stages[3 * P::BYTES];
-  const int tid = threadIdx.x, lane = tid & 63, lr = lane & 15, lg = lane >> 4;
+// SDT: the scale dtype (a.sdt) as a constant.
+template <int MT, int WM, int WN, int GPK, int PL, bool SW, int SDT>
+__global__ __launch_bounds__(64 * WM * WN, 2) void gg_kernel(GgArgs a) {
+  using P = Gg<MT, WM, WN, GPK, PL, SW>;
+  __shared__ __attribute__((aligned(256))) uint8_t st[3 * P::BYTES];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int h = lane >> 5, l15 = lane & 15, l31 = lane & 31, t16 = (lane >> 4) & 1;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), wm = wave % WM, wn = wave / WM;
   // this workgroup's rows
   int e = 0, row0, mrows;
@@ -307,163 +218,394 @@ __global__ __launch_bounds__(64 * WM * WN) void gg_kernel(GgArgs a) {
   e = __builtin_amdgcn_readfirstlane(e);
   row0 = __builtin_amdgcn_readfirstlane(row0);
   mrows = __builtin_amdgcn_readfirstlane(mrows);
-  const int live = mrows - wm * P::RM;
-  const int mt_live = live <= 0 ? 0 : (live + 15) >> 4;  // this wave's M-tiles holding rows
-  const int KB = a.K >> 7, NG = a.K / a.G;
+  const int KB = a.K >> 7, NG = a.K / a.G, KPG = GPK > 1 ? 1 : a.G >> 7;
   const int ntiles = (a.N + 15) >> 4;
   const int T0 = blockIdx.x * (P::OUTC / 16);
   constexpr int TM = SW ? P::NT16 / 2 : P::NT16;  // tiles per matrix per workgroup
   const int tv = __builtin_amdgcn_readfirstlane(ntiles - T0 > TM ? TM : ntiles - T0);
   const size_t eo = (size_t)e * a.estride;
-  const int half = SW ? (wave >= P::W / 2 ? 1 : 0) : 0;
-  const uint8_t *wm0 = half ? a.w1 : a.w0, *sm0 = half ? a.s1 : a.s0;
-  GgLd d;
-  d.wr = rsrc(wm0 + eo + (size_t)T0 * KB * 1024, (size_t)tv * KB * 1024);
-  d.sr = rsrc(sm0 + eo + (size_t)T0 * NG * 32, (size_t)tv * NG * 32);
-  d.xr0 = rsrc(a.x + (size_t)row0 * a.K, (size_t)mrows * a.K * 2);
-  d.xr1 = rsrc(HILO ? a.x2 + (size_t)row0 * a.K : a.x, HILO ? (size_t)mrows * a.K * 2 : 0);
-  d.qr = rsrc(a.seeds + row0, ((size_t)(KB * GPK - 1) * a.rows_pad + P::BM) * 4);
-  d.K = a.K;
-  d.KB = KB;
-  d.NG = NG;
-  d.G = a.G;
-  d.Rp = a.rows_pad;
-  d.wave = wave;
-  d.lane = lane;
-  d.half = half;
-  d.mrows = mrows;
-  d.ind = 0;
-  // rows through a row map: the grouped one-plane shapes only (gg_grouped
-  // refuses the others); uniform
-  if constexpr (!HILO && P::AL <= 4 && GPK * P::BM / P::W <= 64) {
-    if (a.row_map) {
-      d.ind = 1;
-      d.xr0 = rsrc(a.x, (size_t)a.x_rows * a.K * 2);
-      d.qr = rsrc(a.seeds, (size_t)KB * GPK * a.rows_pad * 4);
+  const size_t wo = eo + (size_t)T0 * KB * 1024, so = eo + (size_t)T0 * NG * 32;
+  const size_t wbytes = (size_t)tv * KB * 1024, sbytes = (size_t)tv * NG * 32;
+  const uint32_t lds0 = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(const lds_void *)st);
+
+  // ---- this wave's loads of a stage: descriptors and per-lane offsets ----
+  const bool up = SW && wave >= P::W / 2;  // SwiGLU: the upper waves load up's tiles
+  const rsrc_t wr = rsrc_scalar((up ? a.w1 : a.w0) + wo, wbytes);
+  rsrc_t xr0 = rsrc(a.x + (size_t)row0 * a.K, (size_t)mrows * a.K * 2);
+  const rsrc_t xr1 = rsrc(PL == 2 ? a.x2 + (size_t)row0 * a.K : a.x,
+                          PL == 2 ? (size_t)mrows * a.K * 2 : 0);
+  const bool ind = PL == 1 && a.row_map != nullptr;  // rows through a row map
+  if (ind) xr0 = rsrc(a.x, (size_t)a.x_rows * a.K * 2);
+  uint32_t va[P::AL], vb[P::BL], vm[P::MPW];
 #pragma unroll
-      for (int l = 0; l < 4; ++l) {
-        const int blk = wave * P::AL + l, rb = blk % (P::BM / 4);
-        const int row = 4 * rb + (lane >> 4), q = (lane & 15) ^ (row & 15);
-        d.aoff[l] = l < P::AL && row < mrows
-                        ? (uint32_t)(((size_t)a.row_map[row0 + row] * a.K + 8 * q) * 2)
-                        : kGgOOB;
-      }
-      constexpr int XL4 = GPK * P::BM / P::W;
-      const int idx = wave * XL4 + lane, g = idx / P::BM, rq = idx - g * P::BM;
-      d.soff = lane < XL4 && rq < mrows
-                   ? (uint32_t)(((size_t)g * a.rows_pad + a.row_map[row0 + rq]) * 4)
-                   : kGgOOB;
-    }
+  for (int l = 0; l < P::AL; ++l) {
+    const int blk = wave * P::AL + l, rb = blk % (P::BM / 4);
+    const int row = 4 * rb + (lane >> 4), q = l15 ^ (row & 15);
+    if (ind)
+      va[l] = row < mrows ? (uint32_t)(((size_t)a.row_map[row0 + row] * a.K + 8 * q) * 2) : kGgOOB;
+    else
+      va[l] = row < mrows ? (uint32_t)(row * a.K + 8 * q) * 2 : kGgOOB;
   }
-
-  f32x4_t acc[MS][NT];
 #pragma unroll
-  for (int i = 0; i < MS; ++i)
+  for (int l = 0; l < P::BL; ++l) {
+    const int tile = wave * P::BL + l - (up ? P::NT16 / 2 : 0);
+    vb[l] = (uint32_t)(tile * KB) * 1024 + 16 * lane;
+  }
+  // pieces m = wave, wave + W, ...: scales (8 / GPK tiles' 32 GPK bytes), seeds, spare
+  rsrc_t mr[P::MPW];
+  bool mx[P::MPW];
 #pragma unroll
-    for (int j = 0; j < NT; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-
+  for (int k = 0; k < P::MPW; ++k) {
+    const int m = wave + k * P::W, mm = m < P::SLD + P::XLD ? m : m - P::SLD - P::XLD;
+    mx[k] = mm >= P::SLD;
+    const bool u = SW && mm >= P::SLD / 2;
+    const void *mb = (u ? a.s1 : a.s0) + so;
+    size_t ms = sbytes;
+    if (!mx[k]) {
+      const int lane_tile = mm * (8 / GPK) + lane / (8 * GPK), j = lane % (8 * GPK);
+      vm[k] = (uint32_t)((lane_tile - (u ? P::NT16 / 2 : 0)) * NG * 32 + 4 * j);
+    } else {
+      const int idx = (mm - P::SLD) * 64 + lane, g = idx / P::BM, r = idx - g * P::BM;
+      mb = ind ? a.seeds : a.seeds + row0;
+      ms = ((size_t)KB * GPK * a.rows_pad - (ind ? 0 : row0)) * 4;
+      vm[k] = r < mrows ? (uint32_t)(((size_t)g * a.rows_pad + (ind ? a.row_map[row0 + r] : r)) * 4)
+                        : kGgOOB;
+    }
+    mr[k] = rsrc_scalar(mb, ms);
+  }
+  // load l of this wave for k-block kb (scale group row g = first group of kb)
+  auto issue1 = [&](int l, int buf, int kb, int g) {
+    const uint32_t L = lds0 + buf * P::BYTES;
+    if (l < P::AL) {
+      const int blk = wave * P::AL + l;
+      gg_dma<16>(PL == 2 && blk >= P::BM / 4 ? xr1 : xr0, L + P::A + blk * 1024, va[l < P::AL ? l : 0],
+                 (uint32_t)kb * 256);
+    } else if (l < P::AL + P::BL) {
+      const int t = l - P::AL;
+      gg_dma<16>(wr, L + P::B + (wave * P::BL + t) * 1024, vb[t < P::BL ? t : 0],
+                 (uint32_t)kb * 1024);
+    } else {
+      const int k = l - P::AL - P::BL < P::MPW ? l - P::AL - P::BL : 0;
+      gg_dma<4>(mr[k], L + P::S + (wave + k * P::W) * 256, vm[k],
+                mx[k] ? (uint32_t)(kb * GPK * a.rows_pad) * 4 : (uint32_t)g * 32);
+    }
+  };
   const int kb0 = blockIdx.z * a.kper, KE = min(KB, kb0 + a.kper);
 #pragma unroll
-  for (int l = 0; l < P::LOADS; ++l) gg_load<P, GPK, SW>(l, stages, d, kb0);
-  if (kb0 + 1 < KE) {
+  for (int s = 0; s < 3; ++s)
+    if (kb0 + s < KE) {
 #pragma unroll
-    for (int l = 0; l < P::LOADS; ++l) gg_load<P, GPK, SW>(l, stages + P::BYTES, d, kb0 + 1);
-  }
-  // one stage per iteration, not unrolled: the stage buffers rotate at run
-  // time, so the compiler cannot hoist one stage's work into another's
-  int cur = 0;
-#pragma unroll 1
-  for (int kb = kb0; kb < KE; ++kb) {
-    const int nx2 = cur == 0 ? 2 : cur - 1;  // (cur + 2) % 3
-    gg_stage<P, MS, NT, GPK, HILO, SW>(stages + cur * P::BYTES, stages + nx2 * P::BYTES, d, kb,
-                                       KE, wm, wn, SDT, mt_live, acc);
-    cur = cur == 2 ? 0 : cur + 1;
-  }
+      for (int l = 0; l < P::LOADS; ++l)
+        issue1(l, s, kb0 + s, GPK > 1 ? (kb0 + s) * GPK : (kb0 + s) / KPG);
+    }
 
-  // epilogue: D lane l holds column l % 16 and rows 4 (l / 16) + v
-  constexpr int NOUT = SW ? NT / 2 : NT;
-  // SwiGLU: this lane's sum of hi + lo over its NOUT columns, per row
-  float rsum[SW ? MS : 1][4];
+  // ---- LDS read offsets within a stage ----
+  // A row 32 i + l31; the fragment of sub-step s, step q: chunk (GPK 1: 4 (2 q + h)
+  // + s; else 4 s + 2 q + h) ^ (row & 15); rows and stages are 256-byte aligned,
+  // so the constant part of the chunk is one XOR of the address
+  const uint32_t ax = lds0 + P::A + (uint32_t)(wm * P::RM + l31) * 256 +
+                      16 * ((GPK == 1 ? 4 * h : h) ^ l15);
+  // B: tile (4 wn + 2 j + t16; SwiGLU: 2 wn + t16 of gate, of up), chunk 2 q + h, row l15
+  constexpr int JT = SW ? P::NT16 / 2 : 2;  // tiles between j = 0 and j = 1
+  const int bt = (SW ? 2 : 4) * wn + t16;
+  const uint32_t bx = lds0 + P::B + (uint32_t)bt * 1024 + h * 256 + l15 * 16;
+  const uint32_t sx = lds0 + P::S + (uint32_t)bt * 32 * GPK + l15 * 2;
+  const uint32_t xx = lds0 + P::X + (uint32_t)(wm * P::RM + 4 * h) * 4;
+
+  float acc[MT][2][16];
+  f32x16_t p[MT][2], seed[MT];
 #pragma unroll
-  for (int i = 0; i < (SW ? MS : 1); ++i)
+  for (int i = 0; i < MT; ++i)
 #pragma unroll
-    for (int v = 0; v < 4; ++v) rsum[i][v] = 0.f;
+    for (int j = 0; j < 2; ++j)
 #pragma unroll
-  for (int i = 0; i < MS; ++i) {
+      for (int v = 0; v < 16; ++v) acc[i][j][v] = p[i][j][v] = 0.f;
+  u32x4_t af[2][P::NT][2], b[2][2], d[PL == 2 ? 4 : 2];
+  uint32_t dx = 0, dy = 0;
+  uint32_t su[2], sn[2];            // scale bits of the group in flight, of the next
+  float sc[2] = {0.f, 0.f};         // scales of the group being added
+  uint32_t base = 0, nbase = 0;  // byte offsets of this k-block's stage and the next
+  auto read_a1 = [&](uint32_t from, int s, int buf, int r) {  // fragment r = q NT + t
+    const int q = r / P::NT, t = r % P::NT;
+    const uint32_t at = (ax + from) ^ (16 * (GPK == 1 ? 8 * q + s : 4 * s + 2 * q));
+    af[buf][t][q] = lds_at<u32x4_t>(at, t * (PL == 2 ? P::BM * 256 : 32 * 256));
+  };
+  auto read_b1 = [&](uint32_t from, int f) {  // fragment f = 2 q + j
+    b[f & 1][f >> 1] = lds_at<u32x4_t>(from + bx, (f & 1) * JT * 1024 + (f >> 1) * 512);
+  };
+  auto read_seed1 = [&](uint32_t from, int g, int r) {  // rows 32 (r / 4) + 8 (r % 4) ..
+    const f32x4_t t = lds_at<f32x4_t>(from + xx, g * P::BM * 4 + (32 * (r >> 2) + 8 * (r & 3)) * 4);
 #pragma unroll
-    for (int j = 0; j < NOUT; ++j) {
-      const int n = T0 * 16 + 16 * (SW ? wn * (NT / 2) + j : NT * wn + j) + lr;
-      if (n >= a.N) continue;
+    for (int v = 0; v < 4; ++v) seed[r >> 2][4 * (r & 3) + v] = t[v];
+  };
+  auto read_scale = [&](uint32_t from, int g, int j) -> uint32_t {
+    return lds_at<uint16_t>(from + sx, j * JT * 32 * GPK + g * 32);
+  };
+  // eight scaled adds: acc += s * p, half `c & 1` of tile (i, j)
+  auto add8 = [&](int c) {
+    const int i = MT == 2 ? (c >> 1) & 1 : 0, j = MT == 2 ? c >> 2 : c >> 1;
 #pragma unroll
-      for (int v = 0; v < 4; ++v) {
-        const int m = wm * P::RM + 16 * i + 4 * lg + v;
-        if (m >= mrows) continue;
-        const size_t o = (size_t)(row0 + m) * a.ldy + n;
-        const float y = acc[i][j][v];
-        if constexpr (SW) {
-          const float h = silu_f32(y) * acc[i][j + NT / 2][v];
-          const uint32_t hb = fbits(h) >> 16;  // hi = h truncated, lo = RNE(h - hi)
-          const uint32_t lb = f32_to_bf16_rne(h - bitsf(hb << 16));
-          reinterpret_cast<uint16_t *>(a.y)[o] = (uint16_t)hb;
-          reinterpret_cast<uint16_t *>(a.y2)[o] = (uint16_t)lb;
-          rsum[SW ? i : 0][v] += bitsf(hb << 16) + bf16_to_f32(lb);
-        } else if (a.part) {
-          a.part[(size_t)blockIdx.z * a.M * a.N + (size_t)(row0 + m) * a.N + n] = y;
-        } else if (a.epi == GG_F32) {
-          reinterpret_cast<float *>(a.y)[o] = y;
-        } else {
-          reinterpret_cast<uint16_t *>(a.y)[o] = (uint16_t)f32_to_bf16_rne(y);
+    for (int v = 0; v < 8; ++v) acc[i][j][8 * (c & 1) + v] += sc[j] * p[i][j][8 * (c & 1) + v];
+    float *o = &acc[i][j][8 * (c & 1)];
+    gg_pin(o[0], o[1], o[2], o[3], o[4], o[5], o[6], o[7]);
+  };
+
+  if (kb0 + 2 < KE)
+    gg_wait_barrier<2 * P::LOADS>();
+  else if (kb0 + 1 < KE)
+    gg_wait_barrier<P::LOADS>();
+  else
+    gg_wait_barrier<0>();
+  int cur = 0;
+
+  if (wm * P::RM < mrows) {
+#pragma unroll
+    for (int r = 0; r < 2 * P::NT; ++r) read_a1(0, 0, 0, r);
+#pragma unroll
+    for (int f = 0; f < 4; ++f) read_b1(0, f);
+#pragma unroll
+    for (int r = 0; r < 4 * MT; ++r) read_seed1(0, 0, r);
+    sn[0] = read_scale(0, 0, 0);
+    sn[1] = read_scale(0, 0, 1);
+    // fragments decoded before the first slot: one ahead of their use (PL 2: two)
+    d[0] = decode8(b[0][0][0]);
+    if (PL == 2) d[1] = decode8(b[1][0][0]);
+
+    // One k-block.  Slot n of a sub-step issues one MFMA and the work beside
+    // it: half a weight fragment's decode (one or two fragments ahead), an LDS
+    // read for the next sub-step, a stage load, eight of the last group's
+    // scaled adds.  A scheduling barrier ends every slot.
+    auto kblock = [&](auto dma_tag, int kb, int g3) {
+      constexpr bool DMA = decltype(dma_tag)::value;
+      base = cur * P::BYTES;
+      const int nxt = cur == 2 ? 0 : cur + 1;
+      nbase = nxt * P::BYTES;
+#pragma unroll
+      for (int s = 0; s < 4; ++s) {
+        constexpr int SPG = 4 / GPK;  // sub-steps per group
+        const bool first = s % SPG == 0, last = s % SPG == SPG - 1;
+        const int g = s / SPG;
+#pragma unroll
+        for (int n = 0; n < P::SLOTS; ++n) {
+          constexpr int NT = P::NT, SL = P::SLOTS;
+          const int q = n / (2 * NT);
+          const int t = MT == 2 ? n & 1 : PL == 2 ? (n >> 1) & 1 : 0;
+          const int j = MT == 2 ? (n >> 1) & 1 : n & 1;
+          const int i = MT == 2 ? t : 0;
+          if (s == 3 && n == 0) {
+            if (DMA)
+              gg_wait_barrier<P::LOADS>();
+            else if (kb + 1 < KE)
+              gg_wait_barrier<0>();
+          }
+          // LDS reads: the next sub-step's activations, the group's scales, the
+          // next group's seeds, the next k-block's weights once their last
+          // dword is decoded
+          const uint32_t from = s == 3 ? nbase : base;
+          if ((n & 1) == 0) read_a1(from, (s + 1) & 3, (s + 1) & 1, n / 2);
+          if (first && n == 0) su[0] = sn[0], su[1] = sn[1];
+          if (last && n >= SL / 2) {
+            if (n < SL / 2 + 2)
+              sn[n - SL / 2] = read_scale(from, GPK > 1 ? (g + 1) % GPK : 0, n - SL / 2);
+            constexpr int RS = 4 * MT / (SL / 2);  // seed reads per slot: 2 (MT 1, PL 2: 1)
+#pragma unroll
+            for (int r = 0; r < RS; ++r)
+              read_seed1(from, GPK > 1 ? (g + 1) % GPK : 0, (n - SL / 2) * RS + r);
+          }
+          if (s == 3) {
+#pragma unroll
+            for (int f = 0; f < 4; ++f)
+              if (n == (NT == 1 ? f : PL == 2 ? (f < 3 ? f : 4) : 2 * f)) read_b1(nbase, f);
+          }
+          // the adds that must precede this slot's MFMA (it overwrites their p)
+          if (MT == 2) {
+            if (first && n == 0) add8(3), add8(4);
+            if (first && n == 1) add8(5);
+            if (first && n == 2) add8(6), add8(7);
+            if (last && n == 6) {
+              sc[0] = scale_to_f32<SDT>(su[0]);
+              add8(0);
+            }
+            if (last && n == 7) {
+              add8(1), add8(2);
+            }
+          } else {
+            if (first && n == 0) add8(0), add8(1);
+            if (first && n == 1) add8(2), add8(3);
+          }
+          p[i][j] = mfma32_bf16(af[s & 1][t][q], d[PL == 2 ? 2 * q + j : (2 * q + j) & 1],
+                                first && q == 0 && (PL == 1 || t == 0) ? seed[i] : p[i][j]);
+#ifdef __HIP_DEVICE_COMPILE__
+          // the seeds stay live past their last use: that MFMA must not take
+          // their registers for its result (64 copies per k-block if it does)
+          if (first && n == (MT == 2 ? 3 : 1)) {
+            asm volatile("" ::"v"(seed[0]));
+            if (MT == 2) asm volatile("" ::"v"(seed[MT - 1]));
+          }
+#endif
+          // the scales replace the last group's once its adds are done
+          if (last && n == SL - 1) {
+            if (MT == 1) sc[0] = scale_to_f32<SDT>(su[0]);
+            sc[1] = scale_to_f32<SDT>(su[1]);
+          }
+          // decode: half a fragment per slot (MT 1 with one plane: a whole one)
+          const int f = (NT == 1 ? n + 1 : PL == 2 ? (n >> 1) + 2 : (n >> 1) + 1);
+          const int fs = (s + (f >> 2)) & 3, fj = f & 1, fq = (f >> 1) & 1;
+          const uint32_t w = b[fj][fq][fs];
+          u32x4_t &o = d[PL == 2 ? f & 3 : f & 1];
+          if (NT == 1) {
+            o = decode8(w);
+          } else if ((n & 1) == 0) {
+            const uint32_t lo = w & 0x0F0F0F0Fu;
+            dx = __builtin_amdgcn_perm(0x43434343u, lo, 0x04010400u);
+            dy = __builtin_amdgcn_perm(0x43434343u, lo, 0x04030402u);
+          } else {
+            const uint32_t hi = (w >> 4) & 0x0F0F0F0Fu;
+            o.x = dx;
+            o.y = dy;
+            o.z = __builtin_amdgcn_perm(0x43434343u, hi, 0x04010400u);
+            o.w = __builtin_amdgcn_perm(0x43434343u, hi, 0x04030402u);
+          }
+          if (DMA && s == 3) {
+#pragma unroll
+            for (int l = 0; l < P::LOADS; ++l)
+              if (l * SL / P::LOADS == n) issue1(l, cur, kb + 3, g3);
+          }
+          __builtin_amdgcn_sched_barrier(0);
+          asm volatile("" ::: "memory");
         }
       }
+      cur = nxt;
+    };
+    int kb = kb0;
+    int g3 = GPK > 1 ? (kb0 + 3) * GPK : (kb0 + 3) / KPG, gr = GPK > 1 ? 0 : (kb0 + 3) % KPG;
+#pragma unroll 1
+    for (; kb + 3 < KE; ++kb) {
+      kblock(GgTrue{}, kb, g3);
+      if (GPK > 1) {
+        g3 += GPK;
+      } else if (++gr == KPG) {
+        gr = 0;
+        ++g3;
+      }
     }
-  }
-  if constexpr (SW) {
-    // the seeds of the planes just written, for the GEMM that reads them as A
-    // (in place of a pass over them): per row, the 16 lanes of a DPP row add
-    // their columns; a group wider than one wave's 8 NT columns adds its
-    // waves' sums through LDS in wave order
-    if (a.seeds_out) {
-      const int per = a.seeds_gw / (8 * NT);  // waves (wn) per group: 1, 2 or 4
-      const int c0 = T0 * 16 + 16 * wn * (NT / 2);  // the wave's first output column
-      float t[MS][4];
+#pragma unroll 1
+    for (; kb < KE; ++kb) kblock(GgFalse{}, kb, 0);
 #pragma unroll
-      for (int i = 0; i < MS; ++i)
+    for (int c = MT == 2 ? 3 : 0; c < 4 * MT; ++c) add8(c);
+  } else {
+    // no live rows in this wave's tiles: its loads and barriers only
+    int g3 = GPK > 1 ? (kb0 + 3) * GPK : (kb0 + 3) / KPG, gr = GPK > 1 ? 0 : (kb0 + 3) % KPG;
+#pragma unroll 1
+    for (int kb = kb0; kb + 1 < KE; ++kb) {
+      if (kb + 3 < KE) {
+        gg_wait_barrier<P::LOADS>();
 #pragma unroll
-        for (int v = 0; v < 4; ++v) t[i][v] = row16_sum(rsum[i][v]);
-      float *so = a.seeds_out + (size_t)(c0 / a.seeds_gw) * a.seeds_rp + row0;
-      if (per == 1) {
-        if (lr == 0 && c0 < a.N) {
-#pragma unroll
-          for (int i = 0; i < MS; ++i)
-#pragma unroll
-            for (int v = 0; v < 4; ++v) {
-              const int m = wm * P::RM + 16 * i + 4 * lg + v;
-              if (m < mrows) so[m] = -136.f * t[i][v];
-            }
+        for (int l = 0; l < P::LOADS; ++l) issue1(l, cur, kb + 3, g3);
+        if (GPK > 1) {
+          g3 += GPK;
+        } else if (++gr == KPG) {
+          gr = 0;
+          ++g3;
         }
       } else {
-        __syncthreads();  // every wave is past its last read of the stages
-        float *part = reinterpret_cast<float *>(stages);  // [WN][BM]
-        if (lr == 0) {
+        gg_wait_barrier<0>();
+      }
+      cur = cur == 2 ? 0 : cur + 1;
+    }
+  }
+
+  // ---- epilogue: D lane l holds column l31 and rows 8 (v / 4) + 4 h + v % 4 ----
+  const bool live = wm * P::RM < mrows;
+  if constexpr (SW) {
+    if (a.part) {  // a slice of K: gate and up partials, columns n and N + n
+      float *part = a.part + (size_t)blockIdx.z * a.M * 2 * a.N;
+      const int n = T0 * 16 + 32 * wn + l31;
+      if (live && n < a.N) {
 #pragma unroll
-          for (int i = 0; i < MS; ++i)
+        for (int i = 0; i < MT; ++i)
 #pragma unroll
-            for (int v = 0; v < 4; ++v) part[wn * P::BM + wm * P::RM + 16 * i + 4 * lg + v] = t[i][v];
+          for (int v = 0; v < 16; ++v) {
+            const int m = wm * P::RM + 32 * i + 8 * (v >> 2) + 4 * h + (v & 3);
+            if (m >= mrows) continue;
+            float *o = part + (size_t)(row0 + m) * 2 * a.N + n;
+            o[0] = acc[i][0][v];
+            o[a.N] = acc[i][1][v];
+          }
+      }
+      return;
+    }
+    // hi = h truncated, lo = RNE(h - hi) of h = silu(g) * u, through LDS so that
+    // the planes are stored 16 bytes a lane
+    constexpr int pitch = P::OUTC * 2 + 16;
+    uint8_t *lo_t = st + P::BM * pitch;
+    __syncthreads();  // every wave is past its last read of the stages
+    if (live) {
+#pragma unroll
+      for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) {
+          const int m = wm * P::RM + 32 * i + 8 * (v >> 2) + 4 * h + (v & 3);
+          const float y = silu_f32(acc[i][0][v]) * acc[i][1][v];
+          const uint32_t hb = fbits(y) >> 16;
+          const uint32_t o = m * pitch + (32 * wn + l31) * 2;
+          *reinterpret_cast<uint16_t *>(st + o) = (uint16_t)hb;
+          *reinterpret_cast<uint16_t *>(lo_t + o) = (uint16_t)f32_to_bf16_rne(y - bitsf(hb << 16));
         }
-        __syncthreads();
-        if (wn % per == 0 && lr == 0 && c0 < a.N) {
-#pragma unroll
-          for (int i = 0; i < MS; ++i)
-#pragma unroll
-            for (int v = 0; v < 4; ++v) {
-              const int m = wm * P::RM + 16 * i + 4 * lg + v;
-              float sum = part[wn * P::BM + m];
-              for (int q = 1; q < per; ++q) sum += part[(wn + q) * P::BM + m];
-              if (m < mrows) so[m] = -136.f * sum;
-            }
-        }
+    }
+    __syncthreads();
+    gg_store_tile<P::OUTC>(st, pitch, reinterpret_cast<uint16_t *>(a.y), row0, mrows, T0 * 16, a.N,
+                           a.ldy, tid, 64 * P::W);
+    gg_store_tile<P::OUTC>(lo_t, pitch, reinterpret_cast<uint16_t *>(a.y2), row0, mrows, T0 * 16,
+                           a.N, a.ldy, tid, 64 * P::W);
+    if (a.seeds_out) {
+      // the seeds of the planes just written, for the GEMM that reads them as A
+      // (in place of a pass over them): 16 consecutive lanes hold a row's 128
+      // columns, 16 / GPK of them a group
+      constexpr int L = 16 / GPK;
+      for (int c = tid; c < P::BM * 16; c += 64 * P::W) {
+        const int m = c >> 4, col = 8 * (c & 15), n = T0 * 16 + col;
+        const uint32_t o = m * pitch + col * 2;
+        float t = sum8_bf16(*reinterpret_cast<const u32x4_t *>(st + o)) +
+                  sum8_bf16(*reinterpret_cast<const u32x4_t *>(lo_t + o));
+        t = lane_group_sum<L>(t);
+        if ((c & (L - 1)) == 0 && m < mrows && n < a.N)
+          a.seeds_out[(size_t)(n / (8 * L)) * a.seeds_rp + row0 + m] = -136.f * t;
       }
     }
+  } else if (a.part || a.epi == GG_F32) {
+    float *y = a.part ? a.part + (size_t)blockIdx.z * a.M * a.N : reinterpret_cast<float *>(a.y);
+    const size_t ld = a.part ? a.N : a.ldy;
+    if (live) {
+#pragma unroll
+      for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) {
+          const int m = wm * P::RM + 32 * i + 8 * (v >> 2) + 4 * h + (v & 3);
+          const int n = T0 * 16 + 64 * wn + l31;
+          if (m >= mrows) continue;
+          float *o = y + (size_t)(row0 + m) * ld + n;
+          if (n < a.N) o[0] = acc[i][0][v];
+          if (n + 32 < a.N) o[32] = acc[i][1][v];
+        }
+    }
+  } else {
+    constexpr int pitch = P::BN * 2 + 16;
+    __syncthreads();
+    if (live) {
+#pragma unroll
+      for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) {
+          const int m = wm * P::RM + 32 * i + 8 * (v >> 2) + 4 * h + (v & 3);
+          uint8_t *o = st + m * pitch + (64 * wn + l31) * 2;
+          *reinterpret_cast<uint16_t *>(o) = (uint16_t)f32_to_bf16_rne(acc[i][0][v]);
+          *reinterpret_cast<uint16_t *>(o + 64) = (uint16_t)f32_to_bf16_rne(acc[i][1][v]);
+        }
+    }
+    __syncthreads();
+    gg_store_tile<P::OUTC>(st, pitch, reinterpret_cast<uint16_t *>(a.y), row0, mrows, T0 * 16, a.N,
+                           a.ldy, tid, 64 * P::W);
   }
 }
 
@@ -506,17 +648,10 @@ __global__ __launch_bounds__(256) void gg_reduce_kernel(const float *part, void 
 // gg_prep: seeds (and converted activations), one wave per row
 // ---------------------------------------------------------------------------
 
-// Sum over groups of L consecutive lanes (L = 4, 8, 16 within a DPP row):
-// quad sums, then a half-row mirror (lane i <- 7 - i of its 8 lanes: the other
-// quad of the same half), then a row mirror (the other half).
-template <int L>
-CAI4_DEV float lane_group_sum(float t) {
-  t += dpp_f32<0xB1>(t);                          // quad_perm 1,0,3,2
-  t += dpp_f32<0x4E>(t);                          // quad_perm 2,3,0,1
-  if constexpr (L >= 8) t += dpp_f32<0x141>(t);   // row_half_mirror
-  if constexpr (L >= 16) t += dpp_f32<0x140>(t);  // row_mirror
-  return t;
-}
+// One wave per row and kGgPrepPasses passes of 512 columns (blockIdx.y: which),
+// every load issued before the first sum: the pass is latency-bound, so it is
+// spread over as many waves as the rows and columns give.
+constexpr int kGgPrepPasses = 2;
 
 template <int L>
 __global__ __launch_bounds__(256) void gg_prep_kernel(int mode, const void *src, const void *src2,
@@ -524,6 +659,7 @@ __global__ __launch_bounds__(256) void gg_prep_kernel(int mode, const void *src,
                                                       uint16_t *out2, float *seeds, int rows,
                                                       int rows_pad, int K,
                                                       const int32_t *rows_dev) {
+  constexpr int P = kGgPrepPasses;
   const int lane = threadIdx.x & 63;
   const int r = blockIdx.x * 4 + (threadIdx.x >> 6);
   if (rows_dev) rows = *rows_dev;
@@ -531,65 +667,78 @@ __global__ __launch_bounds__(256) void gg_prep_kernel(int mode, const void *src,
   const int gw = 8 * L;   // columns per seed group
   size_t srow = (size_t)r;
   if (mode == 2 && row_map) srow = (size_t)row_map[r];
-  for (int c0 = 0; c0 < K; c0 += 512) {
-    const int c = c0 + 8 * lane;
-    float t = 0.f;
-    if (c < K) {
-      if (mode <= 1) {
-        const u32x4_t v = *reinterpret_cast<const u32x4_t *>(
-            reinterpret_cast<const uint16_t *>(src) + srow * K + c);
-        t = sum8_bf16(v);
-        if (mode == 1)
-          t += sum8_bf16(*reinterpret_cast<const u32x4_t *>(
-              reinterpret_cast<const uint16_t *>(src2) + srow * K + c));
-      } else {
-        const float *f = reinterpret_cast<const float *>(src) + srow * K + c;
-        const f32x4_t a = *reinterpret_cast<const f32x4_t *>(f);
-        const f32x4_t b = *reinterpret_cast<const f32x4_t *>(f + 4);
-        if (mode == 2) {
-          u32x4_t o;
-          o.x = f32_to_bf16_rne(a.x) | (f32_to_bf16_rne(a.y) << 16);
-          o.y = f32_to_bf16_rne(a.z) | (f32_to_bf16_rne(a.w) << 16);
-          o.z = f32_to_bf16_rne(b.x) | (f32_to_bf16_rne(b.y) << 16);
-          o.w = f32_to_bf16_rne(b.z) | (f32_to_bf16_rne(b.w) << 16);
-          *reinterpret_cast<u32x4_t *>(out + (size_t)r * K + c) = o;
-          t = sum8_bf16(o);
-        } else {
-          const u32x4_t hi = act_split_f32_nat(a, b, false), lo = act_split_f32_nat(a, b, true);
-          *reinterpret_cast<u32x4_t *>(out + (size_t)r * K + c) = hi;
-          *reinterpret_cast<u32x4_t *>(out2 + (size_t)r * K + c) = lo;
-          t = sum8_bf16(hi) + sum8_bf16(lo);
-        }
+  const int c0 = blockIdx.y * P * 512 + 8 * lane;
+  u32x4_t v[P], w[P];  // 8 columns a pass: bf16 hi (and lo), or two halves of f32
+#pragma unroll
+  for (int q = 0; q < P; ++q) {
+    const int c = c0 + 512 * q;
+    v[q] = w[q] = u32x4_t{0u, 0u, 0u, 0u};
+    if (c >= K) continue;
+    if (mode <= 1) {
+      v[q] = *reinterpret_cast<const u32x4_t *>(static_cast<const uint16_t *>(src) + srow * K + c);
+      if (mode == 1)
+        w[q] = *reinterpret_cast<const u32x4_t *>(static_cast<const uint16_t *>(src2) + srow * K + c);
+    } else {
+      const float *f = static_cast<const float *>(src) + srow * K + c;
+      v[q] = *reinterpret_cast<const u32x4_t *>(f);
+      w[q] = *reinterpret_cast<const u32x4_t *>(f + 4);
+    }
+  }
+#pragma unroll
+  for (int q = 0; q < P; ++q) {
+    const int c = c0 + 512 * q;
+    float t;
+    if (mode <= 1) {
+      t = sum8_bf16(v[q]);
+      if (mode == 1) t += sum8_bf16(w[q]);
+    } else if (mode == 2) {
+      u32x4_t o;
+      o.x = f32_to_bf16_rne(bitsf(v[q].x)) | (f32_to_bf16_rne(bitsf(v[q].y)) << 16);
+      o.y = f32_to_bf16_rne(bitsf(v[q].z)) | (f32_to_bf16_rne(bitsf(v[q].w)) << 16);
+      o.z = f32_to_bf16_rne(bitsf(w[q].x)) | (f32_to_bf16_rne(bitsf(w[q].y)) << 16);
+      o.w = f32_to_bf16_rne(bitsf(w[q].z)) | (f32_to_bf16_rne(bitsf(w[q].w)) << 16);
+      if (c < K) *reinterpret_cast<u32x4_t *>(out + (size_t)r * K + c) = o;
+      t = sum8_bf16(o);
+    } else {
+      const f32x4_t fa = __builtin_bit_cast(f32x4_t, v[q]), fb = __builtin_bit_cast(f32x4_t, w[q]);
+      const u32x4_t hi = act_split_f32_nat(fa, fb, false), lo = act_split_f32_nat(fa, fb, true);
+      if (c < K) {
+        *reinterpret_cast<u32x4_t *>(out + (size_t)r * K + c) = hi;
+        *reinterpret_cast<u32x4_t *>(out2 + (size_t)r * K + c) = lo;
       }
+      t = sum8_bf16(hi) + sum8_bf16(lo);
     }
     t = lane_group_sum<L>(t);
     if ((lane & (L - 1)) == 0 && c < K) seeds[(size_t)(c / gw) * rows_pad + r] = -136.f * t;
   }
 }
 
-template <int MS, int NT, int WM, int WN, int GPK, bool HILO, bool SW>
-hipError_t gg_launch(const GgArgs &a, dim3 grid, hipStream_t st) {
+template <int MT, int WM, int WN, int GPK, int PL, bool SW>
+hipError_t gg_launch(const GgArgs &a, int rows_y, int nsl, hipStream_t st) {
+  using P = Gg<MT, WM, WN, GPK, PL, SW>;
+  const dim3 grid((a.N + P::OUTC - 1) / P::OUTC, rows_y ? rows_y : (a.M + P::BM - 1) / P::BM, nsl);
   if (a.sdt)
-    hipLaunchKernelGGL((gg_kernel<MS, NT, WM, WN, GPK, HILO, SW, SCALE_F16>), grid,
-                       dim3(64 * WM * WN), 0, st, a);
+    hipLaunchKernelGGL((gg_kernel<MT, WM, WN, GPK, PL, SW, SCALE_F16>), grid, dim3(64 * P::W), 0, st,
+                       a);
   else
-    hipLaunchKernelGGL((gg_kernel<MS, NT, WM, WN, GPK, HILO, SW, SCALE_BF16>), grid,
-                       dim3(64 * WM * WN), 0, st, a);
+    hipLaunchKernelGGL((gg_kernel<MT, WM, WN, GPK, PL, SW, SCALE_BF16>), grid, dim3(64 * P::W), 0,
+                       st, a);
   return hipGetLastError();
 }
 
-template <int MS, int NT, int WM, int WN, bool HILO, bool SW>
-hipError_t gg_launch_g(const GgArgs &a, dim3 grid, hipStream_t st) {
+// rows_y: workgroup rows (0: as many as a.M takes); nsl: slices of K.
+template <int MT, int WM, int WN, int PL, bool SW>
+hipError_t gg_launch_g(const GgArgs &a, int rows_y, int nsl, hipStream_t st) {
   switch (a.G == 32 ? 4 : a.G == 64 ? 2 : 1) {
-    case 4: return gg_launch<MS, NT, WM, WN, 4, HILO, SW>(a, grid, st);
-    case 2: return gg_launch<MS, NT, WM, WN, 2, HILO, SW>(a, grid, st);
-    default: return gg_launch<MS, NT, WM, WN, 1, HILO, SW>(a, grid, st);
+    case 4: return gg_launch<MT, WM, WN, 4, PL, SW>(a, rows_y, nsl, st);
+    case 2: return gg_launch<MT, WM, WN, 2, PL, SW>(a, rows_y, nsl, st);
+    default: return gg_launch<MT, WM, WN, 1, PL, SW>(a, rows_y, nsl, st);
   }
 }
 
 // Dense tile shapes (rows x output columns): 128 x 256 (8 waves) in up to 4
 // slices of K when the tiles alone leave CUs idle, else 128 x 128 or 64 x 128
-// (4 waves) -- the choices prefill.hip measured.  Two-plane A: 64 x 256.
+// (4 waves).  Two-plane A: 64 x 256.
 int gg_dense_ksplit(int M, int N, int K, int num_cus) {
   const long tiles = (long)((N + 255) / 256) * ((M + 127) / 128);
   const int KB = K / 128;
@@ -606,13 +755,13 @@ bool gg_supported(int K, int G, int tiled) {
   return tiled && K % 128 == 0 && (G == 32 || G == 64 || G % 128 == 0) && K % G == 0;
 }
 
-int gg_rows_pad(int rows) { return (rows + 255) / 128 * 128; }
+int gg_rows_pad(int rows) { return (rows + 127) / 128 * 128; }
 
 hipError_t gg_prep(int mode, const void *src, const void *src2, const int32_t *row_map,
                    uint16_t *out, uint16_t *out2, float *seeds, int rows, int rows_pad, int K,
                    int G, const int32_t *rows_dev, hipStream_t st) {
   if (rows <= 0) return hipSuccess;
-  const dim3 grid((rows + 3) / 4), block(256);
+  const dim3 grid((rows + 3) / 4, (K + 512 * kGgPrepPasses - 1) / (512 * kGgPrepPasses)), block(256);
   const int gw = gg_group_width(G);
   if (gw == 32)
     hipLaunchKernelGGL(gg_prep_kernel<4>, grid, block, 0, st, mode, src, src2, row_map, out, out2,
@@ -666,16 +815,14 @@ hipError_t gg_dense(GgArgs a, int amode, void *ws, int num_cus, hipStream_t st) 
                                       a.rows_pad, a.K, a.G, nullptr, st)) {
       return e;
     }
-    const dim3 grid((a.N + (sw ? 127 : 255)) / (sw ? 128 : 256), (a.M + 63) / 64, 1);
-    if (sw) return gg_launch_g<2, 4, 2, 4, true, true>(a, grid, st);
-    return gg_launch_g<2, 4, 2, 4, true, false>(a, grid, st);
+    if (sw) return gg_launch_g<1, 2, 4, 2, true>(a, 0, 1, st);
+    return gg_launch_g<1, 2, 4, 2, false>(a, 0, 1, st);
   }
   if (hipError_t e = gg_prep(0, a.x, nullptr, nullptr, nullptr, nullptr, seeds, a.M, a.rows_pad,
                              a.K, a.G, nullptr, st))
     return e;
   if (sw)
-    return gg_launch_g<4, 4, 2, 4, false, true>(a, dim3((a.N + 127) / 128, (a.M + 127) / 128, 1),
-                                                st);
+    return gg_launch_g<2, 2, 4, 1, true>(a, 0, 1, st);
   const int ks = gg_dense_ksplit(a.M, a.N, a.K, num_cus);
   if (ks >= 1) {
     int nsl = 1;
@@ -684,8 +831,7 @@ hipError_t gg_dense(GgArgs a, int amode, void *ws, int num_cus, hipStream_t st) 
       nsl = (a.K / 128 + a.kper - 1) / a.kper;
       a.part = reinterpret_cast<float *>(w);
     }
-    const dim3 grid((a.N + 255) / 256, (a.M + 127) / 128, nsl);
-    if (hipError_t e = gg_launch_g<4, 4, 2, 4, false, false>(a, grid, st)) return e;
+    if (hipError_t e = gg_launch_g<2, 2, 4, 1, false>(a, 0, nsl, st)) return e;
     if (nsl > 1) {
       const size_t n = (size_t)a.M * a.N;
       hipLaunchKernelGGL(gg_reduce_kernel, dim3((unsigned)((n / 4 + 255) / 256)), dim3(256), 0,
@@ -694,11 +840,7 @@ hipError_t gg_dense(GgArgs a, int amode, void *ws, int num_cus, hipStream_t st) 
     }
     return hipSuccess;
   }
-  const long tiles_mid = (long)((a.N + 127) / 128) * ((a.M + 127) / 128);
-  if (tiles_mid >= num_cus)
-    return gg_launch_g<4, 4, 2, 2, false, false>(a, dim3((a.N + 127) / 128, (a.M + 127) / 128, 1),
-                                                 st);
-  return gg_launch_g<2, 4, 2, 2, false, false>(a, dim3((a.N + 127) / 128, (a.M + 63) / 64, 1), st);
+  return gg_launch_g<1, 2, 2, 1, false>(a, 0, 1, st);
 }
 
 hipError_t gg_grouped(const GgArgs &a0, int max_tiles, hipStream_t st) {
@@ -714,17 +856,14 @@ hipError_t gg_grouped(const GgArgs &a0, int max_tiles, hipStream_t st) {
   // rows through a row map: one bf16 plane, x rows addressable in 31 bits
   if (a.row_map && (a.hilo || a.x_rows <= 0 || (size_t)a.x_rows * a.K * 2 > 0x7FFFFFFFu))
     return hipErrorInvalidValue;
-  const unsigned gx = sw ? (a.N + 127) / 128 : (a.N + 255) / 256;
   if (a.hilo) {  // 64-row tiles: two per table entry
     a.tile_split = kGgChunkRows / 64;
-    const dim3 grid(gx, max_tiles * a.tile_split, 1);
-    if (sw) return gg_launch_g<2, 4, 2, 4, true, true>(a, grid, st);
-    return gg_launch_g<2, 4, 2, 4, true, false>(a, grid, st);
+    if (sw) return gg_launch_g<1, 2, 4, 2, true>(a, max_tiles * a.tile_split, 1, st);
+    return gg_launch_g<1, 2, 4, 2, false>(a, max_tiles * a.tile_split, 1, st);
   }
   a.tile_split = kGgChunkRows / 128;
-  const dim3 grid(gx, max_tiles * a.tile_split, 1);
-  if (sw) return gg_launch_g<4, 4, 2, 4, false, true>(a, grid, st);
-  return gg_launch_g<4, 4, 2, 4, false, false>(a, grid, st);
+  if (sw) return gg_launch_g<2, 2, 4, 1, true>(a, max_tiles * a.tile_split, 1, st);
+  return gg_launch_g<2, 2, 4, 1, false>(a, max_tiles * a.tile_split, 1, st);
 }
 
 }  // namespace cai4

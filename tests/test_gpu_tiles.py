@@ -66,6 +66,33 @@ def test_expert_forward_tiles(cl, orc, tuning, M, h, i, g, sdt):
     assert_bf16_close(host(out).view(np.uint16).reshape(M, h), want, f"tiles M{M} G{g}")
 
 
+@pytest.mark.parametrize("n,k,g,sdt,M", [
+    # one to four k-blocks (fewer than the pipeline's stages, and one more), a
+    # single 16-row weight tile, the 32- and 64-column edges of a wave, ragged
+    # rows around the 32 / 64 / 128-row edges, groups of several k-blocks
+    (16, 128, 32, F16, 64), (17, 128, 128, F16, 65), (255, 256, 64, BF16, 96),
+    (257, 384, 32, BF16, 127), (272, 512, 128, F16, 129), (31, 768, 256, F16, 161),
+    (1000, 1536, 512, BF16, 300), (4097, 1024, 64, F16, 70)])
+def test_gemm_tile_edges(cl, orc, n, k, g, sdt, M):
+    """gemm_int4_bf16 (bf16 out) and bf16-in / f32-out over tiled weights at
+    the tile kernel's edges, against the oracle."""
+    packed = orc.fill_bytes(n + M, 1, n * k // 2)
+    scales = orc.fill_scales(n + M, 2, n * (k // g), sdt).view(np.uint8).copy()
+    pt, st = cl.tile_weights(dev(packed), dev(scales), n, k, g)
+    xb = orc.fill_normal_bf16(k, M, M * k)
+    xd = dev(xb.view(np.int16))
+    want = orc.gemm_multi(packed, scales, orc.bf16_to_f32(xb), n, k, M, g, sdt)
+    ys = torch.empty(M * n, dtype=torch.float32, device="cuda")
+    cl.dequant_gemm_int4_multi_auto(pt, st, xd, n, k, M, ys, group_size=g, scale_dtype=sdt,
+                                    tiling=cl.TILING_MFMA)
+    assert_f32_close(host(ys).reshape(M, n), want, f"f32 out {n}x{k} G{g} M{M}")
+    yb = torch.empty(M * n, dtype=torch.int16, device="cuda")
+    cl.gemm_int4_bf16(pt, st, xd, n, k, M, yb, group_size=g, scale_dtype=sdt,
+                      tiling=cl.TILING_MFMA)
+    assert_bf16_close(host(yb).view(np.uint16).reshape(M, n), orc.f32_to_bf16(want),
+                      f"bf16 out {n}x{k} G{g} M{M}")
+
+
 @pytest.mark.parametrize("M,g", [(65, 32), (100, 64), (200, 128)])
 def test_ffn_f32_tiles(cl, orc, tuning, M, g):
     """The f32-in / f32-out FFN (the shared expert) over M rows: x split into
