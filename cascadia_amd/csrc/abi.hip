@@ -243,46 +243,100 @@ int run_gemm(const uint8_t *w0, const uint8_t *s0, const uint8_t *w1, const uint
   return hip_status(cai4::skinny_launch(a, p, amode, epi, st));
 }
 
-// Tokens from which an expert FFN runs on the MFMA-tile GEMMs (grouped.hip)
-// rather than the skinny kernel's 64-row passes (measured: the tiles win from
-// 512 rows at the K2.6 and Llama-3-8B FFN shapes; below, too few workgroups).
-// CASCADIA_INT4_FFN_TILE_TOKENS overrides.
+// Whether many tokens run on the MFMA-tile GEMMs (grouped.hip) rather than in
+// the skinny kernel's passes of `pass` rows, which stream the weights (`bytes`)
+// once each: from `min_tokens` rows and `min_bytes` streamed in all.  Below
+// that the tile path's extra launches (seeds, split-K reduce) cost more than
+// the passes.  Measured (us, tiles / skinny):
+//   FFN bf16  4096 x 14336 G128: 32 rows 59.7 / 63.4, 48: 62 / 108, 200: 110 / 216
+//             7168 x 2048 G32: 64 rows 49.5 / 37.1, 100: 50.4 / 51.4, 200: 58 / 108
+//             3072 x 1536 G128: 200 rows 40.0 / 37.5, 400: 43.3 / 50.3
+//   FFN f32   7168 x 2048 G32: 32 rows 40.3 / 34.5, 64: 44.2 / 45.5, 256: 71 / 159
+//   GEMM f32  7168 x 8192 G32: 17 rows 23 / 37, 333: 98 / 264
+//             1536 x 7168 G32: 96 rows 24.3 / 20.0, 128: 25.1 / 36.9
+//             4096 x 4096 G128: 64 rows 20.0 / 16.2, 96: 22.8 / 26.5, 333: 35 / 57
+//             576 x 7168 G32: 200 rows 25.6 / 20.7, 333: 27.1 / 38.6
+//   GEMM bf16 14336 x 4096 G128: 32 rows 18.5 / 16.9, 48: 21 / 27
+//             7168 x 8192 G32: 32 rows 19.1 / 19.5, 48: 24 / 38
+bool tiles_pay(uint32_t tokens, uint32_t pass, size_t bytes, uint32_t min_tokens,
+               size_t min_bytes) {
+  return tokens >= min_tokens && (size_t)((tokens + pass - 1) / pass) * bytes >= min_bytes;
+}
+
+// Tokens from which an expert FFN always runs on the tile GEMMs (also where
+// the workspace is no larger than the seeds need, without splitting K).
+// CASCADIA_INT4_FFN_TILE_TOKENS overrides, and is then the only rule.
 uint32_t ffn_tile_tokens() {
   const int n = cai4::tuning_env("CASCADIA_INT4_FFN_TILE_TOKENS", 0);
   return n > 0 ? (uint32_t)n : 512u;
 }
+bool ffn_tiles_pay(uint32_t hidden, uint32_t inter, uint32_t n_tokens, bool x_f32) {
+  if (n_tokens >= ffn_tile_tokens()) return true;
+  if (cai4::tuning_env("CASCADIA_INT4_FFN_TILE_TOKENS", 0) > 0) return false;
+  return tiles_pay(n_tokens, x_f32 ? 32 : 64, (size_t)hidden * inter * 3 / 2, 32, (size_t)44 << 20);
+}
 
-bool ffn_tile_shape(uint32_t hidden, uint32_t inter, uint32_t group, uint32_t n_tokens) {
-  return n_tokens >= ffn_tile_tokens() && cai4::gg_supported((int)hidden, (int)group, 1) &&
+bool ffn_tile_shape(uint32_t hidden, uint32_t inter, uint32_t group) {
+  return cai4::gg_supported((int)hidden, (int)group, 1) &&
          cai4::gg_supported((int)inter, (int)group, 1);
 }
 
 // Workspace of an expert FFN: the SwiGLU intermediate as two bf16 planes,
 // then the split-K partials of whichever of its two GEMMs needs more; or, for
-// many tokens, the planes and the MFMA-tile GEMMs' seeds / split activations.
+// many tokens, the planes, their seeds and the MFMA-tile GEMMs' own (tile); or
+// the same without splitting K and with the down's seeds in the GEMMs' share
+// (lean), where no more memory can be had.
 struct FfnWorkspace {
-  size_t planes, partials, tile;
-  size_t total() const { return planes + partials > tile ? planes + partials : tile; }
+  size_t planes, partials, tile, lean;
+  size_t skinny() const { return planes + partials; }
+  size_t least() const { return skinny() > lean ? skinny() : lean; }
+  size_t total() const { return least() > tile ? least() : tile; }
 };
+size_t ffn_plane_bytes(uint32_t inter, uint32_t n_tokens) {
+  return ((size_t)n_tokens * inter * 2 + 255) & ~(size_t)255;
+}
+// The intermediate's seeds, left by the gate/up for the down.
+size_t ffn_seed_bytes(uint32_t inter, uint32_t group, uint32_t n_tokens) {
+  return (((size_t)(inter / cai4::gg_group_width((int)group)) *
+           cai4::gg_rows_pad((int)n_tokens) * 4) + 255) & ~(size_t)255;
+}
 size_t ffn_tile_workspace(int num_cus, uint32_t hidden, uint32_t inter, uint32_t group,
-                          uint32_t n_tokens, bool x_f32, bool out_bf16) {
-  const size_t planes = 2 * (((size_t)n_tokens * inter * 2 + 255) & ~(size_t)255);
+                          uint32_t n_tokens, bool x_f32, bool out_bf16, bool lean) {
+  if (lean) {  // two planes, then the seeds of x (and its planes) or of the intermediate
+    const size_t rp = (size_t)cai4::gg_rows_pad((int)n_tokens) + 128;
+    const int gw = cai4::gg_group_width((int)group);
+    auto al = [](size_t v) { return (v + 255) & ~(size_t)255; };
+    const size_t a = al(hidden / gw * rp * 4) + (x_f32 ? 2 * al((size_t)n_tokens * hidden * 2) : 0);
+    const size_t b = al(inter / gw * rp * 4);
+    return 2 * ffn_plane_bytes(inter, n_tokens) + (a > b ? a : b);
+  }
   const size_t a = cai4::gg_dense_workspace((int)n_tokens, (int)inter, (int)hidden, (int)group,
                                             x_f32 ? cai4::GG_A_F32 : cai4::GG_A_BF16,
                                             cai4::GG_SWIGLU_HILO, num_cus);
   const size_t b = cai4::gg_dense_workspace((int)n_tokens, (int)hidden, (int)inter, (int)group,
                                             cai4::GG_A_PLANES,
-                                            out_bf16 ? cai4::GG_BF16 : cai4::GG_F32, num_cus);
-  return planes + (a > b ? a : b);
+                                            out_bf16 ? cai4::GG_BF16 : cai4::GG_F32, num_cus,
+                                            true);
+  return 2 * ffn_plane_bytes(inter, n_tokens) + ffn_seed_bytes(inter, group, n_tokens) +
+         (a > b ? a : b);
 }
 FfnWorkspace ffn_workspace(int dev, uint32_t hidden, uint32_t inter, uint32_t group,
                            uint32_t n_tokens, bool x_f32) {
   const cai4::SkinnyDevice d = device_props(dev);
-  size_t tile = 0;
-  if (ffn_tile_shape(hidden, inter, group, n_tokens)) {
-    const size_t t0 = ffn_tile_workspace(d.num_cus, hidden, inter, group, n_tokens, x_f32, false);
-    const size_t t1 = ffn_tile_workspace(d.num_cus, hidden, inter, group, n_tokens, x_f32, true);
-    tile = t0 > t1 ? t0 : t1;
+  size_t tile = 0, lean = 0;
+  if (ffn_tile_shape(hidden, inter, group)) {
+    for (int bf = 0; bf < 2; ++bf) {
+      if (ffn_tiles_pay(hidden, inter, n_tokens, x_f32)) {
+        const size_t t =
+            ffn_tile_workspace(d.num_cus, hidden, inter, group, n_tokens, x_f32, bf, false);
+        tile = t > tile ? t : tile;
+      }
+      if (n_tokens >= ffn_tile_tokens()) {
+        const size_t t =
+            ffn_tile_workspace(d.num_cus, hidden, inter, group, n_tokens, x_f32, bf, true);
+        lean = t > lean ? t : lean;
+      }
+    }
   }
   const cai4::SkinnyPlan gu =
       cai4::skinny_plan((int)inter, (int)hidden, (int)group, (int)n_tokens,
@@ -292,18 +346,26 @@ FfnWorkspace ffn_workspace(int dev, uint32_t hidden, uint32_t inter, uint32_t gr
   const size_t planes = ((size_t)n_tokens * inter * 2 * sizeof(uint16_t) + 255) & ~(size_t)255;
   return FfnWorkspace{planes,
                       gu.partial_bytes > dn.partial_bytes ? gu.partial_bytes : dn.partial_bytes,
-                      tile};
+                      tile, lean};
 }
 
 // The expert FFN on the MFMA-tile GEMMs: gate/up with the SwiGLU epilogue
-// into hi / lo planes, then down over the planes (grouped.hip, dense mode).
+// into hi / lo planes (and their seeds), then down over the planes
+// (grouped.hip, dense mode).
 int ffn_tiles(uint32_t hidden, uint32_t inter, uint32_t group, uint32_t sdt,
               const cascadia_int4_expert *e, const void *x, bool x_f32, uint32_t n_tokens,
-              void *out, bool out_bf16, void *ws, int num_cus, hipStream_t st) {
-  const size_t plane = ((size_t)n_tokens * inter * 2 + 255) & ~(size_t)255;
-  uint16_t *hi = static_cast<uint16_t *>(ws);
-  uint16_t *lo = reinterpret_cast<uint16_t *>(static_cast<uint8_t *>(ws) + plane);
-  void *rest = static_cast<uint8_t *>(ws) + 2 * plane;
+              void *out, bool out_bf16, void *ws, bool lean, int num_cus, hipStream_t st) {
+  const size_t plane = ffn_plane_bytes(inter, n_tokens);
+  const int slices = lean ? 1 : 8;
+  uint8_t *b = static_cast<uint8_t *>(ws);
+  uint16_t *hi = reinterpret_cast<uint16_t *>(b);
+  uint16_t *lo = reinterpret_cast<uint16_t *>(b + plane);
+  b += 2 * plane;
+  float *seeds = nullptr;
+  if (!lean) {
+    seeds = reinterpret_cast<float *>(b);
+    b += ffn_seed_bytes(inter, group, n_tokens);
+  }
   cai4::GgArgs g{};
   g.w0 = e->gate_packed;
   g.s0 = e->gate_scale;
@@ -319,14 +381,19 @@ int ffn_tiles(uint32_t hidden, uint32_t inter, uint32_t group, uint32_t sdt,
   g.sdt = (int)sdt;
   g.ldy = (int)inter;
   g.epi = cai4::GG_SWIGLU_HILO;
+  g.seeds_out = seeds;
+  g.seeds_gw = cai4::gg_group_width((int)group);
+  g.seeds_rp = cai4::gg_rows_pad((int)n_tokens);
   if (hipError_t err =
-          cai4::gg_dense(g, x_f32 ? cai4::GG_A_F32 : cai4::GG_A_BF16, rest, num_cus, st))
+          cai4::gg_dense(g, x_f32 ? cai4::GG_A_F32 : cai4::GG_A_BF16, b, num_cus, st, slices))
     return hip_status(err);
   cai4::GgArgs dn{};
   dn.w0 = e->down_packed;
   dn.s0 = e->down_scale;
   dn.x = hi;
   dn.x2 = lo;
+  dn.seeds = seeds;
+  dn.rows_pad = g.seeds_rp;
   dn.y = out;
   dn.M = (int)n_tokens;
   dn.N = (int)hidden;
@@ -335,7 +402,7 @@ int ffn_tiles(uint32_t hidden, uint32_t inter, uint32_t group, uint32_t sdt,
   dn.sdt = (int)sdt;
   dn.ldy = (int)hidden;
   dn.epi = out_bf16 ? cai4::GG_BF16 : cai4::GG_F32;
-  return hip_status(cai4::gg_dense(dn, cai4::GG_A_PLANES, rest, num_cus, st));
+  return hip_status(cai4::gg_dense(dn, cai4::GG_A_PLANES, b, num_cus, st, slices));
 }
 
 void expert_sections(uint32_t hidden, uint32_t inter, uint32_t group, size_t off[6]) {
@@ -371,7 +438,8 @@ int check_expert(uint32_t hidden, uint32_t inter, uint32_t group, uint32_t sdt,
 
 int ffn_common(uint32_t hidden, uint32_t inter, uint32_t group, uint32_t sdt,
                const cascadia_int4_expert *e, const void *x, bool x_f32, uint32_t n_tokens,
-               void *out, bool out_bf16, void *workspace, hipStream_t st) {
+               void *out, bool out_bf16, void *workspace, hipStream_t st,
+               size_t workspace_bytes = ~(size_t)0) {
   if (int rc = check_expert(hidden, inter, group, sdt, e)) return rc;
   if (n_tokens == 0) return CASCADIA_INT4_OK;
   if (!x || !out) return CASCADIA_INT4_ERR_NULL;
@@ -383,15 +451,20 @@ int ffn_common(uint32_t hidden, uint32_t inter, uint32_t group, uint32_t sdt,
     return CASCADIA_INT4_ERR_ARG;
   const FfnWorkspace need = ffn_workspace(dev, hidden, inter, group, n_tokens, x_f32);
   void *ws = workspace;
+  bool lean = need.total() > workspace_bytes;
   if (!ws) {
-    if (int rc = lib_workspace(dev, need.total(), &ws, st)) return rc;
+    // a library workspace that cannot grow now (a capture, no memory) may still
+    // hold what the call needs at least
+    if (lib_workspace(dev, need.total(), &ws, st)) {
+      if (int rc = lib_workspace(dev, need.least(), &ws, st)) return rc;
+      lean = true;
+    }
   } else if (!aligned(ws, 16)) {
     return CASCADIA_INT4_ERR_ARG;
   }
-  if (need.tile && e->tiling == CASCADIA_INT4_TILING_MFMA) {
-    return ffn_tiles(hidden, inter, group, sdt, e, x, x_f32, n_tokens, out, out_bf16, ws,
+  if ((lean ? need.lean : need.tile) && e->tiling == CASCADIA_INT4_TILING_MFMA)
+    return ffn_tiles(hidden, inter, group, sdt, e, x, x_f32, n_tokens, out, out_bf16, ws, lean,
                      device_props(dev).num_cus, st);
-  }
   // the SwiGLU intermediate as two bf16 planes (hi, lo): [n_tokens, inter] each
   uint16_t *hi = reinterpret_cast<uint16_t *>(ws);
   uint16_t *lo = hi + (size_t)n_tokens * inter;
@@ -820,24 +893,29 @@ void expert_blob_sections(uint32_t hidden, uint32_t inter, uint32_t group, uint3
   }
 }
 
-// Prefill GEMM (M >= 64 tokens, MFMA-tiled weights).
+// Prefill GEMM (many tokens, MFMA-tiled weights): bf16 x, or f32 x as two planes.
 int run_prefill(const cascadia_int4_layout *L, const uint8_t *packed, const uint8_t *scales,
-                const uint16_t *x, uint32_t M, void *y, bool out_f32, hipStream_t st) {
+                const void *x, bool x_f32, uint32_t M, void *y, bool out_f32, hipStream_t st) {
   int dev;
   if (int rc = current_device(&dev)) return rc;
   if ((size_t)M * L->k_cols * 2 >= 0x7FFFFFFFu) return CASCADIA_INT4_ERR_ARG;
   const int cus = device_props(dev).num_cus;
+  const int amode = x_f32 ? cai4::GG_A_F32 : cai4::GG_A_BF16;
+  const int epi = out_f32 ? cai4::GG_F32 : cai4::GG_BF16;
   void *ws = nullptr;
-  if (int rc = lib_workspace(
-          dev,
-          cai4::gg_dense_workspace((int)M, (int)L->n_rows, (int)L->k_cols, (int)L->group_size,
-                                   cai4::GG_A_BF16, out_f32 ? cai4::GG_F32 : cai4::GG_BF16, cus),
-          &ws, st))
-    return rc;
+  int slices = 8;
+  auto bytes = [&] {
+    return cai4::gg_dense_workspace((int)M, (int)L->n_rows, (int)L->k_cols, (int)L->group_size,
+                                    amode, epi, cus, false, slices);
+  };
+  if (lib_workspace(dev, bytes(), &ws, st)) {
+    slices = 1;  // a workspace that cannot grow now: no partials
+    if (int rc = lib_workspace(dev, bytes(), &ws, st)) return rc;
+  }
   cai4::GgArgs a{};
   a.w0 = packed;
   a.s0 = scales;
-  a.x = x;
+  a.x = static_cast<const uint16_t *>(x);
   a.y = y;
   a.M = (int)M;
   a.N = (int)L->n_rows;
@@ -845,14 +923,26 @@ int run_prefill(const cascadia_int4_layout *L, const uint8_t *packed, const uint
   a.G = (int)L->group_size;
   a.sdt = (int)L->scale_dtype;
   a.ldy = (int)L->n_rows;
-  a.epi = out_f32 ? cai4::GG_F32 : cai4::GG_BF16;
-  return hip_status(cai4::gg_dense(a, cai4::GG_A_BF16, ws, cus, st));
+  a.epi = epi;
+  return hip_status(cai4::gg_dense(a, amode, ws, cus, st, slices));
 }
 
-// Many tokens over MFMA-tiled weights: the tile GEMM (grouped.hip).
-bool prefill_shape(const cascadia_int4_layout *L, uint32_t seq) {
-  if (!L->tiling || seq < 64 || L->n_rows < 16) return false;
-  return cai4::gg_supported((int)L->k_cols, (int)L->group_size, 1);
+// A tile route that the library's workspace cannot grow for (a capture, no
+// memory): the call then takes the route it has without it.
+bool fall_back(int rc) { return rc == CASCADIA_INT4_ERR_ARG || rc == CASCADIA_INT4_ERR_NOMEM; }
+
+// Many rows over MFMA-tiled weights: the tile GEMM (grouped.hip), for bf16 rows
+// from 64 on, else where it pays (tiles_pay).
+bool prefill_shape(const cascadia_int4_layout *L, uint32_t seq, bool x_f32) {
+  if (!L->tiling || L->n_rows < 16 ||
+      !cai4::gg_supported((int)L->k_cols, (int)L->group_size, 1))
+    return false;
+  const int env = x_f32 ? cai4::tuning_env("CASCADIA_INT4_F32_TILE_TOKENS", 0)
+                        : cai4::tuning_env("CASCADIA_INT4_BF16_TILE_TOKENS", 0);
+  if (env > 0) return seq >= (uint32_t)env;
+  const size_t bytes = (size_t)L->n_rows * L->k_cols / 2;
+  if (x_f32) return tiles_pay(seq, 32, bytes, 17, (size_t)22 << 20);
+  return seq >= 64 || tiles_pay(seq, 64, bytes, 33, (size_t)22 << 20);
 }
 
 // ---- sparse-MoE layer ----
@@ -1408,6 +1498,13 @@ int cascadia_int4_dequant_gemm_multi(const cascadia_int4_layout *L, const uint8_
   if (!xs || !ys) return CASCADIA_INT4_ERR_NULL;
   if (seq == 0) return CASCADIA_INT4_ERR_ARG;  // the crate asserts seq >= 1
   if (!aligned(xs, 16) || !aligned(ys, 4)) return CASCADIA_INT4_ERR_ARG;
+  // many tokens over tiled weights: two planes through the tile GEMM, unless
+  // the library's workspace cannot grow to hold them (then, as for fewer
+  // tokens, the skinny kernel's passes)
+  if (prefill_shape(L, seq, true) && act_fits((int)seq, (int)L->k_cols, cai4::A_XF32)) {
+    const int rc = run_prefill(L, packed, scale_bits, xs, true, seq, ys, true, (hipStream_t)stream);
+    if (!fall_back(rc)) return rc;
+  }
   return run_gemm(packed, scale_bits, nullptr, nullptr, (int)L->n_rows, (int)L->k_cols,
                   (int)L->group_size, (int)L->scale_dtype, (int)L->tiling, xs, nullptr, cai4::A_XF32, (int)seq,
                   ys, nullptr, cai4::EPI_F32, (hipStream_t)stream);
@@ -1421,8 +1518,11 @@ int cascadia_int4_dequant_gemm_bf16in(const cascadia_int4_layout *L, const uint8
   if (!xs_bf16 || !ys) return CASCADIA_INT4_ERR_NULL;
   if (seq == 0) return CASCADIA_INT4_ERR_ARG;
   if (!aligned(xs_bf16, 16) || !aligned(ys, 4)) return CASCADIA_INT4_ERR_ARG;
-  if (prefill_shape(L, seq))
-    return run_prefill(L, packed, scale_bits, xs_bf16, seq, ys, true, (hipStream_t)stream);
+  if (prefill_shape(L, seq, false)) {
+    const int rc =
+        run_prefill(L, packed, scale_bits, xs_bf16, false, seq, ys, true, (hipStream_t)stream);
+    if (seq >= 64 || !fall_back(rc)) return rc;
+  }
   return run_gemm(packed, scale_bits, nullptr, nullptr, (int)L->n_rows, (int)L->k_cols,
                   (int)L->group_size, (int)L->scale_dtype, (int)L->tiling, xs_bf16, nullptr,
                   cai4::A_BF16,
@@ -1437,8 +1537,11 @@ int cascadia_int4_gemm_bf16(const cascadia_int4_layout *L, const uint8_t *packed
   if (!xs_bf16 || !ys_bf16) return CASCADIA_INT4_ERR_NULL;
   if (seq == 0) return CASCADIA_INT4_ERR_ARG;
   if (!aligned(xs_bf16, 16) || !aligned(ys_bf16, 2)) return CASCADIA_INT4_ERR_ARG;
-  if (prefill_shape(L, seq))
-    return run_prefill(L, packed, scale_bits, xs_bf16, seq, ys_bf16, false, (hipStream_t)stream);
+  if (prefill_shape(L, seq, false)) {
+    const int rc = run_prefill(L, packed, scale_bits, xs_bf16, false, seq, ys_bf16, false,
+                               (hipStream_t)stream);
+    if (seq >= 64 || !fall_back(rc)) return rc;
+  }
   return run_gemm(packed, scale_bits, nullptr, nullptr, (int)L->n_rows, (int)L->k_cols,
                   (int)L->group_size, (int)L->scale_dtype, (int)L->tiling, xs_bf16, nullptr,
                   cai4::A_BF16,
@@ -1556,11 +1659,11 @@ int cascadia_int4_expert_forward_noalloc(uint32_t hidden, uint32_t inter, uint32
   int dev;
   if (int rc = current_device(&dev)) return rc;
   const FfnWorkspace need = ffn_workspace(dev, hidden, inter, group_size, n_tokens, false);
-  if (need.total() > kNoAllocScratchBytes) return CASCADIA_INT4_ERR_ARG;
+  if (need.least() > kNoAllocScratchBytes) return CASCADIA_INT4_ERR_ARG;
   void *ws = nullptr;
   if (int rc = noalloc_scratch(dev, &ws)) return rc;
   return ffn_common(hidden, inter, group_size, scale_dtype, expert, x_bf16, false, n_tokens,
-                    out_bf16, true, ws, (hipStream_t)stream);
+                    out_bf16, true, ws, (hipStream_t)stream, kNoAllocScratchBytes);
 }
 
 int cascadia_int4_ffn_forward_f32(uint32_t hidden, uint32_t inter, uint32_t group_size,

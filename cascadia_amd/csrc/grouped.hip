@@ -8,8 +8,8 @@
 // exact products and f32 accumulation.
 //
 // Arithmetic: weights enter v_mfma_f32_32x32x16_bf16 as the exact bf16 value
-// 128 + nibble; each group's partial starts from the seed -136 * sum(x) over
-// the group's columns (computed once per row and group by gg_prep) and is
+// 128 + nibble (or 16 + nibble: gg_small_offset); each group's partial starts
+// from the seed -136 (-24) * sum(x) over the group's columns (computed once per row and group by gg_prep) and is
 // scaled in f32 when the group ends, acc += s * p.  A k-block of 128 columns is
 // four sub-steps of 32: a sub-step is dword s of every weight fragment.  Groups
 // of 32 or 64 columns end with a sub-step: the tiled layout stores those
@@ -136,6 +136,15 @@ struct Gg {
   static_assert(3 * BYTES <= 160 * 1024, "LDS");
 };
 
+// The hi plane of a split f32 value: x rounded to bf16 (to nearest even: the lo
+// plane, bf16 of the exact remainder, then holds x to half the error that a
+// truncated hi leaves it), truncated where rounding would reach infinity.
+CAI4_DEV uint32_t split_hi(float x) {
+  const uint32_t b = fbits(x), r = (b + 0x7FFFu + ((b >> 16) & 1u)) >> 16;
+  return (r & 0x7F80u) == 0x7F80u ? b >> 16 : r;
+}
+CAI4_DEV uint32_t split_lo(float x, uint32_t hi) { return f32_to_bf16_rne(x - bitsf(hi << 16)); }
+
 // Keeps these values' computation in its slot: the instruction selector orders
 // arithmetic freely between scheduling barriers unless something there uses it.
 CAI4_DEV void gg_pin(float &a, float &b, float &c, float &d, float &e, float &f, float &g,
@@ -155,6 +164,32 @@ CAI4_DEV T lds_at(uint32_t at, int off) {
 }
 
 constexpr uint32_t kGgOOB = 0x80000000u;  // an offset past every range: no data moves
+
+// The weights' encoding: bf16 128 + n (0x43 over the nibble), offset 136 with
+// the zero point; or 16 + n (0x41 over 0x80 | n << 3), offset 24, one
+// instruction more per half fragment.  A group's partial starts at -offset *
+// sum(x) and comes down to sum((n - 8) x), so its f32 roundings grow with the
+// offset and the group: two planes in groups of 128 columns take the small one
+// (FFN 4096 x 14336, f32, 130 rows: 9.9e-6 off 64 bits with the large one, and
+// the skinny kernel, whose planes add up apart, 8.7e-6).
+constexpr bool gg_small_offset(int GPK, int PL) { return GPK == 1 && PL == 2; }
+constexpr float gg_seed_factor(int GPK, int PL) { return gg_small_offset(GPK, PL) ? -24.f : -136.f; }
+
+// Bytes of the low (0) or high (1) nibbles of w, encoded.
+template <bool SMALL>
+CAI4_DEV uint32_t gg_nibbles(uint32_t w, int hi) {
+  if constexpr (SMALL)
+    return ((hi ? w >> 1 : w << 3) & 0x78787878u) | 0x80808080u;
+  else
+    return (hi ? w >> 4 : w) & 0x0F0F0F0Fu;
+}
+template <bool SMALL>
+CAI4_DEV u32x4_t gg_decode8(uint32_t w) {
+  const uint32_t C = SMALL ? 0x41414141u : 0x43434343u;
+  const uint32_t t = gg_nibbles<SMALL>(w, 0), u = gg_nibbles<SMALL>(w, 1);
+  return u32x4_t{__builtin_amdgcn_perm(C, t, 0x04010400u), __builtin_amdgcn_perm(C, t, 0x04030402u),
+                 __builtin_amdgcn_perm(C, u, 0x04010400u), __builtin_amdgcn_perm(C, u, 0x04030402u)};
+}
 
 struct GgTrue { static constexpr bool value = true; };
 struct GgFalse { static constexpr bool value = false; };
@@ -313,14 +348,20 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gg_kernel(GgArgs a) {
   const uint32_t xx = lds0 + P::X + (uint32_t)(wm * P::RM + 4 * h) * 4;
 
   float acc[MT][2][16];
-  f32x16_t p[MT][2], seed[MT];
+  // With one M-tile there are registers for two sets of partials: groups that
+  // end with a sub-step (GPK 2, 4) alternate, so that a group's adds spread
+  // over the next one's slots
+  constexpr int PB = MT == 1 && GPK > 1 ? 2 : 1;
+  f32x16_t p[PB][MT][2], seed[MT];
 #pragma unroll
   for (int i = 0; i < MT; ++i)
 #pragma unroll
     for (int j = 0; j < 2; ++j)
 #pragma unroll
-      for (int v = 0; v < 16; ++v) acc[i][j][v] = p[i][j][v] = 0.f;
+      for (int v = 0; v < 16; ++v) acc[i][j][v] = p[0][i][j][v] = p[PB - 1][i][j][v] = 0.f;
   u32x4_t af[2][P::NT][2], b[2][2], d[PL == 2 ? 4 : 2];
+  constexpr bool SMALL = gg_small_offset(GPK, PL);
+  constexpr uint32_t C = SMALL ? 0x41414141u : 0x43434343u;
   uint32_t dx = 0, dy = 0;
   uint32_t su[2], sn[2];            // scale bits of the group in flight, of the next
   float sc[2] = {0.f, 0.f};         // scales of the group being added
@@ -342,10 +383,10 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gg_kernel(GgArgs a) {
     return lds_at<uint16_t>(from + sx, j * JT * 32 * GPK + g * 32);
   };
   // eight scaled adds: acc += s * p, half `c & 1` of tile (i, j)
-  auto add8 = [&](int c) {
+  auto add8 = [&](int c, int pb = 0) {
     const int i = MT == 2 ? (c >> 1) & 1 : 0, j = MT == 2 ? c >> 2 : c >> 1;
 #pragma unroll
-    for (int v = 0; v < 8; ++v) acc[i][j][8 * (c & 1) + v] += sc[j] * p[i][j][8 * (c & 1) + v];
+    for (int v = 0; v < 8; ++v) acc[i][j][8 * (c & 1) + v] += sc[j] * p[pb][i][j][8 * (c & 1) + v];
     float *o = &acc[i][j][8 * (c & 1)];
     gg_pin(o[0], o[1], o[2], o[3], o[4], o[5], o[6], o[7]);
   };
@@ -368,8 +409,8 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gg_kernel(GgArgs a) {
     sn[0] = read_scale(0, 0, 0);
     sn[1] = read_scale(0, 0, 1);
     // fragments decoded before the first slot: one ahead of their use (PL 2: two)
-    d[0] = decode8(b[0][0][0]);
-    if (PL == 2) d[1] = decode8(b[1][0][0]);
+    d[0] = gg_decode8<SMALL>(b[0][0][0]);
+    if (PL == 2) d[1] = gg_decode8<SMALL>(b[1][0][0]);
 
     // One k-block.  Slot n of a sub-step issues one MFMA and the work beside
     // it: half a weight fragment's decode (one or two fragments ahead), an LDS
@@ -384,7 +425,7 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gg_kernel(GgArgs a) {
       for (int s = 0; s < 4; ++s) {
         constexpr int SPG = 4 / GPK;  // sub-steps per group
         const bool first = s % SPG == 0, last = s % SPG == SPG - 1;
-        const int g = s / SPG;
+        const int g = s / SPG, pb = PB == 2 ? g & 1 : 0;
 #pragma unroll
         for (int n = 0; n < P::SLOTS; ++n) {
           constexpr int NT = P::NT, SL = P::SLOTS;
@@ -430,11 +471,15 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gg_kernel(GgArgs a) {
               add8(1), add8(2);
             }
           } else {
-            if (first && n == 0) add8(0), add8(1);
-            if (first && n == 1) add8(2), add8(3);
+            if (PB == 2) {
+              if (first && n >= SL / 8 && n < SL / 8 + 4) add8(n - SL / 8, pb ^ 1);
+            } else {
+              if (first && n == 0) add8(0), add8(1);
+              if (first && n == 1) add8(2), add8(3);
+            }
           }
-          p[i][j] = mfma32_bf16(af[s & 1][t][q], d[PL == 2 ? 2 * q + j : (2 * q + j) & 1],
-                                first && q == 0 && (PL == 1 || t == 0) ? seed[i] : p[i][j]);
+          p[pb][i][j] = mfma32_bf16(af[s & 1][t][q], d[PL == 2 ? 2 * q + j : (2 * q + j) & 1],
+                                    first && q == 0 && (PL == 1 || t == 0) ? seed[i] : p[pb][i][j]);
 #ifdef __HIP_DEVICE_COMPILE__
           // the seeds stay live past their last use: that MFMA must not take
           // their registers for its result (64 copies per k-block if it does)
@@ -454,17 +499,17 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gg_kernel(GgArgs a) {
           const uint32_t w = b[fj][fq][fs];
           u32x4_t &o = d[PL == 2 ? f & 3 : f & 1];
           if (NT == 1) {
-            o = decode8(w);
+            o = gg_decode8<SMALL>(w);
           } else if ((n & 1) == 0) {
-            const uint32_t lo = w & 0x0F0F0F0Fu;
-            dx = __builtin_amdgcn_perm(0x43434343u, lo, 0x04010400u);
-            dy = __builtin_amdgcn_perm(0x43434343u, lo, 0x04030402u);
+            const uint32_t lo = gg_nibbles<SMALL>(w, 0);
+            dx = __builtin_amdgcn_perm(C, lo, 0x04010400u);
+            dy = __builtin_amdgcn_perm(C, lo, 0x04030402u);
           } else {
-            const uint32_t hi = (w >> 4) & 0x0F0F0F0Fu;
+            const uint32_t hi = gg_nibbles<SMALL>(w, 1);
             o.x = dx;
             o.y = dy;
-            o.z = __builtin_amdgcn_perm(0x43434343u, hi, 0x04010400u);
-            o.w = __builtin_amdgcn_perm(0x43434343u, hi, 0x04030402u);
+            o.z = __builtin_amdgcn_perm(C, hi, 0x04010400u);
+            o.w = __builtin_amdgcn_perm(C, hi, 0x04030402u);
           }
           if (DMA && s == 3) {
 #pragma unroll
@@ -492,7 +537,7 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gg_kernel(GgArgs a) {
 #pragma unroll 1
     for (; kb < KE; ++kb) kblock(GgFalse{}, kb, 0);
 #pragma unroll
-    for (int c = MT == 2 ? 3 : 0; c < 4 * MT; ++c) add8(c);
+    for (int c = MT == 2 ? 3 : 0; c < 4 * MT; ++c) add8(c, PB - 1);
   } else {
     // no live rows in this wave's tiles: its loads and barriers only
     int g3 = GPK > 1 ? (kb0 + 3) * GPK : (kb0 + 3) / KPG, gr = GPK > 1 ? 0 : (kb0 + 3) % KPG;
@@ -535,8 +580,7 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gg_kernel(GgArgs a) {
       }
       return;
     }
-    // hi = h truncated, lo = RNE(h - hi) of h = silu(g) * u, through LDS so that
-    // the planes are stored 16 bytes a lane
+    // hi / lo of silu(g) * u, through LDS so that the planes are stored 16 bytes a lane
     constexpr int pitch = P::OUTC * 2 + 16;
     uint8_t *lo_t = st + P::BM * pitch;
     __syncthreads();  // every wave is past its last read of the stages
@@ -547,10 +591,10 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gg_kernel(GgArgs a) {
         for (int v = 0; v < 16; ++v) {
           const int m = wm * P::RM + 32 * i + 8 * (v >> 2) + 4 * h + (v & 3);
           const float y = silu_f32(acc[i][0][v]) * acc[i][1][v];
-          const uint32_t hb = fbits(y) >> 16;
+          const uint32_t hb = split_hi(y);
           const uint32_t o = m * pitch + (32 * wn + l31) * 2;
           *reinterpret_cast<uint16_t *>(st + o) = (uint16_t)hb;
-          *reinterpret_cast<uint16_t *>(lo_t + o) = (uint16_t)f32_to_bf16_rne(y - bitsf(hb << 16));
+          *reinterpret_cast<uint16_t *>(lo_t + o) = (uint16_t)split_lo(y, hb);
         }
     }
     __syncthreads();
@@ -570,7 +614,7 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gg_kernel(GgArgs a) {
                   sum8_bf16(*reinterpret_cast<const u32x4_t *>(lo_t + o));
         t = lane_group_sum<L>(t);
         if ((c & (L - 1)) == 0 && m < mrows && n < a.N)
-          a.seeds_out[(size_t)(n / (8 * L)) * a.seeds_rp + row0 + m] = -136.f * t;
+          a.seeds_out[(size_t)(n / (8 * L)) * a.seeds_rp + row0 + m] = gg_seed_factor(GPK, 2) * t;
       }
     }
   } else if (a.part || a.epi == GG_F32) {
@@ -609,38 +653,103 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gg_kernel(GgArgs a) {
   }
 }
 
-// y = sum over the ksplit partials, in slice order; bf16 (RNE) or f32.
+// The sum of the nsl slices' partials at part + i (slices `stride` apart), in
+// slice order; four slices' loads are issued before their adds (clamped: all in
+// range) and pinned there.
+CAI4_DEV f32x4_t sum_slices(const float *part, size_t stride, size_t i, int nsl) {
+  f32x4_t s = *reinterpret_cast<const f32x4_t *>(part + i);
+  for (int z0 = 1; z0 < nsl; z0 += 4) {
+    f32x4_t v[4];
+#pragma unroll
+    for (int z = 0; z < 4; ++z)
+      v[z] = *reinterpret_cast<const f32x4_t *>(part + (size_t)min(z0 + z, nsl - 1) * stride + i);
+#pragma unroll
+    for (int z = 0; z < 4; ++z) asm volatile("" : "+v"(v[z]));
+#pragma unroll
+    for (int z = 0; z < 4; ++z)
+      if (z0 + z < nsl) s += v[z];
+  }
+  return s;
+}
+
+// y = sum over the K slices' partials, in slice order; bf16 (RNE) or f32.
 __global__ __launch_bounds__(256) void gg_reduce_kernel(const float *part, void *y, int M, int N,
-                                                        int ldy, int ksplit, int out_f32) {
+                                                        int ldy, int nsl, int out_f32) {
   const size_t i = ((size_t)blockIdx.x * blockDim.x + threadIdx.x) * 4;
   const size_t n = (size_t)M * N;
   if (i >= n) return;  // n is a multiple of 4
-  f32x4_t s = *reinterpret_cast<const f32x4_t *>(part + i);
-  // ksplit <= 4: the other slices' loads all issued (clamped to the last
-  // slice) before the adds, which go in slice order
-  f32x4_t v[3];
-#pragma unroll
-  for (int z = 1; z < 4; ++z)
-    v[z - 1] = *reinterpret_cast<const f32x4_t *>(part + (size_t)min(z, ksplit - 1) * n + i);
-#pragma unroll
-  for (int z = 1; z < 4; ++z) asm volatile("" : "+v"(v[z - 1]));
-#pragma unroll
-  for (int z = 1; z < 4; ++z)
-    if (z < ksplit) s += v[z - 1];
+  const f32x4_t s = sum_slices(part, n, i, nsl);
   const size_t r = i / N, c = i - r * N;  // N % 4 == 0: the four stay in one row
   const size_t o = r * ldy + c;
   if (out_f32) {
     float *yf = reinterpret_cast<float *>(y) + o;
-    yf[0] = s.x;
-    yf[1] = s.y;
-    yf[2] = s.z;
-    yf[3] = s.w;
+    if (((uintptr_t)yf & 15) == 0) {
+      *reinterpret_cast<f32x4_t *>(yf) = s;
+    } else {
+      yf[0] = s.x;
+      yf[1] = s.y;
+      yf[2] = s.z;
+      yf[3] = s.w;
+    }
   } else {
     uint16_t *yb = reinterpret_cast<uint16_t *>(y) + o;
-    yb[0] = (uint16_t)f32_to_bf16_rne(s.x);
-    yb[1] = (uint16_t)f32_to_bf16_rne(s.y);
-    yb[2] = (uint16_t)f32_to_bf16_rne(s.z);
-    yb[3] = (uint16_t)f32_to_bf16_rne(s.w);
+    u32x2_t b;
+    b.x = f32_to_bf16_rne(s.x) | (f32_to_bf16_rne(s.y) << 16);
+    b.y = f32_to_bf16_rne(s.z) | (f32_to_bf16_rne(s.w) << 16);
+    if (((uintptr_t)yb & 7) == 0) {
+      *reinterpret_cast<u32x2_t *>(yb) = b;
+    } else {
+      yb[0] = (uint16_t)b.x;
+      yb[1] = (uint16_t)(b.x >> 16);
+      yb[2] = (uint16_t)b.y;
+      yb[3] = (uint16_t)(b.y >> 16);
+    }
+  }
+}
+
+// The SwiGLU of gate / up partials [nsl][M][gate N | up N], in slice order: the
+// hi / lo planes of silu(g) * u ([M, ldy]) and, with seeds, their seeds per
+// group of 8 L columns (N a multiple of 8 L): what the tile kernel's epilogue
+// writes when K is not split.  A thread per eight columns.
+template <int L>
+__global__ __launch_bounds__(256) void gg_swiglu_reduce_kernel(const float *part, uint16_t *hi,
+                                                               uint16_t *lo, float *seeds, int M,
+                                                               int N, int ldy, int nsl,
+                                                               int seeds_rp) {
+  const int per = N / 8;
+  const size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (t >= (size_t)M * per) return;  // whole groups of L lanes: per is a multiple of L
+  const size_t r = t / per;
+  const int c = 8 * (int)(t - r * per);
+  const size_t stride = (size_t)M * 2 * N, i = r * 2 * N + c;
+  float g[8], u[8];
+#pragma unroll
+  for (int q = 0; q < 2; ++q) {
+    const f32x4_t a = sum_slices(part, stride, i + 4 * q, nsl);
+    const f32x4_t b = sum_slices(part, stride, i + N + 4 * q, nsl);
+#pragma unroll
+    for (int v = 0; v < 4; ++v) g[4 * q + v] = a[v], u[4 * q + v] = b[v];
+  }
+  u32x4_t h, l;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    uint32_t hb[2], lb[2];
+#pragma unroll
+    for (int v = 0; v < 2; ++v) {
+      const float y = silu_f32(g[2 * e + v]) * u[2 * e + v];
+      hb[v] = split_hi(y);
+      lb[v] = split_lo(y, hb[v]);
+    }
+    h[e] = hb[0] | (hb[1] << 16);
+    l[e] = lb[0] | (lb[1] << 16);
+  }
+  const size_t o = r * ldy + c;
+  *reinterpret_cast<u32x4_t *>(hi + o) = h;
+  *reinterpret_cast<u32x4_t *>(lo + o) = l;
+  if (seeds) {
+    const float sum = lane_group_sum<L>(sum8_bf16(h) + sum8_bf16(l));
+    if ((t & (L - 1)) == 0)
+      seeds[(size_t)(c / (8 * L)) * seeds_rp + r] = gg_seed_factor(16 / L, 2) * sum;
   }
 }
 
@@ -700,8 +809,15 @@ __global__ __launch_bounds__(256) void gg_prep_kernel(int mode, const void *src,
       if (c < K) *reinterpret_cast<u32x4_t *>(out + (size_t)r * K + c) = o;
       t = sum8_bf16(o);
     } else {
-      const f32x4_t fa = __builtin_bit_cast(f32x4_t, v[q]), fb = __builtin_bit_cast(f32x4_t, w[q]);
-      const u32x4_t hi = act_split_f32_nat(fa, fb, false), lo = act_split_f32_nat(fa, fb, true);
+      u32x4_t hi, lo;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const float x0 = bitsf(e < 2 ? v[q][2 * e] : w[q][2 * e - 4]);
+        const float x1 = bitsf(e < 2 ? v[q][2 * e + 1] : w[q][2 * e - 3]);
+        const uint32_t h0 = split_hi(x0), h1 = split_hi(x1);
+        hi[e] = h0 | (h1 << 16);
+        lo[e] = split_lo(x0, h0) | (split_lo(x1, h1) << 16);
+      }
       if (c < K) {
         *reinterpret_cast<u32x4_t *>(out + (size_t)r * K + c) = hi;
         *reinterpret_cast<u32x4_t *>(out2 + (size_t)r * K + c) = lo;
@@ -709,7 +825,9 @@ __global__ __launch_bounds__(256) void gg_prep_kernel(int mode, const void *src,
       t = sum8_bf16(hi) + sum8_bf16(lo);
     }
     t = lane_group_sum<L>(t);
-    if ((lane & (L - 1)) == 0 && c < K) seeds[(size_t)(c / gw) * rows_pad + r] = -136.f * t;
+    if ((lane & (L - 1)) == 0 && c < K)
+      seeds[(size_t)(c / gw) * rows_pad + r] =
+          (mode & 1 ? gg_seed_factor(16 / L, 2) : gg_seed_factor(16 / L, 1)) * t;
   }
 }
 
@@ -736,17 +854,42 @@ hipError_t gg_launch_g(const GgArgs &a, int rows_y, int nsl, hipStream_t st) {
   }
 }
 
-// Dense tile shapes (rows x output columns): 128 x 256 (8 waves) in up to 4
-// slices of K when the tiles alone leave CUs idle, else 128 x 128 or 64 x 128
-// (4 waves).  Two-plane A: 64 x 256.
-int gg_dense_ksplit(int M, int N, int K, int num_cus) {
-  const long tiles = (long)((N + 255) / 256) * ((M + 127) / 128);
-  const int KB = K / 128;
-  for (int s = 1; s <= 4; ++s) {
-    if (s > 1 && (KB / s < 6 || N % 4)) break;
-    if (8 * tiles * s >= 7L * num_cus) return s;
+// How a dense GEMM runs: the tile and the slices of K.
+struct GgPlan {
+  bool small;  // one-plane, not SwiGLU: 64 x 128 tiles (4 waves, two workgroups per CU)
+  int nsl, kper;
+};
+
+// The plan with the least estimated time, from times measured on the card: a
+// k-block of a 128 x 256 (64 x 256 with two planes, 64 x 128) tile, a tile's
+// prologue and epilogue, and the reduce launch with its partials written and
+// read.  Slices of at least four k-blocks (the pipeline's depth), at most
+// eight.  max_slices 1: no partials (a workspace that cannot grow).
+GgPlan gg_plan(int M, int N, int K, int G, bool two, bool sw, int num_cus, int max_slices) {
+  const int KB = K / 128, ncol = sw ? 2 * N : N;
+  const double tkb128 = G == 32 ? 2.4 : G == 64 ? 1.9 : 1.5;
+  const double tkb64x2 = G == 32 ? 1.6 : 1.4, tkb_small = G == 32 ? 1.8 : 1.25;
+  constexpr double kTile = 6.0, kReduce = 3.0, kBytesPerUs = 1.2e7;
+  GgPlan best{false, 1, KB};
+  double best_t = -1.0;
+  for (int small = 0; small < (two || sw ? 1 : 2); ++small) {
+    const int bm = small || two ? 64 : 128, bn = small ? 128 : sw ? 128 : 256;
+    const long tiles = (long)((N + bn - 1) / bn) * ((M + bm - 1) / bm);
+    const long slots = small ? 2L * num_cus : num_cus;
+    const double tkb = small ? tkb_small : two ? tkb64x2 : tkb128;
+    for (int s = 1; s <= max_slices && s <= 8; ++s) {
+      if (s > 1 && (KB / s < 4 || N % 4)) break;
+      const int kper = (KB + s - 1) / s, nsl = (KB + kper - 1) / kper;
+      const long rounds = (tiles * nsl + slots - 1) / slots;
+      double t = rounds * (kper * tkb + kTile);
+      if (nsl > 1) t += kReduce + (double)nsl * M * ncol * 8.0 / kBytesPerUs;
+      if (best_t < 0 || t < best_t) {
+        best_t = t;
+        best = GgPlan{small != 0, nsl, kper};
+      }
+    }
   }
-  return 0;
+  return best;
 }
 
 }  // namespace
@@ -779,68 +922,82 @@ namespace {
 size_t al256(size_t v) { return (v + 255) & ~(size_t)255; }
 }  // namespace
 
-size_t gg_dense_workspace(int M, int N, int K, int G, int amode, int epi, int num_cus) {
-  const int gw = gg_group_width(G);
-  size_t b = al256((size_t)(K / gw) * gg_rows_pad(M) * 4);
+size_t gg_dense_workspace(int M, int N, int K, int G, int amode, int epi, int num_cus,
+                          bool have_seeds, int max_slices) {
+  const bool sw = epi == GG_SWIGLU_HILO;
+  size_t b = have_seeds ? 0 : al256((size_t)(K / gg_group_width(G)) * gg_rows_pad(M) * 4);
   if (amode == GG_A_F32) b += 2 * al256((size_t)M * K * 2);  // the A planes
-  const int ks = (amode != GG_A_BF16 || epi == GG_SWIGLU_HILO) ? 1
-                                                               : gg_dense_ksplit(M, N, K, num_cus);
-  return b + (ks > 1 ? (size_t)ks * M * N * 4 : 0);
+  const GgPlan p = gg_plan(M, N, K, G, amode != GG_A_BF16, sw, num_cus, max_slices);
+  return b + (p.nsl > 1 ? (size_t)p.nsl * M * (sw ? 2 * (size_t)N : N) * 4 : 0);
 }
 
-hipError_t gg_dense(GgArgs a, int amode, void *ws, int num_cus, hipStream_t st) {
-  a.rows_pad = gg_rows_pad(a.M);
-  a.seeds_out = nullptr;  // (the dense FFN's down makes its own seeds)
+hipError_t gg_dense(GgArgs a, int amode, void *ws, int num_cus, hipStream_t st, int max_slices) {
   a.row_map = nullptr;
-  uint8_t *w = static_cast<uint8_t *>(ws);
-  float *seeds = reinterpret_cast<float *>(w);
-  a.seeds = seeds;
-  w += al256((size_t)(a.K / gg_group_width(a.G)) * a.rows_pad * 4);
   a.tiles = nullptr;
   a.tile_split = 1;
-  a.kper = a.K / 128;
-  a.part = nullptr;
   a.hilo = amode != GG_A_BF16;
   const bool sw = a.epi == GG_SWIGLU_HILO;
-  if (a.hilo) {
+  if (a.seeds_out && !sw) return hipErrorInvalidValue;
+  uint8_t *w = static_cast<uint8_t *>(ws);
+  if (!a.seeds) {
+    a.rows_pad = gg_rows_pad(a.M);
+    float *seeds = reinterpret_cast<float *>(w);
+    a.seeds = seeds;
+    w += al256((size_t)(a.K / gg_group_width(a.G)) * a.rows_pad * 4);
+    hipError_t e;
     if (amode == GG_A_F32) {
       uint16_t *hi = reinterpret_cast<uint16_t *>(w);
-      uint16_t *lo = reinterpret_cast<uint16_t *>(w + al256((size_t)a.M * a.K * 2));
-      if (hipError_t e = gg_prep(3, a.x, nullptr, nullptr, hi, lo, seeds, a.M, a.rows_pad, a.K,
-                                 a.G, nullptr, st))
-        return e;
+      w += al256((size_t)a.M * a.K * 2);
+      uint16_t *lo = reinterpret_cast<uint16_t *>(w);
+      w += al256((size_t)a.M * a.K * 2);
+      e = gg_prep(3, a.x, nullptr, nullptr, hi, lo, seeds, a.M, a.rows_pad, a.K, a.G, nullptr, st);
       a.x = hi;
       a.x2 = lo;
-    } else if (hipError_t e = gg_prep(1, a.x, a.x2, nullptr, nullptr, nullptr, seeds, a.M,
-                                      a.rows_pad, a.K, a.G, nullptr, st)) {
-      return e;
+    } else {
+      e = gg_prep(a.hilo ? 1 : 0, a.x, a.x2, nullptr, nullptr, nullptr, seeds, a.M, a.rows_pad,
+                  a.K, a.G, nullptr, st);
     }
-    if (sw) return gg_launch_g<1, 2, 4, 2, true>(a, 0, 1, st);
-    return gg_launch_g<1, 2, 4, 2, false>(a, 0, 1, st);
+    if (e != hipSuccess) return e;
+  } else if (amode == GG_A_F32) {
+    return hipErrorInvalidValue;  // the planes are made here, their seeds with them
   }
-  if (hipError_t e = gg_prep(0, a.x, nullptr, nullptr, nullptr, nullptr, seeds, a.M, a.rows_pad,
-                             a.K, a.G, nullptr, st))
-    return e;
-  if (sw)
-    return gg_launch_g<2, 2, 4, 1, true>(a, 0, 1, st);
-  const int ks = gg_dense_ksplit(a.M, a.N, a.K, num_cus);
-  if (ks >= 1) {
-    int nsl = 1;
-    if (ks > 1) {
-      a.kper = (a.K / 128 + ks - 1) / ks;
-      nsl = (a.K / 128 + a.kper - 1) / a.kper;
-      a.part = reinterpret_cast<float *>(w);
+  const GgPlan p = gg_plan(a.M, a.N, a.K, a.G, a.hilo, sw, num_cus, max_slices);
+  a.kper = p.kper;
+  a.part = p.nsl > 1 ? reinterpret_cast<float *>(w) : nullptr;
+  hipError_t e;
+  if (a.hilo)
+    e = sw ? gg_launch_g<1, 2, 4, 2, true>(a, 0, p.nsl, st)
+           : gg_launch_g<1, 2, 4, 2, false>(a, 0, p.nsl, st);
+  else if (sw)
+    e = gg_launch_g<2, 2, 4, 1, true>(a, 0, p.nsl, st);
+  else if (p.small)
+    e = gg_launch_g<1, 2, 2, 1, false>(a, 0, p.nsl, st);
+  else
+    e = gg_launch_g<2, 2, 4, 1, false>(a, 0, p.nsl, st);
+  if (e != hipSuccess || p.nsl == 1) return e;
+  if (sw) {
+    const size_t n = (size_t)a.M * (a.N / 8);
+    const dim3 grid((unsigned)((n + 255) / 256)), block(256);
+    uint16_t *hi = static_cast<uint16_t *>(a.y), *lo = static_cast<uint16_t *>(a.y2);
+    switch (gg_group_width(a.G)) {
+      case 32:
+        hipLaunchKernelGGL(gg_swiglu_reduce_kernel<4>, grid, block, 0, st, a.part, hi, lo,
+                           a.seeds_out, a.M, a.N, a.ldy, p.nsl, a.seeds_rp);
+        break;
+      case 64:
+        hipLaunchKernelGGL(gg_swiglu_reduce_kernel<8>, grid, block, 0, st, a.part, hi, lo,
+                           a.seeds_out, a.M, a.N, a.ldy, p.nsl, a.seeds_rp);
+        break;
+      default:
+        hipLaunchKernelGGL(gg_swiglu_reduce_kernel<16>, grid, block, 0, st, a.part, hi, lo,
+                           a.seeds_out, a.M, a.N, a.ldy, p.nsl, a.seeds_rp);
     }
-    if (hipError_t e = gg_launch_g<2, 2, 4, 1, false>(a, 0, nsl, st)) return e;
-    if (nsl > 1) {
-      const size_t n = (size_t)a.M * a.N;
-      hipLaunchKernelGGL(gg_reduce_kernel, dim3((unsigned)((n / 4 + 255) / 256)), dim3(256), 0,
-                         st, a.part, a.y, a.M, a.N, a.ldy, nsl, a.epi == GG_F32 ? 1 : 0);
-      return hipGetLastError();
-    }
-    return hipSuccess;
+    return hipGetLastError();
   }
-  return gg_launch_g<1, 2, 2, 1, false>(a, 0, 1, st);
+  const size_t n = (size_t)a.M * a.N;
+  hipLaunchKernelGGL(gg_reduce_kernel, dim3((unsigned)((n / 4 + 255) / 256)), dim3(256), 0, st,
+                     a.part, a.y, a.M, a.N, a.ldy, p.nsl, a.epi == GG_F32 ? 1 : 0);
+  return hipGetLastError();
 }
 
 hipError_t gg_grouped(const GgArgs &a0, int max_tiles, hipStream_t st) {

@@ -11,7 +11,7 @@
 namespace cai4 {
 
 // Output of a GEMM: f32, bf16 (RNE), or -- for a gate/up pair -- SwiGLU as the
-// two bf16 planes hi = trunc(h), lo = RNE(h - hi) of h = silu(gate) * up.
+// two bf16 planes hi = bf16(h), lo = bf16(h - hi) of h = silu(gate) * up.
 enum GgEpi { GG_F32 = 0, GG_BF16 = 1, GG_SWIGLU_HILO = 2 };
 
 struct GgArgs {
@@ -21,7 +21,7 @@ struct GgArgs {
   size_t estride;
   const uint16_t *x;   // A: bf16 [rows, K] (the hi plane with hilo)
   const uint16_t *x2;  // hilo: the lo plane
-  const float *seeds;  // [K / gw][rows_pad]: -136 * sum of A over each group of gw columns
+  const float *seeds;  // [K / gw][rows_pad]: the zero point's share of each group's sum (grouped.hip)
   void *y, *y2;        // [rows, ldy]: f32 / bf16, or the hi / lo planes (SwiGLU)
   const SkinnyChunk *tiles;  // grouped: one (expert, row0, count) per workgroup row; null: dense
   int tile_split;  // grouped: workgroup rows per table entry (the entry's rows in BM parts)
@@ -72,10 +72,15 @@ constexpr int kGgChunkRows = 128;
 // hi / lo planes in the workspace); hi / lo planes a.x / a.x2.
 enum GgAMode { GG_A_BF16 = 0, GG_A_F32 = 1, GG_A_PLANES = 2 };
 
-// Dense: workspace bytes (seeds, split planes, split-K partials) and the
-// launches (gg_prep, the GEMM, the split-K reduce).
-size_t gg_dense_workspace(int M, int N, int K, int G, int amode, int epi, int num_cus);
-hipError_t gg_dense(GgArgs a, int amode, void *ws, int num_cus, hipStream_t st);
+// Dense: workspace bytes (seeds unless the caller has them, split planes,
+// split-K partials) and the launches (gg_prep unless a.seeds is given, the
+// GEMM, the split-K reduce).  With GG_SWIGLU_HILO and a.seeds_out the seeds of
+// the planes written are left there.  max_slices 1: no split of K (no
+// partials), for a workspace that cannot grow.
+size_t gg_dense_workspace(int M, int N, int K, int G, int amode, int epi, int num_cus,
+                          bool have_seeds = false, int max_slices = 8);
+hipError_t gg_dense(GgArgs a, int amode, void *ws, int num_cus, hipStream_t st,
+                    int max_slices = 8);
 
 // Grouped: tiles = max_tiles entries (count 0: empty) of at most
 // 128 rows; a.seeds over a.rows_pad rows made by gg_prep.

@@ -93,6 +93,75 @@ def test_gemm_tile_edges(cl, orc, n, k, g, sdt, M):
                       f"bf16 out {n}x{k} G{g} M{M}")
 
 
+@pytest.mark.parametrize("n,k,g,sdt,M", [
+    (16, 128, 128, BF16, 17), (33, 384, 32, F16, 63), (300, 1024, 64, BF16, 64),
+    (1000, 4096, 32, BF16, 65), (257, 2048, 256, F16, 130)])
+def test_gemm_f32_tiles(cl, orc, tuning, n, k, g, sdt, M):
+    """f32 rows over tiled weights as two planes through the tile GEMM, whole
+    and with K split (long K, few tiles), against the oracle.  The planes hold x
+    to 2^-18 of its size and the sums are f32: 1e-5 of the result's norm."""
+    tuning("CASCADIA_INT4_F32_TILE_TOKENS", "17")
+    packed = orc.fill_bytes(n + M, 3, n * k // 2)
+    scales = orc.fill_scales(n + M, 4, n * (k // g), sdt).view(np.uint8).copy()
+    pt, st = cl.tile_weights(dev(packed), dev(scales), n, k, g)
+    xs = orc.fill_normal_f32(k, M, M * k)
+    want = orc.gemm_multi(packed, scales, xs, n, k, M, g, sdt)
+    ys = torch.empty(M * n, dtype=torch.float32, device="cuda")
+    cl.dequant_gemm_int4_multi_auto(pt, st, dev(xs), n, k, M, ys, group_size=g, scale_dtype=sdt,
+                                    tiling=cl.TILING_MFMA)
+    got = host(ys).reshape(M, n)
+    assert_f32_close(got, want, f"f32 tiles {n}x{k} G{g} M{M}")
+    assert rel_l2(got, want) <= 1e-5
+
+
+def test_gemm_f32_capture(cl, orc):
+    """A stream capture cannot grow the library's workspace: the f32 GEMM of a
+    shape not seen before is recorded all the same (without the tile route if
+    need be), and every replay gives the eager result."""
+    n, k, g, M = 3000, 4096, 128, 333
+    packed = orc.fill_bytes(5, 5, n * k // 2)
+    scales = orc.fill_scales(5, 6, n * (k // g), F16).view(np.uint8).copy()
+    pt, st = cl.tile_weights(dev(packed), dev(scales), n, k, g)
+    xs = orc.fill_normal_f32(5, 7, M * k)
+    xd = dev(xs)
+    want = orc.gemm_multi(packed, scales, xs, n, k, M, g, F16)
+    ys = torch.empty(M * n, dtype=torch.float32, device="cuda")
+    call = lambda: cl.dequant_gemm_int4_multi_auto(  # noqa: E731
+        pt, st, xd, n, k, M, ys, group_size=g, scale_dtype=F16, tiling=cl.TILING_MFMA)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        call()
+    for _ in range(3):
+        ys.zero_()
+        graph.replay()
+        assert_f32_close(host(ys).reshape(M, n), want, "replay")
+        call()
+        assert_f32_close(host(ys).reshape(M, n), want, "eager")
+
+
+@pytest.mark.parametrize("M,h,i,g", [(33, 2048, 1024, 32), (100, 1024, 2048, 64),
+                                     (161, 2048, 1536, 128)])
+def test_ffn_split_tiles(cl, orc, tuning, M, h, i, g):
+    """An FFN whose gate/up and down split K (few tiles): the SwiGLU and the
+    planes' seeds made by the reduce, bf16 and f32 rows."""
+    tuning("CASCADIA_INT4_FFN_TILE_TOKENS", "33")
+    flat = expert(orc, h, i, g, F16, M + g)
+    W = cl.ExpertWeights(dev(flat), h, i, g, F16).tiled()
+    xb = orc.fill_normal_bf16(M, 52, M * h)
+    out = torch.empty(M * h, dtype=torch.int16, device="cuda")
+    cl.expert_forward(dev(xb.view(np.int16).reshape(M, h)), *W.slices(), out, group_size=g,
+                      scale_dtype=F16, tiling=cl.TILING_MFMA)
+    assert_bf16_close(host(out).view(np.uint16).reshape(M, h),
+                      orc.cpu_expert_forward(xb, M, flat, h, i, g, F16), f"split M{M} G{g}")
+    x = orc.fill_normal_f32(8, M, M * h).reshape(M, h)
+    of = torch.empty((M, h), dtype=torch.float32, device="cuda")
+    cl.ffn_forward_sparse_f32(dev(x), h, i, *W.slices(), of, 0.0, group_size=g, scale_dtype=F16,
+                              tiling=cl.TILING_MFMA)
+    want = np.stack([orc.ffn_forward_f32(x[t], flat, h, i, g, F16)[0] for t in range(M)])
+    assert_f32_close(host(of), want, f"split f32 M{M} G{g}")
+
+
 @pytest.mark.parametrize("M,g", [(65, 32), (100, 64), (200, 128)])
 def test_ffn_f32_tiles(cl, orc, tuning, M, g):
     """The f32-in / f32-out FFN (the shared expert) over M rows: x split into
