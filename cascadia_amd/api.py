@@ -13,6 +13,7 @@ libcascadia_int4_hip.so.
 from __future__ import annotations
 
 import ctypes as C
+import functools
 
 import numpy as np
 import torch
@@ -28,12 +29,21 @@ GROUP_SIZE = 32
 NIBBLES_PER_INT32 = 8
 
 
+# The current stream's handle without building a Stream object per call (a
+# decode call is a few microseconds of GPU time; measured, torch's
+# current_stream().cuda_stream was about 1.5 of the 10.8 us of a GEMV call).
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+_cur_device = getattr(torch._C, "_cuda_getDevice", None)
+
+
 def _stream() -> int:
-    return torch.cuda.current_stream().cuda_stream
+    if _raw_stream is None or _cur_device is None or not torch.cuda.is_initialized():
+        return torch.cuda.current_stream().cuda_stream
+    return _raw_stream(_cur_device())
 
 
 def _nbytes(t: torch.Tensor) -> int:
-    return t.numel() * t.element_size()
+    return t.nbytes
 
 
 def _dev(t: torch.Tensor, name: str) -> torch.Tensor:
@@ -53,29 +63,48 @@ def _is_bf16_bits(t: torch.Tensor) -> bool:
     return t.dtype in (torch.bfloat16, torch.int16, torch.uint16)
 
 
-def _layout(n_rows, k_cols, group_size, scale_dtype, tiling=TILING_CRATE) -> Layout:
-    return Layout(n_rows, k_cols, group_size, scale_dtype, tiling)
+@functools.lru_cache(maxsize=1024, typed=True)
+def _layout_of(n_rows, k_cols, group_size, scale_dtype, tiling):
+    L = Layout(n_rows, k_cols, group_size, scale_dtype, tiling)
+    return L, C.byref(L)  # (the struct is kept with its reference)
+
+
+def _layout(n_rows, k_cols, group_size, scale_dtype, tiling=TILING_CRATE):
+    """A reference to the layout struct of these values, made once per set of
+    values (the library only reads it)."""
+    return _layout_of(n_rows, k_cols, group_size, scale_dtype, tiling)[1]
 
 
 def tiled_sizes(n_rows, k_cols, group_size=GROUP_SIZE):
     """(packed, scale) byte sizes of the MFMA-tiled copy of a matrix."""
+    if (type(n_rows) is int and type(k_cols) is int and type(group_size) is int
+            and 0 < n_rows <= 1 << 30 and 0 < k_cols <= 1 << 30 and group_size > 0
+            and group_size % 32 == 0 and k_cols % group_size == 0):
+        # 16-row by 128-column blocks of 1 KB; 32 bytes of scales per tile and group
+        tiles = (n_rows + 15) // 16
+        return tiles * ((k_cols + 127) // 128) * 1024, tiles * (k_cols // group_size) * 32
+    # anything else: the library's own checks and error
     pb, sb = C.c_size_t(), C.c_size_t()
     L = _layout(n_rows, k_cols, group_size, SCALE_BF16)
-    check("cascadia_int4_tiled_sizes", lib().cascadia_int4_tiled_sizes(C.byref(L), C.byref(pb), C.byref(sb)))
+    check("cascadia_int4_tiled_sizes", lib().cascadia_int4_tiled_sizes(L, C.byref(pb), C.byref(sb)))
     return pb.value, sb.value
 
 
 def _check_weights(packed, scale_bits, n_rows, k_cols, group_size, tiling=TILING_CRATE):
+    # (messages are built only when they are raised: this runs in every call)
     _dev(packed, "packed")
     _dev(scale_bits, "scale_bits")
-    _expect(group_size % 32 == 0 and k_cols % group_size == 0,
-            f"k_cols {k_cols} must be a multiple of group_size {group_size} (a multiple of 32)")
+    if not (group_size % 32 == 0 and k_cols % group_size == 0):
+        raise ValueError(f"k_cols {k_cols} must be a multiple of group_size {group_size} "
+                         "(a multiple of 32)")
     if tiling == TILING_MFMA:
         pb, sb = tiled_sizes(n_rows, k_cols, group_size)
     else:
         pb, sb = n_rows * (k_cols // 2), n_rows * (k_cols // group_size) * 2
-    _expect(_nbytes(packed) == pb, f"packed has {_nbytes(packed)} bytes, expected {pb}")
-    _expect(_nbytes(scale_bits) == sb, f"scale_bits has {_nbytes(scale_bits)} bytes, expected {sb}")
+    if packed.nbytes != pb:
+        raise ValueError(f"packed has {packed.nbytes} bytes, expected {pb}")
+    if scale_bits.nbytes != sb:
+        raise ValueError(f"scale_bits has {scale_bits.nbytes} bytes, expected {sb}")
 
 
 def tile_weights(packed, scale_bits, n_rows, k_cols, group_size=GROUP_SIZE):
@@ -86,7 +115,7 @@ def tile_weights(packed, scale_bits, n_rows, k_cols, group_size=GROUP_SIZE):
     st = torch.empty(sb, dtype=torch.uint8, device=packed.device)
     L = _layout(n_rows, k_cols, group_size, SCALE_BF16)
     check("cascadia_int4_tile_weights", lib().cascadia_int4_tile_weights(
-        C.byref(L), packed.data_ptr(), scale_bits.data_ptr(), pt.data_ptr(), st.data_ptr(),
+        L, packed.data_ptr(), scale_bits.data_ptr(), pt.data_ptr(), st.data_ptr(),
         _stream()))
     return pt, st
 
@@ -104,7 +133,7 @@ def dequant_gemv_int4(packed, scale_bits, x, n_rows, k_cols, y, group_size=GROUP
     _expect(y.dtype == torch.float32 and y.numel() == n_rows, "y must be f32 [n_rows]")
     L = _layout(n_rows, k_cols, group_size, scale_dtype, tiling)
     check("cascadia_int4_dequant_gemv", lib().cascadia_int4_dequant_gemv(
-        C.byref(L), packed.data_ptr(), scale_bits.data_ptr(), x.data_ptr(), y.data_ptr(),
+        L, packed.data_ptr(), scale_bits.data_ptr(), x.data_ptr(), y.data_ptr(),
         _stream()))
     return y
 
@@ -127,7 +156,7 @@ def dequant_gemv_int4_rows_subset(packed, scale_bits, x, n_rows, k_cols, y, acti
             "active_rows must hold 32-bit row ids")
     L = _layout(n_rows, k_cols, group_size, scale_dtype, tiling)
     check("cascadia_int4_dequant_gemv_rows_subset", lib().cascadia_int4_dequant_gemv_rows_subset(
-        C.byref(L), packed.data_ptr(), scale_bits.data_ptr(), x.data_ptr(), y.data_ptr(),
+        L, packed.data_ptr(), scale_bits.data_ptr(), x.data_ptr(), y.data_ptr(),
         active_rows.data_ptr(), active_rows.numel(), _stream()))
     return y
 
@@ -263,16 +292,17 @@ def dequant_gemm_int4_multi_auto(packed, scale_bits, xs, n_rows, k_cols, seq, ys
     _check_weights(packed, scale_bits, n_rows, k_cols, group_size, tiling)
     _dev(xs, "xs"), _dev(ys, "ys")
     _expect(seq >= 1, "seq must be >= 1")
-    _expect(xs.numel() == seq * k_cols, f"xs must hold seq*k_cols = {seq * k_cols} values")
-    _expect(ys.dtype == torch.float32 and ys.numel() == seq * n_rows,
-            f"ys must be f32 [seq*n_rows = {seq * n_rows}]")
+    if xs.numel() != seq * k_cols:
+        raise ValueError(f"xs must hold seq*k_cols = {seq * k_cols} values")
+    if not (ys.dtype == torch.float32 and ys.numel() == seq * n_rows):
+        raise ValueError(f"ys must be f32 [seq*n_rows = {seq * n_rows}]")
     L = _layout(n_rows, k_cols, group_size, scale_dtype, tiling)
     if xs.dtype == torch.float32:
         fn = "cascadia_int4_dequant_gemm_multi"
     else:
         _expect(_is_bf16_bits(xs), "xs must be f32 or bf16")
         fn = "cascadia_int4_dequant_gemm_bf16in"
-    check(fn, getattr(lib(), fn)(C.byref(L), packed.data_ptr(), scale_bits.data_ptr(),
+    check(fn, getattr(lib(), fn)(L, packed.data_ptr(), scale_bits.data_ptr(),
                                  xs.data_ptr(), seq, ys.data_ptr(), _stream()))
     return ys
 
@@ -289,7 +319,7 @@ def gemm_int4_bf16(packed, scale_bits, xs_bf16, n_rows, k_cols, seq, ys_bf16,
     _expect(_is_bf16_bits(ys_bf16) and ys_bf16.numel() == seq * n_rows, "ys_bf16 [seq, n_rows] bf16")
     L = _layout(n_rows, k_cols, group_size, scale_dtype, tiling)
     check("cascadia_int4_gemm_bf16", lib().cascadia_int4_gemm_bf16(
-        C.byref(L), packed.data_ptr(), scale_bits.data_ptr(), xs_bf16.data_ptr(), seq,
+        L, packed.data_ptr(), scale_bits.data_ptr(), xs_bf16.data_ptr(), seq,
         ys_bf16.data_ptr(), _stream()))
     return ys_bf16
 
@@ -405,7 +435,7 @@ class ExpertWeights:
         for src_i, (n, k) in ((0, (I, H)), (4, (H, I))):  # gate and down tiled
             L = _layout(n, k, G, self.scale_dtype)
             check("cascadia_int4_tile_weights", lib().cascadia_int4_tile_weights(
-                C.byref(L), self._slices[src_i].data_ptr(), self._slices[src_i + 1].data_ptr(),
+                L, self._slices[src_i].data_ptr(), self._slices[src_i + 1].data_ptr(),
                 dst.data_ptr() + o[src_i], dst.data_ptr() + o[src_i + 1], _stream()))
         for j in (2, 3):  # up as it is
             dst[o[j]:o[j] + sz[j]].copy_(self._slices[j])
@@ -906,7 +936,7 @@ def debug_dequant(packed, scale_bits, n_rows, k_cols, group_size=GROUP_SIZE,
         out = torch.empty((n_rows, k_cols), dtype=torch.float32, device=packed.device)
     L = _layout(n_rows, k_cols, group_size, scale_dtype)
     check("cascadia_int4_debug_dequant", lib().cascadia_int4_debug_dequant(
-        C.byref(L), packed.data_ptr(), scale_bits.data_ptr(), out.data_ptr(), _stream()))
+        L, packed.data_ptr(), scale_bits.data_ptr(), out.data_ptr(), _stream()))
     return out
 
 
