@@ -40,68 +40,84 @@ void tiled_sizes(int N, int K, int G, size_t *packed_bytes, size_t *scale_bytes)
   *scale_bytes = tiles * (size_t)(K / G) * 16 * 2;
 }
 
+// Nibbles n0 .. n7 of d -> bytes n0 | n4, n1 | n5, n2 | n6, n3 | n7.
 CAI4_DEV uint32_t swizzle_dword(uint32_t d) {
-  uint32_t r = 0;
-#pragma unroll
-  for (int e = 0; e < 4; ++e) r |= ((d >> (4 * e)) & 0xFu) << (8 * e);
-#pragma unroll
-  for (int e = 4; e < 8; ++e) r |= ((d >> (4 * e)) & 0xFu) << (8 * (e - 4) + 4);
-  return r;
+  uint32_t lo = d & 0xFFFFu, hi = d >> 16;
+  lo = (lo | (lo << 8)) & 0x00FF00FFu;
+  hi = (hi | (hi << 8)) & 0x00FF00FFu;
+  lo = (lo | (lo << 4)) & 0x0F0F0F0Fu;
+  hi = (hi | (hi << 4)) & 0x0F0F0F0Fu;
+  return lo | (hi << 4);
 }
 
-__global__ void tile_packed_kernel(const uint8_t *__restrict__ packed, int N, int K, int xposed,
-                                   uint8_t *__restrict__ out) {
-  const size_t kbt = (size_t)(K + 127) / 128;
-  const size_t total = (size_t)((N + 15) / 16) * kbt * 64;  // 16-byte chunks
-  const size_t row_bytes = (size_t)K / 2;
-  const size_t stride = (size_t)gridDim.x * blockDim.x;
-  for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < total; i += stride) {
-    const size_t l = i & 63, blk = i >> 6;
-    const size_t T = blk / kbt, kb = blk % kbt;
-    const size_t r = 16 * T + (l & 15);
-    uint32_t w[4] = {0u, 0u, 0u, 0u};
-    if (r < (size_t)N) {
-      const uint8_t *row = packed + r * row_bytes;
+// Bound: HBM, each byte read and written once.  A wave takes kTileBlocks
+// k-blocks of one tile: lane (r, c) reads row r's 16-byte parts c of each, all
+// in flight (a row's kTileBlocks * 64 bytes are contiguous), and writes the
+// blocks in lane order; where the layout transposes, the lanes' dwords trade
+// places in registers.  Reading each dword of the transposed form from memory
+// (four 4-byte loads a lane, 16 bytes apart) took 22 us for 7168 x 8192, and the
+// scales' launch 7; this one launch 15.  The blocks past the code blocks move
+// the scales, through LDS: [16 rows][64 groups] read along the rows, written
+// along the tile.
+constexpr int kTileBlocks = 4, kTileGroups = 64;
+
+__global__ __launch_bounds__(256) void tile_kernel(const uint8_t *__restrict__ packed,
+                                                   const uint16_t *__restrict__ scales, int N,
+                                                   int K, int NG, int xposed,
+                                                   unsigned code_blocks,
+                                                   uint8_t *__restrict__ out,
+                                                   uint16_t *__restrict__ out_s) {
+  if (blockIdx.x < code_blocks) {
+    const size_t kbt = (size_t)(K + 127) / 128, per = (kbt + kTileBlocks - 1) / kTileBlocks;
+    const size_t wave = (size_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+    const size_t T = wave / per, kb0 = (wave - T * per) * kTileBlocks;
+    if (T >= (size_t)(N + 15) / 16) return;
+    const int lane = threadIdx.x & 63;
+    const size_t r = 16 * T + (lane & 15), row_bytes = (size_t)K / 2;
+    u32x4_t w[kTileBlocks];
 #pragma unroll
-      for (int s = 0; s < 4; ++s) {
-        // untransposed: dword s of the lane's own 16 bytes; transposed: dword
-        // (lane row) of lane row s's 16 bytes.  row_bytes is a multiple of 16:
-        // a 16-byte part is wholly inside the row or past it.
-        const size_t part = kb * 64 + 16 * (xposed ? (size_t)s : (l >> 4));
-        const size_t dw = xposed ? (l >> 4) : (size_t)s;
-        if (part < row_bytes)
-          w[s] = swizzle_dword(*reinterpret_cast<const uint32_t *>(row + part + 4 * dw));
-      }
+    for (int i = 0; i < kTileBlocks; ++i) {
+      // row_bytes is a multiple of 16: a part is wholly inside the row or past it
+      const size_t part = (kb0 + i) * 64 + 16 * (lane >> 4);
+      w[i] = u32x4_t{0u, 0u, 0u, 0u};
+      if (r < (size_t)N && part < row_bytes)
+        w[i] = *reinterpret_cast<const u32x4_t *>(packed + r * row_bytes + part);
     }
-    reinterpret_cast<u32x4_t *>(out)[i] = u32x4_t{w[0], w[1], w[2], w[3]};
+#pragma unroll
+    for (int i = 0; i < kTileBlocks; ++i) {
+      if (kb0 + i >= kbt) break;  // uniform in the wave
+      const u32x4_t v = xposed ? xpose_rows(w[i]) : w[i];
+      reinterpret_cast<u32x4_t *>(out)[(T * kbt + kb0 + i) * 64 + lane] =
+          u32x4_t{swizzle_dword(v.x), swizzle_dword(v.y), swizzle_dword(v.z), swizzle_dword(v.w)};
+    }
+    return;
   }
-}
-
-__global__ void tile_scales_kernel(const uint16_t *__restrict__ scales, int N, int NG,
-                                   uint16_t *__restrict__ out) {
-  const size_t total = (size_t)((N + 15) / 16) * NG * 16;
-  const size_t stride = (size_t)gridDim.x * blockDim.x;
-  for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < total; i += stride) {
-    const size_t rr = i & 15, tg = i >> 4;
-    const size_t T = tg / NG, g = tg % NG;
-    const size_t r = 16 * T + rr;
-    out[i] = r < (size_t)N ? scales[r * NG + g] : (uint16_t)0;
+  __shared__ uint16_t t[kTileGroups][18];
+  const size_t blk = blockIdx.x - code_blocks, nb = (size_t)(NG + kTileGroups - 1) / kTileGroups;
+  const size_t T = blk / nb;
+  const int g0 = (int)(blk - T * nb) * kTileGroups;
+  const int ng = NG - g0 < kTileGroups ? NG - g0 : kTileGroups;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int g = threadIdx.x & 63, r = (threadIdx.x >> 6) + 4 * i;
+    if (g < ng)
+      t[g][r] = 16 * T + r < (size_t)N ? scales[(16 * T + r) * NG + g0 + g] : (uint16_t)0;
   }
+  __syncthreads();
+  for (int i = threadIdx.x; i < ng * 16; i += 256)
+    out_s[(T * NG + g0) * 16 + i] = t[i >> 4][i & 15];
 }
 
 hipError_t tile_weights(const uint8_t *packed, const uint8_t *scale_bits, int N, int K, int G,
                         uint8_t *packed_tiled, uint8_t *scale_tiled, hipStream_t st) {
-  const size_t chunks = (size_t)((N + 15) / 16) * ((K + 127) / 128) * 64;
-  size_t grid = (chunks + 255) / 256;
-  if (grid > 16384) grid = 16384;
-  hipLaunchKernelGGL(tile_packed_kernel, dim3(grid), dim3(256), 0, st, packed, N, K,
-                     tiled_xposed(G) ? 1 : 0, packed_tiled);
-  if (hipError_t e = hipGetLastError()) return e;
-  const size_t ns = (size_t)((N + 15) / 16) * (K / G) * 16;
-  grid = (ns + 255) / 256;
-  if (grid > 16384) grid = 16384;
-  hipLaunchKernelGGL(tile_scales_kernel, dim3(grid), dim3(256), 0, st,
-                     reinterpret_cast<const uint16_t *>(scale_bits), N, K / G,
+  const size_t tiles = (size_t)(N + 15) / 16, kbt = (size_t)(K + 127) / 128;
+  const int NG = K / G;
+  const size_t code = (tiles * ((kbt + kTileBlocks - 1) / kTileBlocks) + 3) / 4;
+  const size_t sc = tiles * (size_t)((NG + kTileGroups - 1) / kTileGroups);
+  if (code + sc > 0x7FFFFFFFu) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(tile_kernel, dim3((unsigned)(code + sc)), dim3(256), 0, st, packed,
+                     reinterpret_cast<const uint16_t *>(scale_bits), N, K, NG,
+                     tiled_xposed(G) ? 1 : 0, (unsigned)code, packed_tiled,
                      reinterpret_cast<uint16_t *>(scale_tiled));
   return hipGetLastError();
 }

@@ -66,6 +66,26 @@ def test_quantize_bit_identical_to_oracle(cl, orc, n, k, g):
         assert np.array_equal(q, want_q), "rounding ties"
 
 
+@pytest.mark.parametrize("n,k,g", [
+    # chunks that are no multiple of a workgroup's, the widest group a wave
+    # shares and the first it does not, one group in all
+    (1, 32, 32), (5, 224, 32), (3, 8192, 64), (37, 1536, 128), (3, 1024, 512), (2, 1024, 1024),
+    (9, 160, 160)])
+def test_quantize_edges(cl, orc, n, k, g):
+    """Shapes at the edges of the lane-per-chunk quantiser, and weights next to
+    its rounding points: 0.5 and its float neighbours, infinities, NaN."""
+    wb = weights_bf16(orc, n, k, g, n + k + g).reshape(n, k)
+    wb[0, 1:9] = np.array([0x3EFF, 0x3F00, 0x3F01, 0xBEFF, 0xBF00, 0x7FC0, 0x8000, 0x0001], np.uint16)
+    wb[0, 0] = 0x40E0  # 7.0: scale 1, so the codes are the rounded weights
+    if n > 4:
+        wb[4, 0], wb[4, 3] = 0x7F80, 0xFF80
+    wb = wb.reshape(-1)
+    packed, scales = cl.quantize_int4_group(dev(wb.view(np.int16)), n, k, g)
+    want_p, want_s = orc.quantize_int4_group(wb, n, k, g)
+    assert np.array_equal(host(scales), want_s.view(np.uint8).reshape(-1))
+    assert np.array_equal(host(packed), want_p.reshape(-1))
+
+
 def test_quantize_then_gemv(cl, orc):
     """GPU-quantised weights, tiled, through the one-token GEMV: the oracle
     GEMV on the oracle's bytes."""
