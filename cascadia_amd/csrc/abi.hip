@@ -15,6 +15,7 @@
 #include "moe.hpp"
 #include "ov.hpp"
 #include "gemv.hpp"
+#include "few.hpp"
 #include "grouped.hpp"
 #include "quant.hpp"
 #include "skinny.hpp"
@@ -281,16 +282,41 @@ bool ffn_tile_shape(uint32_t hidden, uint32_t inter, uint32_t group) {
          cai4::gg_supported((int)inter, (int)group, 1);
 }
 
+// Whether a decode batch's FFN runs on few.hip: bf16 rows, 9 .. 32 of them, and
+// enough weights that its column blocks (64 / 128 wide) fill the CUs in few
+// slices of K.  Below 9 rows the skinny kernel stages little and keeps two
+// workgroups per CU.  Measured (us per FFN, few / skinny or tiles, in a graph):
+//   4096 x 14336 G128: 8 rows 32.3 / 30.6, 12: 34.5 / 37.2, 16: 33.7 / 36.0,
+//                      24: 42 / 62, 32: 42.7 / 62.5
+//   4096 x 14336 G32:  8 rows 33.7 / 33.8, 16: 35.0 / 47.4, 32: 48.2 / 75.5
+//   5120 x 8192 G64:   8 rows 30.0 / 29.6, 16: 31.2 / 35.4, 32: 39.1 / 49.3
+//   7168 x 2048 G32:   16 rows 22.9 / 21.8, 32: 28.6 / 28.2 (21 MiB)
+//   4096 x 4096 G128:  16 rows 22.6 / 23.9, 32: 27.8 / 26.7 (24 MiB)
+// CASCADIA_INT4_FEW_MIN_TOKENS overrides, and is then the only rule.
+bool ffn_few_pays(uint32_t hidden, uint32_t inter, uint32_t group, uint32_t n_tokens,
+                  bool x_f32) {
+  if (x_f32 || !cai4::few_supported((int)n_tokens, (int)inter, (int)hidden, (int)group, 1) ||
+      !cai4::few_supported((int)n_tokens, (int)hidden, (int)inter, (int)group, 1))
+    return false;
+  const int env = cai4::tuning_env("CASCADIA_INT4_FEW_MIN_TOKENS", 0);
+  if (env > 0) return (int)n_tokens >= env;
+  return tiles_pay(n_tokens, cai4::kFewMaxRows, (size_t)hidden * inter * 3 / 2, 9,
+                   (size_t)32 << 20);
+}
+
 // Workspace of an expert FFN: the SwiGLU intermediate as two bf16 planes,
-// then the split-K partials of whichever of its two GEMMs needs more; or, for
-// many tokens, the planes, their seeds and the MFMA-tile GEMMs' own (tile); or
+// then the split-K partials of whichever of its two GEMMs needs more (the same
+// for few.hip's, in few); or, for many tokens, the planes, their seeds and the MFMA-tile GEMMs' own (tile); or
 // the same without splitting K and with the down's seeds in the GEMMs' share
 // (lean), where no more memory can be had.
 struct FfnWorkspace {
-  size_t planes, partials, tile, lean;
+  size_t planes, partials, few, tile, lean;
   size_t skinny() const { return planes + partials; }
   size_t least() const { return skinny() > lean ? skinny() : lean; }
-  size_t total() const { return least() > tile ? least() : tile; }
+  size_t total() const {
+    const size_t t = few > tile ? few : tile;
+    return least() > t ? least() : t;
+  }
 };
 size_t ffn_plane_bytes(uint32_t inter, uint32_t n_tokens) {
   return ((size_t)n_tokens * inter * 2 + 255) & ~(size_t)255;
@@ -344,9 +370,15 @@ FfnWorkspace ffn_workspace(int dev, uint32_t hidden, uint32_t inter, uint32_t gr
   const cai4::SkinnyPlan dn = cai4::skinny_plan((int)hidden, (int)inter, (int)group,
                                                 (int)n_tokens, cai4::A_HILO, cai4::EPI_F32, d);
   const size_t planes = ((size_t)n_tokens * inter * 2 * sizeof(uint16_t) + 255) & ~(size_t)255;
+  size_t few = 0;
+  if (ffn_few_pays(hidden, inter, group, n_tokens, x_f32)) {
+    const size_t a = cai4::few_workspace((int)n_tokens, (int)inter, (int)hidden, true, d.num_cus);
+    const size_t b = cai4::few_workspace((int)n_tokens, (int)hidden, (int)inter, false, d.num_cus);
+    few = 2 * ffn_plane_bytes(inter, n_tokens) + (a > b ? a : b);
+  }
   return FfnWorkspace{planes,
                       gu.partial_bytes > dn.partial_bytes ? gu.partial_bytes : dn.partial_bytes,
-                      tile, lean};
+                      few, tile, lean};
 }
 
 // The expert FFN on the MFMA-tile GEMMs: gate/up with the SwiGLU epilogue
@@ -403,6 +435,49 @@ int ffn_tiles(uint32_t hidden, uint32_t inter, uint32_t group, uint32_t sdt,
   dn.ldy = (int)hidden;
   dn.epi = out_bf16 ? cai4::GG_BF16 : cai4::GG_F32;
   return hip_status(cai4::gg_dense(dn, cai4::GG_A_PLANES, b, num_cus, st, slices));
+}
+
+// The expert FFN of a few bf16 rows: gate/up with the SwiGLU epilogue into
+// hi / lo planes, then down over them (few.hip).
+int ffn_few(uint32_t hidden, uint32_t inter, uint32_t group, uint32_t sdt,
+            const cascadia_int4_expert *e, const void *x, uint32_t n_tokens, void *out,
+            bool out_bf16, void *ws, int num_cus, hipStream_t st) {
+  const size_t plane = ffn_plane_bytes(inter, n_tokens);
+  uint8_t *b = static_cast<uint8_t *>(ws);
+  uint16_t *hi = reinterpret_cast<uint16_t *>(b);
+  uint16_t *lo = reinterpret_cast<uint16_t *>(b + plane);
+  b += 2 * plane;
+  cai4::GgArgs g{};
+  g.w0 = e->gate_packed;
+  g.s0 = e->gate_scale;
+  g.w1 = e->up_packed;
+  g.s1 = e->up_scale;
+  g.x = static_cast<const uint16_t *>(x);
+  g.y = hi;
+  g.y2 = lo;
+  g.M = (int)n_tokens;
+  g.N = (int)inter;
+  g.K = (int)hidden;
+  g.G = (int)group;
+  g.sdt = (int)sdt;
+  g.ldy = (int)inter;
+  g.epi = cai4::GG_SWIGLU_HILO;
+  if (hipError_t err = cai4::few_gemm(g, b, num_cus, st)) return hip_status(err);
+  cai4::GgArgs dn{};
+  dn.w0 = e->down_packed;
+  dn.s0 = e->down_scale;
+  dn.x = hi;
+  dn.x2 = lo;
+  dn.hilo = 1;
+  dn.y = out;
+  dn.M = (int)n_tokens;
+  dn.N = (int)hidden;
+  dn.K = (int)inter;
+  dn.G = (int)group;
+  dn.sdt = (int)sdt;
+  dn.ldy = (int)hidden;
+  dn.epi = out_bf16 ? cai4::GG_BF16 : cai4::GG_F32;
+  return hip_status(cai4::few_gemm(dn, b, num_cus, st));
 }
 
 void expert_sections(uint32_t hidden, uint32_t inter, uint32_t group, size_t off[6]) {
@@ -462,6 +537,9 @@ int ffn_common(uint32_t hidden, uint32_t inter, uint32_t group, uint32_t sdt,
   } else if (!aligned(ws, 16)) {
     return CASCADIA_INT4_ERR_ARG;
   }
+  if (!lean && need.few && e->tiling == CASCADIA_INT4_TILING_MFMA)
+    return ffn_few(hidden, inter, group, sdt, e, x, n_tokens, out, out_bf16, ws,
+                   device_props(dev).num_cus, st);
   if ((lean ? need.lean : need.tile) && e->tiling == CASCADIA_INT4_TILING_MFMA)
     return ffn_tiles(hidden, inter, group, sdt, e, x, x_f32, n_tokens, out, out_bf16, ws, lean,
                      device_props(dev).num_cus, st);

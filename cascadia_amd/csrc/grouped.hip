@@ -9,8 +9,9 @@
 //
 // Arithmetic: weights enter v_mfma_f32_32x32x16_bf16 as the exact bf16 value
 // 128 + nibble (or 16 + nibble: gg_small_offset); each group's partial starts
-// from the seed -136 (-24) * sum(x) over the group's columns (computed once per row and group by gg_prep) and is
-// scaled in f32 when the group ends, acc += s * p.  A k-block of 128 columns is
+// from the seed -136 (-24) * sum(x) over the group's columns (computed once per
+// row and group by gg_prep) and is scaled in f32 when the group ends, acc +=
+// s * p.  A k-block of 128 columns is
 // four sub-steps of 32: a sub-step is dword s of every weight fragment.  Groups
 // of 32 or 64 columns end with a sub-step: the tiled layout stores those
 // matrices' fragments with their four dwords transposed across the lane rows
@@ -56,53 +57,13 @@
 // tokens over 384 experts, G 32: 2.50 -> 2.07 ms a layer.
 #include "grouped.hpp"
 #include "int4_common.hpp"
+#include "lds_dma.hpp"
 
 namespace cai4 {
 
 namespace {
 
-typedef __amdgpu_buffer_rsrc_t rsrc_t;
-typedef __attribute__((address_space(3))) void lds_void;
 typedef float f32x16_t __attribute__((ext_vector_type(16)));
-
-CAI4_DEV rsrc_t rsrc(const void *base, size_t bytes) {
-  const int n = bytes > 0x7FFFFFFFu ? 0x7FFFFFFF : (int)bytes;
-  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(base), (short)0, n, 0x00020000);
-}
-
-// The same with the (wave-uniform) base and size forced into scalar registers.
-CAI4_DEV rsrc_t rsrc_scalar(const void *base, size_t bytes) {
-  const uint64_t b = (uint64_t)base;
-  // (readfirstlane returns int: without the cast its sign would fill the high half)
-  const uint64_t u = (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)b) |
-                     (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)(b >> 32)) << 32;
-  const int n = __builtin_amdgcn_readfirstlane(bytes > 0x7FFFFFFFu ? 0x7FFFFFFF : (int)bytes);
-  return __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<void *>(u), (short)0, n, 0x00020000);
-}
-
-// Wait until at most n of this wave's vector-memory loads are outstanding and
-// its LDS reads have returned, then barrier.  Inline asm with a memory
-// clobber: neither LDS reads nor the LDS-destination loads move across it.
-template <int n>
-CAI4_DEV void gg_wait_barrier() {
-  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(n) : "memory");
-}
-
-// One global -> LDS buffer load (16 or 4 bytes per lane, lane i at M0 +
-// bytes * i) from byte voff + soff.  Inline asm: the compiler cannot tell the
-// stage buffers apart and would make LDS reads of any stage wait for the
-// newest prefetch.  A lane's row limit is in voff (soff only steps along K).
-template <int bytes>
-CAI4_DEV void gg_dma(rsrc_t r, uint32_t lds, uint32_t voff, uint32_t soff) {
-  if constexpr (bytes == 16)
-    asm volatile("buffer_load_dwordx4 %1, %2, %3 offen lds" ::"{m0}"(lds), "v"(voff), "s"(r),
-                 "s"(soff)
-                 : "memory");
-  else
-    asm volatile("buffer_load_dword %1, %2, %3 offen lds" ::"{m0}"(lds), "v"(voff), "s"(r),
-                 "s"(soff)
-                 : "memory");
-}
 
 CAI4_DEV f32x16_t mfma32_bf16(u32x4_t a, u32x4_t b, f32x16_t c) {
   return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, a),
@@ -136,15 +97,6 @@ struct Gg {
   static_assert(3 * BYTES <= 160 * 1024, "LDS");
 };
 
-// The hi plane of a split f32 value: x rounded to bf16 (to nearest even: the lo
-// plane, bf16 of the exact remainder, then holds x to half the error that a
-// truncated hi leaves it), truncated where rounding would reach infinity.
-CAI4_DEV uint32_t split_hi(float x) {
-  const uint32_t b = fbits(x), r = (b + 0x7FFFu + ((b >> 16) & 1u)) >> 16;
-  return (r & 0x7F80u) == 0x7F80u ? b >> 16 : r;
-}
-CAI4_DEV uint32_t split_lo(float x, uint32_t hi) { return f32_to_bf16_rne(x - bitsf(hi << 16)); }
-
 // Keeps these values' computation in its slot: the instruction selector orders
 // arithmetic freely between scheduling barriers unless something there uses it.
 CAI4_DEV void gg_pin(float &a, float &b, float &c, float &d, float &e, float &f, float &g,
@@ -153,17 +105,6 @@ CAI4_DEV void gg_pin(float &a, float &b, float &c, float &d, float &e, float &f,
   asm volatile("" : "+v"(a), "+v"(b), "+v"(c), "+v"(d), "+v"(e), "+v"(f), "+v"(g), "+v"(h));
 #endif
 }
-
-// A read of LDS at byte address at + off.  The constant off is a pointer step,
-// not integer arithmetic, so that it becomes the instruction's offset.
-template <class T>
-CAI4_DEV T lds_at(uint32_t at, int off) {
-  typedef const __attribute__((address_space(3))) uint8_t *bytes_t;
-  return *reinterpret_cast<const __attribute__((address_space(3))) T *>(
-      reinterpret_cast<bytes_t>(at) + off);
-}
-
-constexpr uint32_t kGgOOB = 0x80000000u;  // an offset past every range: no data moves
 
 // The weights' encoding: bf16 128 + n (0x43 over the nibble), offset 136 with
 // the zero point; or 16 + n (0x41 over 0x80 | n << 3), offset 24, one
@@ -277,9 +218,9 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gg_kernel(GgArgs a) {
     const int blk = wave * P::AL + l, rb = blk % (P::BM / 4);
     const int row = 4 * rb + (lane >> 4), q = l15 ^ (row & 15);
     if (ind)
-      va[l] = row < mrows ? (uint32_t)(((size_t)a.row_map[row0 + row] * a.K + 8 * q) * 2) : kGgOOB;
+      va[l] = row < mrows ? (uint32_t)(((size_t)a.row_map[row0 + row] * a.K + 8 * q) * 2) : kDmaOOB;
     else
-      va[l] = row < mrows ? (uint32_t)(row * a.K + 8 * q) * 2 : kGgOOB;
+      va[l] = row < mrows ? (uint32_t)(row * a.K + 8 * q) * 2 : kDmaOOB;
   }
 #pragma unroll
   for (int l = 0; l < P::BL; ++l) {
@@ -304,7 +245,7 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gg_kernel(GgArgs a) {
       mb = ind ? a.seeds : a.seeds + row0;
       ms = ((size_t)KB * GPK * a.rows_pad - (ind ? 0 : row0)) * 4;
       vm[k] = r < mrows ? (uint32_t)(((size_t)g * a.rows_pad + (ind ? a.row_map[row0 + r] : r)) * 4)
-                        : kGgOOB;
+                        : kDmaOOB;
     }
     mr[k] = rsrc_scalar(mb, ms);
   }
@@ -313,15 +254,15 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gg_kernel(GgArgs a) {
     const uint32_t L = lds0 + buf * P::BYTES;
     if (l < P::AL) {
       const int blk = wave * P::AL + l;
-      gg_dma<16>(PL == 2 && blk >= P::BM / 4 ? xr1 : xr0, L + P::A + blk * 1024, va[l < P::AL ? l : 0],
+      lds_dma<16>(PL == 2 && blk >= P::BM / 4 ? xr1 : xr0, L + P::A + blk * 1024, va[l < P::AL ? l : 0],
                  (uint32_t)kb * 256);
     } else if (l < P::AL + P::BL) {
       const int t = l - P::AL;
-      gg_dma<16>(wr, L + P::B + (wave * P::BL + t) * 1024, vb[t < P::BL ? t : 0],
+      lds_dma<16>(wr, L + P::B + (wave * P::BL + t) * 1024, vb[t < P::BL ? t : 0],
                  (uint32_t)kb * 1024);
     } else {
       const int k = l - P::AL - P::BL < P::MPW ? l - P::AL - P::BL : 0;
-      gg_dma<4>(mr[k], L + P::S + (wave + k * P::W) * 256, vm[k],
+      lds_dma<4>(mr[k], L + P::S + (wave + k * P::W) * 256, vm[k],
                 mx[k] ? (uint32_t)(kb * GPK * a.rows_pad) * 4 : (uint32_t)g * 32);
     }
   };
@@ -392,11 +333,11 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gg_kernel(GgArgs a) {
   };
 
   if (kb0 + 2 < KE)
-    gg_wait_barrier<2 * P::LOADS>();
+    dma_wait_barrier<2 * P::LOADS>();
   else if (kb0 + 1 < KE)
-    gg_wait_barrier<P::LOADS>();
+    dma_wait_barrier<P::LOADS>();
   else
-    gg_wait_barrier<0>();
+    dma_wait_barrier<0>();
   int cur = 0;
 
   if (wm * P::RM < mrows) {
@@ -435,9 +376,9 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gg_kernel(GgArgs a) {
           const int i = MT == 2 ? t : 0;
           if (s == 3 && n == 0) {
             if (DMA)
-              gg_wait_barrier<P::LOADS>();
+              dma_wait_barrier<P::LOADS>();
             else if (kb + 1 < KE)
-              gg_wait_barrier<0>();
+              dma_wait_barrier<0>();
           }
           // LDS reads: the next sub-step's activations, the group's scales, the
           // next group's seeds, the next k-block's weights once their last
@@ -544,7 +485,7 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gg_kernel(GgArgs a) {
 #pragma unroll 1
     for (int kb = kb0; kb + 1 < KE; ++kb) {
       if (kb + 3 < KE) {
-        gg_wait_barrier<P::LOADS>();
+        dma_wait_barrier<P::LOADS>();
 #pragma unroll
         for (int l = 0; l < P::LOADS; ++l) issue1(l, cur, kb + 3, g3);
         if (GPK > 1) {
@@ -554,7 +495,7 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gg_kernel(GgArgs a) {
           ++g3;
         }
       } else {
-        gg_wait_barrier<0>();
+        dma_wait_barrier<0>();
       }
       cur = cur == 2 ? 0 : cur + 1;
     }
@@ -657,29 +598,30 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gg_kernel(GgArgs a) {
 // slice order; four slices' loads are issued before their adds (clamped: all in
 // range) and pinned there.
 CAI4_DEV f32x4_t sum_slices(const float *part, size_t stride, size_t i, int nsl) {
-  f32x4_t s = *reinterpret_cast<const f32x4_t *>(part + i);
-  for (int z0 = 1; z0 < nsl; z0 += 4) {
-    f32x4_t v[4];
+  f32x4_t s = {0.f, 0.f, 0.f, 0.f};
+  for (int z0 = 0; z0 < nsl; z0 += 8) {
+    f32x4_t v[8];
 #pragma unroll
-    for (int z = 0; z < 4; ++z)
+    for (int z = 0; z < 8; ++z)
       v[z] = *reinterpret_cast<const f32x4_t *>(part + (size_t)min(z0 + z, nsl - 1) * stride + i);
 #pragma unroll
-    for (int z = 0; z < 4; ++z) asm volatile("" : "+v"(v[z]));
+    for (int z = 0; z < 8; ++z) asm volatile("" : "+v"(v[z]));
 #pragma unroll
-    for (int z = 0; z < 4; ++z)
-      if (z0 + z < nsl) s += v[z];
+    for (int z = 0; z < 8; ++z)
+      if (z0 + z < nsl) s = z0 + z ? s + v[z] : v[z];
   }
   return s;
 }
 
 // y = sum over the K slices' partials, in slice order; bf16 (RNE) or f32.
-__global__ __launch_bounds__(256) void gg_reduce_kernel(const float *part, void *y, int M, int N,
+__global__ __launch_bounds__(64) void gg_reduce_kernel(const float *part, void *y, int M, int N,
                                                         int ldy, int nsl, int out_f32) {
   const size_t i = ((size_t)blockIdx.x * blockDim.x + threadIdx.x) * 4;
   const size_t n = (size_t)M * N;
   if (i >= n) return;  // n is a multiple of 4
   const f32x4_t s = sum_slices(part, n, i, nsl);
-  const size_t r = i / N, c = i - r * N;  // N % 4 == 0: the four stay in one row
+  // N % 4 == 0: the four stay in one row
+  const size_t r = n >> 32 ? i / N : (uint32_t)i / (uint32_t)N, c = i - r * N;
   const size_t o = r * ldy + c;
   if (out_f32) {
     float *yf = reinterpret_cast<float *>(y) + o;
@@ -922,6 +864,33 @@ namespace {
 size_t al256(size_t v) { return (v + 255) & ~(size_t)255; }
 }  // namespace
 
+hipError_t gg_reduce_slices(const GgArgs &a, int nsl, hipStream_t st) {
+  const bool sw = a.epi == GG_SWIGLU_HILO;
+  if (sw) {
+    const size_t n = (size_t)a.M * (a.N / 8);
+    const dim3 grid((unsigned)((n + 255) / 256)), block(256);
+    uint16_t *hi = static_cast<uint16_t *>(a.y), *lo = static_cast<uint16_t *>(a.y2);
+    switch (gg_group_width(a.G)) {
+      case 32:
+        hipLaunchKernelGGL(gg_swiglu_reduce_kernel<4>, grid, block, 0, st, a.part, hi, lo,
+                           a.seeds_out, a.M, a.N, a.ldy, nsl, a.seeds_rp);
+        break;
+      case 64:
+        hipLaunchKernelGGL(gg_swiglu_reduce_kernel<8>, grid, block, 0, st, a.part, hi, lo,
+                           a.seeds_out, a.M, a.N, a.ldy, nsl, a.seeds_rp);
+        break;
+      default:
+        hipLaunchKernelGGL(gg_swiglu_reduce_kernel<16>, grid, block, 0, st, a.part, hi, lo,
+                           a.seeds_out, a.M, a.N, a.ldy, nsl, a.seeds_rp);
+    }
+    return hipGetLastError();
+  }
+  const size_t n = (size_t)a.M * a.N;
+  hipLaunchKernelGGL(gg_reduce_kernel, dim3((unsigned)((n / 4 + 63) / 64)), dim3(64), 0, st,
+                     a.part, a.y, a.M, a.N, a.ldy, nsl, a.epi == GG_F32 ? 1 : 0);
+  return hipGetLastError();
+}
+
 size_t gg_dense_workspace(int M, int N, int K, int G, int amode, int epi, int num_cus,
                           bool have_seeds, int max_slices) {
   const bool sw = epi == GG_SWIGLU_HILO;
@@ -975,29 +944,7 @@ hipError_t gg_dense(GgArgs a, int amode, void *ws, int num_cus, hipStream_t st, 
   else
     e = gg_launch_g<2, 2, 4, 1, false>(a, 0, p.nsl, st);
   if (e != hipSuccess || p.nsl == 1) return e;
-  if (sw) {
-    const size_t n = (size_t)a.M * (a.N / 8);
-    const dim3 grid((unsigned)((n + 255) / 256)), block(256);
-    uint16_t *hi = static_cast<uint16_t *>(a.y), *lo = static_cast<uint16_t *>(a.y2);
-    switch (gg_group_width(a.G)) {
-      case 32:
-        hipLaunchKernelGGL(gg_swiglu_reduce_kernel<4>, grid, block, 0, st, a.part, hi, lo,
-                           a.seeds_out, a.M, a.N, a.ldy, p.nsl, a.seeds_rp);
-        break;
-      case 64:
-        hipLaunchKernelGGL(gg_swiglu_reduce_kernel<8>, grid, block, 0, st, a.part, hi, lo,
-                           a.seeds_out, a.M, a.N, a.ldy, p.nsl, a.seeds_rp);
-        break;
-      default:
-        hipLaunchKernelGGL(gg_swiglu_reduce_kernel<16>, grid, block, 0, st, a.part, hi, lo,
-                           a.seeds_out, a.M, a.N, a.ldy, p.nsl, a.seeds_rp);
-    }
-    return hipGetLastError();
-  }
-  const size_t n = (size_t)a.M * a.N;
-  hipLaunchKernelGGL(gg_reduce_kernel, dim3((unsigned)((n / 4 + 255) / 256)), dim3(256), 0, st,
-                     a.part, a.y, a.M, a.N, a.ldy, p.nsl, a.epi == GG_F32 ? 1 : 0);
-  return hipGetLastError();
+  return gg_reduce_slices(a, p.nsl, st);
 }
 
 hipError_t gg_grouped(const GgArgs &a0, int max_tiles, hipStream_t st) {

@@ -32,8 +32,8 @@ struct GgArgs {
   float *part;   // dense split-K partials [ksplit][M][N] (f32), or null
   int kper;      // k-blocks per K slice (blockIdx.z)
   // SwiGLU only, or null: the seeds of the hi / lo planes the epilogue writes,
-  // for a GEMM that takes them as A: [N / seeds_gw][rows_pad], -136 * the sum
-  // of hi + lo over each group of seeds_gw output columns (32, 64 or 128)
+  // for a GEMM that takes them as A: [N / seeds_gw][rows_pad], the zero point's
+  // share of hi + lo over each group of seeds_gw output columns (32, 64 or 128)
   float *seeds_out;
   int seeds_gw, seeds_rp;  // group width, row stride of seeds_out
   // grouped, one bf16 plane only, or null: A row r of the table is x row
@@ -81,6 +81,9 @@ size_t gg_dense_workspace(int M, int N, int K, int G, int amode, int epi, int nu
                           bool have_seeds = false, int max_slices = 8);
 hipError_t gg_dense(GgArgs a, int amode, void *ws, int num_cus, hipStream_t st,
                     int max_slices = 8);
+
+// The K slices' partials a.part added in order into a.y (a.y2, a.seeds_out).
+hipError_t gg_reduce_slices(const GgArgs &a, int nsl, hipStream_t st);
 
 // Grouped: tiles = max_tiles entries (count 0: empty) of at most
 // 128 rows; a.seeds over a.rows_pad rows made by gg_prep.

@@ -160,6 +160,15 @@ CAI4_DEV u32x4_t act_split_f32_nat(const f32x4_t &a, const f32x4_t &b, bool lo) 
   return u32x4_t{w[0], w[1], w[2], w[3]};
 }
 
+// The hi plane of a split f32 value: x rounded to bf16 (to nearest even: the lo
+// plane, bf16 of the exact remainder, then holds x to half the error that a
+// truncated hi leaves it), truncated where rounding would reach infinity.
+CAI4_DEV uint32_t split_hi(float x) {
+  const uint32_t b = fbits(x), r = (b + 0x7FFFu + ((b >> 16) & 1u)) >> 16;
+  return (r & 0x7F80u) == 0x7F80u ? b >> 16 : r;
+}
+CAI4_DEV uint32_t split_lo(float x, uint32_t hi) { return f32_to_bf16_rne(x - bitsf(hi << 16)); }
+
 // Scale bits (u16 in the low half) -> f32: fp16 if sdt, else bf16.
 CAI4_DEV float scale_bits_f32(uint32_t bits, int sdt) {
   return sdt ? scale_to_f32<SCALE_F16>(bits & 0xFFFFu) : scale_to_f32<SCALE_BF16>(bits & 0xFFFFu);

@@ -162,6 +162,23 @@ def test_ffn_split_tiles(cl, orc, tuning, M, h, i, g):
     assert_f32_close(host(of), want, f"split f32 M{M} G{g}")
 
 
+@pytest.mark.parametrize("M,h,i,g,sdt", [(2, 384, 256, 32, F16), (16, 2048, 1152, 32, BF16),
+                                         (17, 640, 1024, 64, F16), (9, 4096, 1536, 128, BF16),
+                                         (32, 1536, 4608, 128, F16), (31, 2048, 512, 256, F16)])
+def test_ffn_few_rows(cl, orc, tuning, M, h, i, g, sdt):
+    """The kernel of a decode batch (2 .. 32 rows): one and two M-tiles, K of an
+    odd number of blocks, both GEMMs with and without K slices."""
+    tuning("CASCADIA_INT4_FEW_MIN_TOKENS", "2")
+    flat = expert(orc, h, i, g, sdt, M + g)
+    W = cl.ExpertWeights(dev(flat), h, i, g, sdt).tiled()
+    xb = orc.fill_normal_bf16(M, 52, M * h)
+    x = dev(xb.view(np.int16).reshape(M, h))
+    out = torch.empty(M * h, dtype=torch.int16, device="cuda")
+    cl.expert_forward(x, *W.slices(), out, group_size=g, scale_dtype=sdt, tiling=cl.TILING_MFMA)
+    want = orc.cpu_expert_forward(xb, M, flat, h, i, g, sdt)
+    assert_bf16_close(host(out).view(np.uint16).reshape(M, h), want, f"few M{M} G{g}")
+
+
 @pytest.mark.parametrize("M,g", [(65, 32), (100, 64), (200, 128)])
 def test_ffn_f32_tiles(cl, orc, tuning, M, g):
     """The f32-in / f32-out FFN (the shared expert) over M rows: x split into
