@@ -1059,28 +1059,32 @@ struct MoePlan {
   cai4::MoeWorkspace ws;
   bool tiles;  // the MFMA-tile GEMMs (grouped.hip) over 128-row chunks
   int rows_pad;
+  size_t shared_bytes;  // the shared expert's workspace
 };
 
 // Many tokens per layer: experts receive enough rows that 16-row chunks would
 // stream each hot expert's weights many times over; 128-row MFMA tiles read
 // them about once per 128 rows.
-bool moe_tiles(const cascadia_int4_moe_layer *L, uint32_t T) {
-  return L->tiling == CASCADIA_INT4_TILING_MFMA && T >= (uint32_t)cai4::moe_tile_tokens() &&
+bool moe_tiles(const cascadia_int4_moe_layer *L, uint32_t top_k, uint32_t T, bool lean) {
+  return L->tiling == CASCADIA_INT4_TILING_MFMA &&
+         cai4::moe_tiles_pay((int)T, (int)L->n_experts, (int)top_k, lean) &&
          cai4::gg_supported((int)L->hidden, (int)L->group_size, 1) &&
          cai4::gg_supported((int)L->inter, (int)L->group_size, 1);
 }
 
+// lean: the least workspace the layer can run in, where no more can be had.
 MoePlan moe_plan(int dev, const cascadia_int4_moe_layer *L, uint32_t top_k, uint32_t T,
-                 bool given_ids) {
+                 bool given_ids, bool lean = false) {
   const cai4::SkinnyDevice d = device_props(dev);
   const int H = (int)L->hidden, I = (int)L->inter, G = (int)L->group_size;
   MoePlan m{};
-  m.tiles = moe_tiles(L, T);
+  m.tiles = moe_tiles(L, top_k, T, lean);
   size_t sh = 0, sh_ws = 0;
   if (has_shared(L)) {
     const FfnWorkspace f = ffn_workspace(dev, L->hidden, L->shared_inter, L->group_size, T, true);
     sh = (size_t)T * H * sizeof(float);
-    sh_ws = f.total();
+    sh_ws = lean ? f.least() : f.total();
+    m.shared_bytes = sh_ws;
   }
   if (m.tiles) {
     // hot experts in 128-row MFMA tiles; the others in 16-row skinny chunks
@@ -1128,10 +1132,16 @@ int moe_forward(const cascadia_int4_moe_layer *L, const cascadia_int4_routing *R
     return CASCADIA_INT4_ERR_ARG;
   int dev;
   if (int rc = current_device(&dev)) return rc;
-  const MoePlan m = moe_plan(dev, L, R->top_k, T, R->mode == CASCADIA_INT4_ROUTE_IDS);
+  const bool given = R->mode == CASCADIA_INT4_ROUTE_IDS;
+  MoePlan m = moe_plan(dev, L, R->top_k, T, given);
   void *ws = workspace;
   if (!ws) {
-    if (int rc = lib_workspace(dev, m.ws.total, &ws, st)) return rc;
+    // a library workspace that cannot grow now (a capture, no memory) may still
+    // hold what the layer needs at least
+    if (lib_workspace(dev, m.ws.total, &ws, st)) {
+      m = moe_plan(dev, L, R->top_k, T, given, true);
+      if (int rc = lib_workspace(dev, m.ws.total, &ws, st)) return rc;
+    }
   } else if (!aligned(ws, 256)) {
     return CASCADIA_INT4_ERR_ARG;
   }
@@ -1228,7 +1238,7 @@ int moe_forward(const cascadia_int4_moe_layer *L, const cascadia_int4_routing *R
                         (int)L->shared.tiling, x, nullptr, cai4::A_XF32, 1,
                         hi + (size_t)k * I, lo + (size_t)k * I, cai4::EPI_SWIGLU_HILO, on);
       return ffn_common(L->hidden, L->shared_inter, L->group_size, L->scale_dtype, &L->shared,
-                        x, true, T, sh, false, W + m.ws.shared_ws, on);
+                        x, true, T, sh, false, W + m.ws.shared_ws, on, m.shared_bytes);
     };
     hipStream_t side = nullptr;
     hipEvent_t fork = nullptr, join = nullptr;
@@ -1326,7 +1336,7 @@ int moe_forward(const cascadia_int4_moe_layer *L, const cascadia_int4_routing *R
     if (e == hipSuccess)
       e = cai4::moe_group(ids, wts, R->threshold, (int)T, E, k, m.ws.chunk_rows,
                           m.ws.max_chunks, pos, row_map, chunks, counts, st, m.ws.chunk_rows2,
-                          cai4::moe_tile_rows(), chunks2, m.ws.max_chunks2);
+                          cai4::moe_tile_rows((int)T, E, k), chunks2, m.ws.max_chunks2);
     // the skinny kernels' share: experts with few rows, 16-row chunks
     cai4::SkinnyArgs sk{};
     sk.partials = part;

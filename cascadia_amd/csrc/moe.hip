@@ -50,14 +50,33 @@ int moe_chunk_rows(int T, int per_expert_max, bool gemv_rows) {
   return per_expert_max < c ? per_expert_max : c;
 }
 
-int moe_tile_tokens() {
+// From 512 tokens on, or where the experts' mean is 36 rows and more.  Measured
+// (us per layer: skinny chunks only / tiles; hidden 3,584, inter 1,408, top 8):
+//   60 experts G128   200 tokens even 228 / 245, Zipf 246 / 218; 256: 297 / 264,
+//                     284 / 243; 300: 326 / 266, 317 / 285; 400: 422 / 291, 407 / 285
+//   60 experts G32    256 tokens 364 / 367, 350 / 320; 400: 508 / 355, 490 / 358
+//   16 experts G128   128 tokens 143 / 105, 139 / 152; 192: 198 / 109, 195 / 110
+//   128 experts G128  400 tokens 470 / 528, 424 / 336; 512: 547 / 522, 529 / 374
+// (128-256 tokens over 384 experts, Zipf-skewed, would gain 15 %, but the same
+// sizes with even routing lose 5 % to the second set of launches.)
+bool moe_tiles_pay(int T, int E, int top_k, bool lean) {
   const int n = tuning_env("CASCADIA_INT4_MOE_TILE_TOKENS", 0);
-  return n > 0 ? n : 512;
+  if (n > 0) return T >= n;
+  return T >= 512 || (!lean && T >= 192 && (int64_t)T * top_k >= (int64_t)36 * E);
 }
 
-int moe_tile_rows() {
+// Rows from which an expert is worth a 128-row tile rather than 16-row chunks:
+// 24 where the mean expert has as many (one more expert in tiles costs its
+// bytes once), else 32.  Measured (us per layer at thresholds of 48 / 32 / 24 / 16):
+//   256 experts, 3072 x 1536: 512 tokens even 597 / 595 / 627 / 744, Zipf 386 /
+//     347 / 350 / 390; 1,024 even 1029 / 965 / 936 / 909, Zipf 580 / 585 / 567 / 577
+//   128 experts: 512 even 563 / 520 / 522 / 538, Zipf 400 / 380 / 374 / 406
+//   60 experts: 1,024 Zipf 556 / 531 / 500 / 494; 400 even 317 / 292 / 291 / 292
+//   384 experts, 7168 x 2048: 1,024 Zipf 2058 / 2050 / 2067 / 2052
+int moe_tile_rows(int T, int E, int top_k) {
   const int n = tuning_env("CASCADIA_INT4_MOE_TILE_ROWS", 0);
-  return n > 0 ? n : 48;
+  if (n > 0) return n;
+  return (int64_t)T * top_k >= (int64_t)24 * E ? 24 : 32;
 }
 
 int moe_max_chunks(int T, int E, int top_k, int chunk_rows) {

@@ -41,12 +41,13 @@ MoeWorkspace moe_workspace(int T, int H, int I, int E, int top_k, int chunk_rows
                            size_t xg_bytes = 0, size_t seeds_x_bytes = 0,
                            size_t seeds_i_bytes = 0, int chunk_rows2 = 0);
 
-// Tokens from which a layer runs on the MFMA-tile GEMMs (grouped.hip): experts
+// Whether a layer of T tokens runs on the MFMA-tile GEMMs (grouped.hip): experts
 // with at least moe_tile_rows() rows in 128-row chunks over gathered bf16 rows,
-// the others on the skinny kernels.  CASCADIA_INT4_MOE_TILE_TOKENS and
+// the others on the skinny kernels.  lean: only where it always does, whatever
+// the experts' mean.  CASCADIA_INT4_MOE_TILE_TOKENS (then the only rule) and
 // CASCADIA_INT4_MOE_TILE_ROWS override.
-int moe_tile_tokens();
-int moe_tile_rows();
+bool moe_tiles_pay(int T, int E, int top_k, bool lean);
+int moe_tile_rows(int T, int E, int top_k);
 
 // Rows per grouped chunk for T tokens, no expert receiving more than
 // per_expert_max of them (T when routing picks distinct experts per token).

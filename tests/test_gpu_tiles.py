@@ -221,6 +221,24 @@ def test_moe_tiles(cl, orc, tuning, T, g, mode, shared_inter, thr, hot_rows):
                 host(w_o), thr, f"tiles T={T} G{g} mode={mode}")
 
 
+@pytest.mark.parametrize("T,E,k,g", [(191, 12, 4, 32), (192, 12, 4, 64), (192, 24, 4, 128),
+                                     (216, 24, 4, 32)])
+def test_moe_tile_rule(cl, orc, T, E, k, g):
+    """Both sides of the default rule's edges: 192 tokens, 36 rows per expert."""
+    h, i = 384, 256
+    blob, shared, ex = build(cl, orc, E, h, i, g, F16, 67 + g, 128, True)
+    logits = orc.fill_normal_f32(62, T, T * E).reshape(T, E)
+    x = orc.fill_normal_f32(63, T, T * h).reshape(T, h)
+    out = torch.empty((T, h), dtype=torch.float32, device="cuda")
+    ids_o = torch.empty((T, k), dtype=torch.int32, device="cuda")
+    w_o = torch.empty((T, k), dtype=torch.float32, device="cuda")
+    xd = dev(x)
+    cl.moe_forward(ex, xd, out, top_k=k, logits=dev(logits), mode=1, scale=1.0, residual=xd,
+                   ids_out=ids_o, weights_out=w_o)
+    check_layer(orc, host(out), x, blob, shared, 128, E, h, i, g, F16, host(ids_o), host(w_o),
+                0.0, f"rule T={T} E={E} G{g}")
+
+
 def test_moe_tiles_hot_expert(cl, orc, tuning):
     """Given ids sending every token to one expert (300 rows: three 128-row
     chunks, the last partial) plus scattered ones; two calls bit-identical."""
