@@ -239,11 +239,12 @@ int cascadia_int4_expert_forward_device(uint32_t hidden, uint32_t inter, uint32_
  * serving loops, harnesses that forbid hipMalloc).  The SwiGLU intermediate
  * and split-K partials live in a file-scope device array of
  * CASCADIA_INT4_NOALLOC_SCRATCH_BYTES per GPU, held until the process ends;
- * a call whose cascadia_int4_ffn_workspace_bytes(hidden, inter, group_size,
- * n_tokens) exceeds it returns CASCADIA_INT4_ERR_ARG (config 1's Llama-3-8B
- * FFN fits up to 64 tokens).  Every call on one GPU shares that array, so
+ * a call that would need more in any form returns CASCADIA_INT4_ERR_ARG
+ * (config 1's Llama-3-8B FFN fits up to 64 tokens), and one whose
+ * cascadia_int4_ffn_workspace_bytes exceeds it but whose least form fits runs
+ * in that form (results within rounding order of the _device entry point's).  Every call on one GPU shares that array, so
  * calls that overlap on one GPU (different streams, or threads) race;
- * serialise them.  Same kernels and results as the _device entry point. */
+ * serialise them.  Otherwise the same kernels and results as _device. */
 #define CASCADIA_INT4_NOALLOC_SCRATCH_BYTES ((size_t)8 << 20)
 int cascadia_int4_expert_forward_noalloc(uint32_t hidden, uint32_t inter, uint32_t group_size,
                                          uint32_t scale_dtype,
