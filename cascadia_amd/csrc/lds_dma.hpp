@@ -36,15 +36,18 @@ CAI4_DEV void dma_wait_barrier() {
 // bytes * i) from byte voff + soff.  Inline asm: the compiler cannot tell the
 // stage buffers apart and would make LDS reads of any stage wait for the
 // newest prefetch.  A lane's row limit is in voff (soff only steps along K).
+// The load reads M0 one wait state after a scalar write of it at the earliest;
+// the compiler knows that rule for its own instructions and not for asm, and
+// sets M0 right before: the s_nop is that wait state.
 template <int bytes>
 CAI4_DEV void lds_dma(rsrc_t r, uint32_t lds, uint32_t voff, uint32_t soff) {
   if constexpr (bytes == 16)
-    asm volatile("buffer_load_dwordx4 %1, %2, %3 offen lds" ::"{m0}"(lds), "v"(voff), "s"(r),
-                 "s"(soff)
+    asm volatile("s_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"{m0}"(lds), "v"(voff),
+                 "s"(r), "s"(soff)
                  : "memory");
   else
-    asm volatile("buffer_load_dword %1, %2, %3 offen lds" ::"{m0}"(lds), "v"(voff), "s"(r),
-                 "s"(soff)
+    asm volatile("s_nop 0\n\tbuffer_load_dword %1, %2, %3 offen lds" ::"{m0}"(lds), "v"(voff),
+                 "s"(r), "s"(soff)
                  : "memory");
 }
 
