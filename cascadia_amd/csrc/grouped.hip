@@ -110,10 +110,18 @@ CAI4_DEV void gg_pin(float &a, float &b, float &c, float &d, float &e, float &f,
 // the zero point; or 16 + n (0x41 over 0x80 | n << 3), offset 24, one
 // instruction more per half fragment.  A group's partial starts at -offset *
 // sum(x) and comes down to sum((n - 8) x), so its f32 roundings grow with the
-// offset and the group: two planes in groups of 128 columns take the small one
-// (FFN 4096 x 14336, f32, 130 rows: 9.9e-6 off 64 bits with the large one, and
-// the skinny kernel, whose planes add up apart, 8.7e-6).
-constexpr bool gg_small_offset(int GPK, int PL) { return GPK == 1 && PL == 2; }
+// offset and the group, and two planes share one partial, where the skinny
+// kernel adds them up apart.  Two planes in groups of 64 columns and more take
+// the small one.  Error against 64 bits with the large / the small offset / in
+// the skinny kernel:
+//   FFN 4096 x 14336 f32, 130 rows  G 64 8.7e-6 / 4.2e-6 / 8.2e-6 (133 / 139 us)
+//                                   G 128 9.9e-6 / 4.4e-6 / 9.1e-6
+//                                   G 32 7.5e-6 / 4.1e-6 / 8.2e-6
+//   GEMM 7168 x 8192 f32, 333 rows  G 64 3.3e-6 / 2.5e-6 / 4.9e-6 (90 / 93 us)
+//                                   G 32 3.0e-6 / 2.5e-6 / 4.9e-6 (100 / 105 us)
+// (rows of mean 1 instead of 0: G 64 1.8e-6 / 5.3e-7 / 9.3e-7, G 32 1.2e-6 /
+// 4.7e-7 / 9.3e-7 of a result ten times as large.)
+constexpr bool gg_small_offset(int GPK, int PL) { return GPK <= 2 && PL == 2; }
 constexpr float gg_seed_factor(int GPK, int PL) { return gg_small_offset(GPK, PL) ? -24.f : -136.f; }
 
 // Bytes of the low (0) or high (1) nibbles of w, encoded.

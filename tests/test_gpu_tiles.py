@@ -114,6 +114,28 @@ def test_gemm_f32_tiles(cl, orc, tuning, n, k, g, sdt, M):
     assert rel_l2(got, want) <= 1e-5
 
 
+@pytest.mark.parametrize("g,mean", [(32, 0.0), (64, 0.0), (64, 1.0), (128, 0.0), (128, 1.0)])
+def test_gemm_f32_tiles_lose_no_precision(cl, tuning, g, mean):
+    """The tile GEMM's f32 result is no further from 64 bits than the skinny
+    kernel's, whose planes add up apart, also where the zero point's share of a
+    group's sum is large (rows of mean 1)."""
+    n, k, M = 1024, 4096, 64
+    packed = cl.fill_bytes(torch.empty(n * k // 2, dtype=torch.uint8, device="cuda"), 11, 1)
+    scales = cl.fill_scales(torch.empty(n * (k // g), dtype=torch.int16, device="cuda"), 11, 2, F16)
+    x = cl.fill_normal(torch.empty((M, k), dtype=torch.float32, device="cuda"), 11, 3) + mean
+    scales = scales.view(torch.uint8)
+    want = x.double() @ cl.debug_dequant(packed, scales, n, k, g, F16).double().T
+    pt, st = cl.tile_weights(packed, scales, n, k, g)
+    err = {}
+    for route, rows in (("tiles", "17"), ("skinny", "100000")):
+        tuning("CASCADIA_INT4_F32_TILE_TOKENS", rows)
+        ys = torch.empty((M, n), dtype=torch.float32, device="cuda")
+        cl.dequant_gemm_int4_multi_auto(pt, st, x, n, k, M, ys, group_size=g, scale_dtype=F16,
+                                        tiling=cl.TILING_MFMA)
+        err[route] = rel_l2(host(ys), want.cpu().numpy())
+    assert err["tiles"] <= err["skinny"], err
+
+
 def test_gemm_f32_capture(cl, orc):
     """A stream capture cannot grow the library's workspace: the f32 GEMM of a
     shape not seen before is recorded all the same (without the tile route if
