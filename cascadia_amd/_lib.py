@@ -78,6 +78,7 @@ SIGNATURES = {
     "cascadia_int4_version": (C.c_char_p, []),
     "cascadia_int4_synchronize": (_i32, [_vp]),
     "cascadia_int4_reload_tuning": (None, []),
+    "cascadia_int4_tuning_generation": (_u32, []),
     "cascadia_int4_dequant_gemv": (_i32, [_LP, _vp, _vp, _vp, _vp, _vp]),
     "cascadia_int4_dequant_gemv_rows_subset": (_i32, [_LP, _vp, _vp, _vp, _vp, _vp, _u32, _vp]),
     "cascadia_int4_build_active_mask": (_i32, [_vp, _u32, C.c_float, _vp, _vp, _vp, _vp, _vp]),

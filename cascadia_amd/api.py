@@ -54,6 +54,26 @@ def _dev(t: torch.Tensor, name: str) -> torch.Tensor:
     return t
 
 
+@functools.lru_cache(maxsize=1024)
+def _need(fn, tuning, device, *dims):
+    """A *_workspace_bytes result, which follows from these values alone (the
+    tuning variables as of generation `tuning`)."""
+    return int(getattr(lib(), fn)(*dims))
+
+
+def _workspace_ptr(workspace, fn, *dims) -> int:
+    """The address of a caller's workspace (0: none), which has to hold what
+    fn(*dims) asks for."""
+    if workspace is None:
+        return 0
+    _dev(workspace, "workspace")
+    need = _need(fn, lib().cascadia_int4_tuning_generation(), torch.cuda.current_device(),
+                 *map(int, dims))
+    if workspace.nbytes < need:
+        raise ValueError(f"workspace has {workspace.nbytes} bytes, the call needs {need}")
+    return workspace.data_ptr()
+
+
 def _expect(cond: bool, msg: str) -> None:
     if not cond:
         raise ValueError(msg)
@@ -501,8 +521,8 @@ def gate_up_silu(x, gate_packed, gate_scale, up_packed, up_scale, inter_out,
 
 
 def ffn_workspace_bytes(hidden, inter, n_tokens, group_size=GROUP_SIZE) -> int:
-    """Workspace bytes of expert_forward / ffn_forward_sparse_f32 for n_tokens
-    rows on the current device."""
+    """Workspace bytes of expert_forward / ffn_forward_sparse_f32 for up to
+    n_tokens rows on the current device."""
     return int(lib().cascadia_int4_ffn_workspace_bytes(hidden, inter, group_size, n_tokens))
 
 
@@ -520,7 +540,7 @@ def expert_forward(x_bf16, gate_packed, gate_scale, up_packed, up_scale, down_pa
             "x and out must both be [n_tokens, hidden]")
     e = _expert_struct(gate_packed, gate_scale, up_packed, up_scale, down_packed, down_scale,
                        tiling)
-    ws = 0 if workspace is None else _dev(workspace, "workspace").data_ptr()
+    ws = _workspace_ptr(workspace, "cascadia_int4_ffn_workspace_bytes", hidden, inter, group_size, T)
     check("cascadia_int4_expert_forward_device", lib().cascadia_int4_expert_forward_device(
         hidden, inter, group_size, scale_dtype, C.byref(e), x_bf16.data_ptr(), T,
         out_bf16.data_ptr(), ws, _stream()))
@@ -553,8 +573,11 @@ def _sparse_call(x, weights, out, threshold, thresholds, group_size, scale_dtype
         thr = thresholds.contiguous().data_ptr()
     e = _expert_struct(gate_packed, gate_scale, up_packed, up_scale, down_packed, down_scale,
                        tiling)
-    ws = 0 if workspace is None else _dev(workspace, "workspace").data_ptr()
     dense = thresholds is None and threshold <= 0.0  # SparsityMode::is_dense (NaN: sparse)
+    # (dense runs the ordinary FFN; an expert whose up is kept in rows the sparse form)
+    ws = _workspace_ptr(workspace, "cascadia_int4_ffn_workspace_bytes"
+                        if dense and tiling != TILING_MFMA_UP_ROWS
+                        else "cascadia_int4_ffn_sparse_workspace_bytes", h, inter, group_size, T)
     counts = None if dense else torch.empty(T, dtype=torch.int32, device=x.device)
     name = "cascadia_int4_ffn_forward_sparse_f32" if x_f32 else "cascadia_int4_expert_forward_sparse"
     check(name, getattr(lib(), name)(h, inter, group_size, scale_dtype, C.byref(e), x.data_ptr(),
@@ -608,7 +631,8 @@ def ffn_forward_sparse_axpy_f32_mode(x_f32, hidden, intermediate, gate_packed, g
         tau = m.tau
     e = _expert_struct(gate_packed, gate_scale, up_packed, up_scale, down_packed_t,
                        down_scale_t_bits, tiling)
-    ws = 0 if workspace is None else _dev(workspace, "workspace").data_ptr()
+    ws = _workspace_ptr(workspace, "cascadia_int4_ffn_sparse_axpy_workspace_bytes", hidden,
+                        intermediate, group_size, T)
     counts = torch.empty(T, dtype=torch.int32, device=x_f32.device)
     check("cascadia_int4_ffn_forward_sparse_axpy_f32",
           lib().cascadia_int4_ffn_forward_sparse_axpy_f32(
@@ -678,7 +702,7 @@ def dequant_axpy_int4_active(packed_t, scale_t_bits, scalars, active, n_intermed
     _expect(scalars.dtype == torch.float32 and scalars.numel() == n_intermediate, "scalars")
     _expect(y.dtype == torch.float32 and y.numel() == n_hidden, "y")
     _expect(active.element_size() == 4, "active must hold 32-bit row ids")
-    ws = 0 if workspace is None else _dev(workspace, "workspace").data_ptr()
+    ws = _workspace_ptr(workspace, "cascadia_int4_axpy_workspace_bytes", n_hidden, active.numel())
     check("cascadia_int4_dequant_axpy_active", lib().cascadia_int4_dequant_axpy_active(
         packed_t.data_ptr(), scale_t_bits.data_ptr(), scalars.data_ptr(), active.data_ptr(),
         active.numel(), n_intermediate, n_hidden, y.data_ptr(), ws, _stream()))
@@ -689,7 +713,7 @@ dequant_axpy_int4_active_auto = dequant_axpy_int4_active  # ffn_axpy.rs:274
 
 
 def ffn_sparse_workspace_bytes(hidden, inter, n_tokens, group_size=GROUP_SIZE) -> int:
-    """Workspace bytes of the sparse entry points for n_tokens rows."""
+    """Workspace bytes of the sparse entry points for up to n_tokens rows."""
     return int(lib().cascadia_int4_ffn_sparse_workspace_bytes(hidden, inter, group_size,
                                                               n_tokens))
 
@@ -831,6 +855,18 @@ def moe_workspace_bytes(experts: MoEExperts, top_k: int, n_tokens: int) -> int:
     return int(lib().cascadia_int4_moe_workspace_bytes(C.byref(experts._struct()), top_k, n_tokens))
 
 
+@functools.lru_cache(maxsize=1024)
+def _moe_need(tuning, device, hidden, inter, group_size, scale_dtype, tiling, n_experts,
+              shared_inter, shared_tiling, top_k, n_tokens):
+    """moe_workspace_bytes of a layer of these dimensions (its pointers, which
+    the size does not depend on, stand-ins that are not read)."""
+    L = MoeLayer(hidden, inter, group_size, scale_dtype, tiling, n_experts, 256, 1 << 40)
+    if shared_inter is not None:
+        L.shared = Expert(256, 256, 256, 256, 256, 256, shared_tiling)
+        L.shared_inter = shared_inter
+    return int(lib().cascadia_int4_moe_workspace_bytes(C.byref(L), top_k, n_tokens))
+
+
 def moe_forward(experts: MoEExperts, x, out, *, top_k: int, logits=None, bias=None,
                 mode: int = ROUTE_SIGMOID_BIAS, scale: float = 1.0, normalize: bool = True,
                 ids=None, weights=None, threshold: float = 0.0, residual=None,
@@ -877,7 +913,15 @@ def moe_forward(experts: MoEExperts, x, out, *, top_k: int, logits=None, bias=No
         _dev(weights_out, "weights_out")
         _expect(weights_out.dtype == torch.float32 and weights_out.numel() == T * top_k, "weights_out: f32")
         wo = weights_out.data_ptr()
-    ws = 0 if workspace is None else _dev(workspace, "workspace").data_ptr()
+    ws = 0
+    if workspace is not None:
+        ws = _dev(workspace, "workspace").data_ptr()
+        need = _moe_need(lib().cascadia_int4_tuning_generation(), torch.cuda.current_device(),
+                         H, experts.inter, experts.group_size, experts.scale_dtype, experts.tiling,
+                         experts.n_experts, experts.shared and experts.shared.inter,
+                         experts.shared and experts.shared.tiling, top_k, T)
+        if workspace.nbytes < need:
+            raise ValueError(f"workspace has {workspace.nbytes} bytes, the call needs {need}")
     check("cascadia_int4_moe_forward", lib().cascadia_int4_moe_forward(
         C.byref(experts._struct()), C.byref(R), x.data_ptr(), res, T, out.data_ptr(), io, wo, ws,
         _stream()))
@@ -917,7 +961,13 @@ def ov_gemv(segments, k_cols: int, group_size: int, act, out, workspace=None):
     rows = act.numel() // k_cols
     _expect(act.numel() == rows * k_cols and rows >= 1, "act must be [rows, k_cols]")
     _expect(out.numel() == rows * n_total, "out must be [rows, sum of n_rows]")
-    ws = 0 if workspace is None else _dev(workspace, "workspace").data_ptr()
+    ws = 0
+    if workspace is not None:
+        ws = _dev(workspace, "workspace").data_ptr()
+        need = lib().cascadia_int4_ov_gemv_workspace_bytes(segs, len(segments), k_cols, group_size,
+                                                           rows)
+        if workspace.nbytes < need:
+            raise ValueError(f"workspace has {workspace.nbytes} bytes, the call needs {need}")
     check("cascadia_int4_ov_gemv", lib().cascadia_int4_ov_gemv(
         segs, len(segments), k_cols, group_size, act.data_ptr(),
         int(act.dtype == torch.float16), rows, out.data_ptr(), int(out.dtype == torch.float16),

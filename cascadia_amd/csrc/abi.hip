@@ -326,8 +326,10 @@ size_t ffn_seed_bytes(uint32_t inter, uint32_t group, uint32_t n_tokens) {
   return (((size_t)(inter / cai4::gg_group_width((int)group)) *
            cai4::gg_rows_pad((int)n_tokens) * 4) + 255) & ~(size_t)255;
 }
+// n_plan: the rows whose plan it is, of n_tokens or fewer (ffn_workspace).
 size_t ffn_tile_workspace(int num_cus, uint32_t hidden, uint32_t inter, uint32_t group,
-                          uint32_t n_tokens, bool x_f32, bool out_bf16, bool lean) {
+                          uint32_t n_tokens, bool x_f32, bool out_bf16, bool lean,
+                          uint32_t n_plan) {
   if (lean) {  // two planes, then the seeds of x (and its planes) or of the intermediate
     const size_t rp = (size_t)cai4::gg_rows_pad((int)n_tokens) + 128;
     const int gw = cai4::gg_group_width((int)group);
@@ -336,39 +338,45 @@ size_t ffn_tile_workspace(int num_cus, uint32_t hidden, uint32_t inter, uint32_t
     const size_t b = al(inter / gw * rp * 4);
     return 2 * ffn_plane_bytes(inter, n_tokens) + (a > b ? a : b);
   }
-  const size_t a = cai4::gg_dense_workspace((int)n_tokens, (int)inter, (int)hidden, (int)group,
+  const size_t a = cai4::gg_dense_workspace((int)n_plan, (int)inter, (int)hidden, (int)group,
                                             x_f32 ? cai4::GG_A_F32 : cai4::GG_A_BF16,
-                                            cai4::GG_SWIGLU_HILO, num_cus);
-  const size_t b = cai4::gg_dense_workspace((int)n_tokens, (int)hidden, (int)inter, (int)group,
+                                            cai4::GG_SWIGLU_HILO, num_cus, false, 8,
+                                            (int)n_tokens);
+  const size_t b = cai4::gg_dense_workspace((int)n_plan, (int)hidden, (int)inter, (int)group,
                                             cai4::GG_A_PLANES,
                                             out_bf16 ? cai4::GG_BF16 : cai4::GG_F32, num_cus,
-                                            true);
+                                            true, 8, (int)n_tokens);
   return 2 * ffn_plane_bytes(inter, n_tokens) + ffn_seed_bytes(inter, group, n_tokens) +
          (a > b ? a : b);
 }
+// n_plan (0: n_tokens): a bound for every count of rows n_plan .. n_tokens, which
+// lie in one step of 32 (rows_upto).
 FfnWorkspace ffn_workspace(int dev, uint32_t hidden, uint32_t inter, uint32_t group,
-                           uint32_t n_tokens, bool x_f32) {
+                           uint32_t n_tokens, bool x_f32, uint32_t n_plan = 0) {
+  if (!n_plan) n_plan = n_tokens;
   const cai4::SkinnyDevice d = device_props(dev);
   size_t tile = 0, lean = 0;
   if (ffn_tile_shape(hidden, inter, group)) {
     for (int bf = 0; bf < 2; ++bf) {
       if (ffn_tiles_pay(hidden, inter, n_tokens, x_f32)) {
         const size_t t =
-            ffn_tile_workspace(d.num_cus, hidden, inter, group, n_tokens, x_f32, bf, false);
+            ffn_tile_workspace(d.num_cus, hidden, inter, group, n_tokens, x_f32, bf, false,
+                               n_plan);
         tile = t > tile ? t : tile;
       }
       if (n_tokens >= ffn_tile_tokens()) {
         const size_t t =
-            ffn_tile_workspace(d.num_cus, hidden, inter, group, n_tokens, x_f32, bf, true);
+            ffn_tile_workspace(d.num_cus, hidden, inter, group, n_tokens, x_f32, bf, true,
+                               n_plan);
         lean = t > lean ? t : lean;
       }
     }
   }
   const cai4::SkinnyPlan gu =
-      cai4::skinny_plan((int)inter, (int)hidden, (int)group, (int)n_tokens,
+      cai4::skinny_plan((int)inter, (int)hidden, (int)group, (int)n_plan,
                         x_f32 ? cai4::A_XF32 : cai4::A_BF16, cai4::EPI_SWIGLU_HILO, d);
   const cai4::SkinnyPlan dn = cai4::skinny_plan((int)hidden, (int)inter, (int)group,
-                                                (int)n_tokens, cai4::A_HILO, cai4::EPI_F32, d);
+                                                (int)n_plan, cai4::A_HILO, cai4::EPI_F32, d);
   const size_t planes = ((size_t)n_tokens * inter * 2 * sizeof(uint16_t) + 255) & ~(size_t)255;
   size_t few = 0;
   if (ffn_few_pays(hidden, inter, group, n_tokens, x_f32)) {
@@ -379,6 +387,41 @@ FfnWorkspace ffn_workspace(int dev, uint32_t hidden, uint32_t inter, uint32_t gr
   return FfnWorkspace{planes,
                       gu.partial_bytes > dn.partial_bytes ? gu.partial_bytes : dn.partial_bytes,
                       few, tile, lean};
+}
+
+// The largest need(lo, hi) over steps of rows that make up 1 .. n, need(lo, hi)
+// being enough for every count lo .. hi.  More rows can need less (fewer slices
+// of K, so smaller partials): a workspace sized for n rows has to serve every
+// call of fewer too.  Up to 64 rows each count is a step, then every 32: within
+// one, the kernels' row counts and routes are the same (no fewer than hi's for
+// a route that begins inside it), and K is cut into no more slices than for lo
+// (the slices' cost grows with the rows, their gain does not).  accepted: more
+// rows than that no call takes.
+template <class Need>
+size_t rows_upto(uint32_t n, size_t accepted, Need need) {
+  if (n > accepted) n = (uint32_t)accepted;
+  size_t most = 0;
+  for (size_t lo = 1, hi; lo <= n; lo = hi + 1) {
+    hi = lo <= 64 ? lo : (lo + 31) / 32 * 32;
+    if (hi > n) hi = n;
+    const size_t b = need((uint32_t)lo, (uint32_t)hi);
+    if (b > most) most = b;
+  }
+  return most;
+}
+
+// Rows that an FFN of bf16 rows, which takes the most, accepts (act_fits).
+size_t accepted_rows(uint32_t hidden, uint32_t inter) {
+  return 0x7FFFFFFFu / (2 * (size_t)(hidden > inter ? hidden : inter));
+}
+
+// Enough for an FFN of any number of rows up to n, f32 or bf16.
+size_t ffn_workspace_upto(int dev, uint32_t hidden, uint32_t inter, uint32_t group, uint32_t n) {
+  return rows_upto(n, accepted_rows(hidden, inter), [&](uint32_t lo, uint32_t hi) {
+    const size_t f = ffn_workspace(dev, hidden, inter, group, hi, true, lo).total();
+    const size_t b = ffn_workspace(dev, hidden, inter, group, hi, false, lo).total();
+    return f > b ? f : b;
+  });
 }
 
 // The expert FFN on the MFMA-tile GEMMs: gate/up with the SwiGLU epilogue
@@ -577,21 +620,22 @@ struct SparseWorkspace {
   size_t lanes, slots, cnt, partials, total;
 };
 SparseWorkspace sparse_workspace(int dev, uint32_t hidden, uint32_t inter, uint32_t group,
-                                 uint32_t n_tokens) {
+                                 uint32_t n_tokens, uint32_t n_plan = 0) {
+  if (!n_plan) n_plan = n_tokens;  // as ffn_workspace's
   const cai4::SkinnyDevice d = device_props(dev);
   size_t part = 0;
   const cai4::SkinnyPlan plans[6] = {
-      cai4::skinny_plan((int)inter, (int)hidden, (int)group, (int)n_tokens, cai4::A_XF32,
+      cai4::skinny_plan((int)inter, (int)hidden, (int)group, (int)n_plan, cai4::A_XF32,
                         cai4::EPI_PAIR_F32, d),
-      cai4::skinny_plan((int)inter, (int)hidden, (int)group, (int)n_tokens, cai4::A_BF16,
+      cai4::skinny_plan((int)inter, (int)hidden, (int)group, (int)n_plan, cai4::A_BF16,
                         cai4::EPI_PAIR_F32, d),
-      cai4::skinny_plan((int)inter, (int)hidden, (int)group, (int)n_tokens, cai4::A_XF32,
+      cai4::skinny_plan((int)inter, (int)hidden, (int)group, (int)n_plan, cai4::A_XF32,
                         cai4::EPI_F32, d),
-      cai4::skinny_plan((int)inter, (int)hidden, (int)group, (int)n_tokens, cai4::A_BF16,
+      cai4::skinny_plan((int)inter, (int)hidden, (int)group, (int)n_plan, cai4::A_BF16,
                         cai4::EPI_F32, d),
-      cai4::skinny_plan((int)hidden, (int)inter, (int)group, (int)n_tokens, cai4::A_XF32,
+      cai4::skinny_plan((int)hidden, (int)inter, (int)group, (int)n_plan, cai4::A_XF32,
                         cai4::EPI_F32, d),
-      cai4::skinny_plan((int)hidden, (int)inter, (int)group, (int)n_tokens, cai4::A_XF32,
+      cai4::skinny_plan((int)hidden, (int)inter, (int)group, (int)n_plan, cai4::A_XF32,
                         cai4::EPI_BF16, d)};
   for (const cai4::SkinnyPlan &p : plans) part = p.partial_bytes > part ? p.partial_bytes : part;
   SparseWorkspace w;
@@ -602,8 +646,8 @@ SparseWorkspace sparse_workspace(int dev, uint32_t hidden, uint32_t inter, uint3
                    4);
   w.partials = part;
   w.total = 3 * w.lanes + w.slots + w.cnt + part;
-  const FfnWorkspace f = ffn_workspace(dev, hidden, inter, group, n_tokens, true);
-  const FfnWorkspace b = ffn_workspace(dev, hidden, inter, group, n_tokens, false);
+  const FfnWorkspace f = ffn_workspace(dev, hidden, inter, group, n_tokens, true, n_plan);
+  const FfnWorkspace b = ffn_workspace(dev, hidden, inter, group, n_tokens, false, n_plan);
   const size_t dense = f.total() > b.total() ? f.total() : b.total();
   if (dense > w.total) w.total = dense;
   return w;
@@ -813,7 +857,8 @@ struct AxpyFfnWorkspace {
   uint32_t chunk;  // tokens per AXPY launch pair
 };
 AxpyFfnWorkspace axpy_ffn_workspace(int dev, uint32_t hidden, uint32_t inter, uint32_t group,
-                                    uint32_t n_tokens) {
+                                    uint32_t n_tokens, uint32_t n_plan = 0) {
+  if (!n_plan) n_plan = n_tokens;  // as ffn_workspace's
   const cai4::SkinnyDevice d = device_props(dev);
   AxpyFfnWorkspace w;
   // one token's partial rows: one per lane group (128 lanes on the
@@ -829,10 +874,10 @@ AxpyFfnWorkspace axpy_ffn_workspace(int dev, uint32_t hidden, uint32_t inter, ui
   w.lanes = align256((size_t)n_tokens * inter * 4);
   w.slots = sparse_slot_bytes(inter, n_tokens);
   w.cnt = align256((size_t)n_tokens * groups * 4);
-  const size_t pp = cai4::skinny_plan((int)inter, (int)hidden, (int)group, (int)n_tokens,
+  const size_t pp = cai4::skinny_plan((int)inter, (int)hidden, (int)group, (int)n_plan,
                                       cai4::A_XF32, cai4::EPI_PAIR_F32, d)
                         .partial_bytes;
-  const size_t pg = cai4::skinny_plan((int)inter, (int)hidden, (int)group, (int)n_tokens,
+  const size_t pg = cai4::skinny_plan((int)inter, (int)hidden, (int)group, (int)n_plan,
                                       cai4::A_XF32, cai4::EPI_F32, d)
                         .partial_bytes;  // the gate alone (rows-subset path)
   w.part_gemm = align256(pp > pg ? pp : pg);
@@ -1023,6 +1068,22 @@ bool prefill_shape(const cascadia_int4_layout *L, uint32_t seq, bool x_f32) {
   return seq >= 64 || tiles_pay(seq, 64, bytes, 33, (size_t)22 << 20);
 }
 
+// ov_gemv's: the activations as f32, the output as f32, the GEMVs' partials; for
+// every count of rows n_plan .. rows (as ffn_workspace's).
+size_t ov_workspace(int dev, const cascadia_int4_ov_segment *segs, uint32_t n_segs,
+                    uint32_t k_cols, uint32_t group, uint32_t rows, uint32_t n_plan) {
+  const cai4::SkinnyDevice d = device_props(dev);
+  size_t n_total = 0, part = 0;
+  for (uint32_t i = 0; i < n_segs; ++i) {
+    n_total += segs[i].n_rows;
+    const size_t pb = cai4::skinny_plan((int)segs[i].n_rows, (int)k_cols, (int)group, (int)n_plan,
+                                        cai4::A_XF32, cai4::EPI_F32, d)
+                          .partial_bytes;
+    part = pb > part ? pb : part;
+  }
+  return align256((size_t)rows * k_cols * 4) + align256((size_t)rows * n_total * 4) + part;
+}
+
 // ---- sparse-MoE layer ----
 
 bool has_shared(const cascadia_int4_moe_layer *L) {
@@ -1116,6 +1177,45 @@ MoePlan moe_plan(int dev, const cascadia_int4_moe_layer *L, uint32_t top_k, uint
                                                               : m.dn.partial_bytes;
   m.ws = cai4::moe_workspace((int)T, H, I, (int)L->n_experts, (int)top_k, C, part, sh, sh_ws);
   return m;
+}
+
+// Enough for a layer of any number of tokens up to T, with given ids or routed:
+// the regions that grow with the tokens at T, beside the largest partials and
+// shared expert's workspace of any fewer (rows_upto has why those may be larger).
+size_t moe_workspace_upto(int dev, const cascadia_int4_moe_layer *L, uint32_t top_k, uint32_t T) {
+  const cai4::SkinnyDevice d = device_props(dev);
+  const int H = (int)L->hidden, I = (int)L->inter, E = (int)L->n_experts, G = (int)L->group_size;
+  const int k = (int)top_k;
+  const bool mfma = L->tiling == CASCADIA_INT4_TILING_MFMA;
+  size_t part = 0;
+  int seen[2][2] = {{-1, -1}, {-1, -1}};  // the last chunk rows and chunks planned for
+  for (uint32_t t = 1; t <= T; ++t)
+    for (int given = 0; given < 2; ++given) {
+      const int C = moe_tiles(L, top_k, t, false)
+                        ? 16
+                        : cai4::moe_chunk_rows((int)t, given ? (int)t * k : (int)t, mfma);
+      const int maxc = cai4::moe_max_chunks((int)t, E, k, C);
+      if (seen[given][0] == C && seen[given][1] == maxc) continue;
+      seen[given][0] = C;
+      seen[given][1] = maxc;
+      for (const cai4::SkinnyPlan &p :
+           {cai4::skinny_plan_grouped(I, H, G, C, maxc, cai4::A_GATHER, cai4::EPI_SWIGLU_HILO, d),
+            cai4::skinny_plan_grouped(H, I, G, C, maxc, cai4::A_HILO, cai4::EPI_BF16, d)})
+        if (p.partial_bytes > part) part = p.partial_bytes;
+    }
+  size_t sh = 0, sh_ws = 0;
+  if (has_shared(L)) {
+    sh = (size_t)T * H * sizeof(float);
+    sh_ws = ffn_workspace_upto(dev, L->hidden, L->shared_inter, L->group_size, T);
+  }
+  // one row per chunk: as many chunks as any chunk size takes
+  if (!moe_tiles(L, top_k, T, false))
+    return cai4::moe_workspace((int)T, H, I, E, k, 1, part, sh, sh_ws).total;
+  const int gw = cai4::gg_group_width(G);
+  return cai4::moe_workspace((int)T, H, I, E, k, 1, part, sh, sh_ws, (size_t)T * H * 2,
+                             (size_t)(H / gw) * cai4::gg_rows_pad((int)T) * 4,
+                             (size_t)(I / gw) * cai4::gg_rows_pad((int)(T * top_k)) * 4, 16)
+      .total;
 }
 
 int moe_forward(const cascadia_int4_moe_layer *L, const cascadia_int4_routing *R, const float *x,
@@ -1722,10 +1822,8 @@ size_t cascadia_int4_ffn_workspace_bytes(uint32_t hidden, uint32_t inter, uint32
                                          uint32_t n_tokens) {
   int dev;
   if (current_device(&dev)) return 0;
-  if (group_size == 0 || group_size % 32) return 0;
-  const FfnWorkspace f = ffn_workspace(dev, hidden, inter, group_size, n_tokens, true);
-  const FfnWorkspace b = ffn_workspace(dev, hidden, inter, group_size, n_tokens, false);
-  return f.total() > b.total() ? f.total() : b.total();
+  if (hidden == 0 || inter == 0 || group_size == 0 || group_size % 32) return 0;
+  return ffn_workspace_upto(dev, hidden, inter, group_size, n_tokens);
 }
 
 int cascadia_int4_expert_forward_device(uint32_t hidden, uint32_t inter, uint32_t group_size,
@@ -1812,8 +1910,10 @@ size_t cascadia_int4_ffn_sparse_workspace_bytes(uint32_t hidden, uint32_t inter,
                                                 uint32_t group_size, uint32_t n_tokens) {
   int dev;
   if (current_device(&dev)) return 0;
-  if (group_size == 0 || group_size % 32) return 0;
-  return sparse_workspace(dev, hidden, inter, group_size, n_tokens).total;
+  if (hidden == 0 || inter == 0 || group_size == 0 || group_size % 32) return 0;
+  return rows_upto(n_tokens, accepted_rows(hidden, inter), [&](uint32_t lo, uint32_t hi) {
+    return sparse_workspace(dev, hidden, inter, group_size, hi, lo).total;
+  });
 }
 
 int cascadia_int4_ffn_forward_sparse_f32(uint32_t hidden, uint32_t inter, uint32_t group_size,
@@ -1852,16 +1952,10 @@ size_t cascadia_int4_ov_gemv_workspace_bytes(const cascadia_int4_ov_segment *seg
                                              uint32_t group_size, uint32_t rows) {
   int dev;
   if (!segs || current_device(&dev) || group_size == 0 || group_size % 32) return 0;
-  const cai4::SkinnyDevice d = device_props(dev);
-  size_t n_total = 0, part = 0;
-  for (uint32_t i = 0; i < n_segs; ++i) {
-    n_total += segs[i].n_rows;
-    const size_t pb = cai4::skinny_plan((int)segs[i].n_rows, (int)k_cols, (int)group_size,
-                                        (int)rows, cai4::A_XF32, cai4::EPI_F32, d)
-                          .partial_bytes;
-    part = pb > part ? pb : part;
-  }
-  return align256((size_t)rows * k_cols * 4) + align256((size_t)rows * n_total * 4) + part;
+  if (k_cols == 0) return 0;
+  return rows_upto(rows, 0x7FFFFFFFu / (4 * (size_t)k_cols), [&](uint32_t lo, uint32_t hi) {
+    return ov_workspace(dev, segs, n_segs, k_cols, group_size, hi, lo);
+  });
 }
 
 int cascadia_int4_ov_gemv(const cascadia_int4_ov_segment *segs, uint32_t n_segs,
@@ -1886,8 +1980,7 @@ int cascadia_int4_ov_gemv(const cascadia_int4_ov_segment *segs, uint32_t n_segs,
   int dev;
   if (int rc = current_device(&dev)) return rc;
   hipStream_t st = (hipStream_t)stream;
-  const size_t need =
-      cascadia_int4_ov_gemv_workspace_bytes(segs, n_segs, k_cols, group_size, rows);
+  const size_t need = ov_workspace(dev, segs, n_segs, k_cols, group_size, rows, rows);
   void *ws = workspace;
   if (!ws) {
     if (int rc = lib_workspace(dev, need, &ws, st)) return rc;
@@ -1925,8 +2018,10 @@ size_t cascadia_int4_ffn_sparse_axpy_workspace_bytes(uint32_t hidden, uint32_t i
                                                      uint32_t group_size, uint32_t n_tokens) {
   int dev;
   if (current_device(&dev)) return 0;
-  if (group_size == 0 || group_size % 32) return 0;
-  return axpy_ffn_workspace(dev, hidden, inter, group_size, n_tokens).total;
+  if (hidden == 0 || inter == 0 || group_size == 0 || group_size % 32) return 0;
+  return rows_upto(n_tokens, accepted_rows(hidden, inter), [&](uint32_t lo, uint32_t hi) {
+    return axpy_ffn_workspace(dev, hidden, inter, group_size, hi, lo).total;
+  });
 }
 
 int cascadia_int4_ffn_forward_sparse_axpy_f32(uint32_t hidden, uint32_t inter,
@@ -2004,9 +2099,7 @@ size_t cascadia_int4_moe_workspace_bytes(const cascadia_int4_moe_layer *layer, u
   if (moe_check(layer, top_k, n_tokens)) return 0;
   int dev;
   if (current_device(&dev)) return 0;
-  const MoePlan a = moe_plan(dev, layer, top_k, n_tokens, false);
-  const MoePlan b = moe_plan(dev, layer, top_k, n_tokens, true);
-  return a.ws.total > b.ws.total ? a.ws.total : b.ws.total;
+  return moe_workspace_upto(dev, layer, top_k, n_tokens);
 }
 
 int cascadia_int4_moe_forward(const cascadia_int4_moe_layer *layer,

@@ -909,12 +909,13 @@ hipError_t gg_reduce_slices(const GgArgs &a, int nsl, hipStream_t st) {
 }
 
 size_t gg_dense_workspace(int M, int N, int K, int G, int amode, int epi, int num_cus,
-                          bool have_seeds, int max_slices) {
+                          bool have_seeds, int max_slices, int rows) {
   const bool sw = epi == GG_SWIGLU_HILO;
-  size_t b = have_seeds ? 0 : al256((size_t)(K / gg_group_width(G)) * gg_rows_pad(M) * 4);
-  if (amode == GG_A_F32) b += 2 * al256((size_t)M * K * 2);  // the A planes
+  if (!rows) rows = M;
+  size_t b = have_seeds ? 0 : al256((size_t)(K / gg_group_width(G)) * gg_rows_pad(rows) * 4);
+  if (amode == GG_A_F32) b += 2 * al256((size_t)rows * K * 2);  // the A planes
   const GgPlan p = gg_plan(M, N, K, G, amode != GG_A_BF16, sw, num_cus, max_slices);
-  return b + (p.nsl > 1 ? (size_t)p.nsl * M * (sw ? 2 * (size_t)N : N) * 4 : 0);
+  return b + (p.nsl > 1 ? (size_t)p.nsl * rows * (sw ? 2 * (size_t)N : N) * 4 : 0);
 }
 
 hipError_t gg_dense(GgArgs a, int amode, void *ws, int num_cus, hipStream_t st, int max_slices) {

@@ -76,9 +76,11 @@ enum GgAMode { GG_A_BF16 = 0, GG_A_F32 = 1, GG_A_PLANES = 2 };
 // split-K partials) and the launches (gg_prep unless a.seeds is given, the
 // GEMM, the split-K reduce).  With GG_SWIGLU_HILO and a.seeds_out the seeds of
 // the planes written are left there.  max_slices 1: no split of K (no
-// partials), for a workspace that cannot grow.
+// partials), for a workspace that cannot grow.  rows (0: M): the size for that
+// many rows in the plan of M, which lie in one step of 64 rows: its partials
+// are enough for every count M .. rows.
 size_t gg_dense_workspace(int M, int N, int K, int G, int amode, int epi, int num_cus,
-                          bool have_seeds = false, int max_slices = 8);
+                          bool have_seeds = false, int max_slices = 8, int rows = 0);
 hipError_t gg_dense(GgArgs a, int amode, void *ws, int num_cus, hipStream_t st,
                     int max_slices = 8);
 

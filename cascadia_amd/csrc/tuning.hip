@@ -69,3 +69,7 @@ int tuning_env(const char *name, int absent) {
 extern "C" void cascadia_int4_reload_tuning(void) {
   g_gen.fetch_add(1, std::memory_order_acq_rel);
 }
+
+extern "C" uint32_t cascadia_int4_tuning_generation(void) {
+  return g_gen.load(std::memory_order_acquire);
+}

@@ -113,6 +113,10 @@ int cascadia_int4_synchronize(void *stream);
  * counterpart in the crate, which has no plan overrides. */
 void cascadia_int4_reload_tuning(void);
 
+/* A number that changes with every reload_tuning: the *_workspace_bytes
+ * results may change with it. */
+uint32_t cascadia_int4_tuning_generation(void);
+
 /* y[r] = sum_c (nibble[r,c]-8) * scale[r, c/G] * x[c] for one f32 vector.
  * Replaces dequant_gemv_int4 (src/kernel.rs:31-71) and
  * dequant_gemv_int4_auto (src/kernel_avx512.rs:274-297).
@@ -214,9 +218,11 @@ int cascadia_int4_tile_expert(uint32_t hidden, uint32_t inter, uint32_t group_si
                               const cascadia_int4_expert *src, uint8_t *dst,
                               cascadia_int4_expert *out, void *stream);
 
-/* Workspace bytes the expert / FFN entry points need for n_tokens rows on the
- * current device (the launch plan depends on its CU count); 0 on bad
- * arguments.  No counterpart in the crate, which allocates per call. */
+/* Workspace bytes the expert / FFN entry points need for any call of up to
+ * n_tokens rows on the current device (the launch plan depends on its CU
+ * count); 0 on bad arguments.  Every *_workspace_bytes result below is enough
+ * for fewer rows too, so one workspace of the largest batch serves them all.
+ * No counterpart in the crate, which allocates per call. */
 size_t cascadia_int4_ffn_workspace_bytes(uint32_t hidden, uint32_t inter, uint32_t group_size,
                                          uint32_t n_tokens);
 
@@ -240,11 +246,11 @@ int cascadia_int4_expert_forward_device(uint32_t hidden, uint32_t inter, uint32_
  * and split-K partials live in a file-scope device array of
  * CASCADIA_INT4_NOALLOC_SCRATCH_BYTES per GPU, held until the process ends;
  * a call that would need more in any form returns CASCADIA_INT4_ERR_ARG
- * (config 1's Llama-3-8B FFN fits up to 64 tokens), and one whose
- * cascadia_int4_ffn_workspace_bytes exceeds it but whose least form fits runs
- * in that form (results within rounding order of the _device entry point's).  Every call on one GPU shares that array, so
- * calls that overlap on one GPU (different streams, or threads) race;
- * serialise them.  Otherwise the same kernels and results as _device. */
+ * (config 1's Llama-3-8B FFN fits up to 64 tokens), and one whose usual form
+ * needs more but whose least form fits runs in that form (results within
+ * rounding order of the _device entry point's).  Every call on one GPU shares
+ * that array, so calls that overlap on one GPU (different streams, or threads)
+ * race; serialise them.  Otherwise the same kernels and results as _device. */
 #define CASCADIA_INT4_NOALLOC_SCRATCH_BYTES ((size_t)8 << 20)
 int cascadia_int4_expert_forward_noalloc(uint32_t hidden, uint32_t inter, uint32_t group_size,
                                          uint32_t scale_dtype,
