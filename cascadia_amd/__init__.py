@@ -31,7 +31,8 @@ from .api import (GROUP_SIZE, HIDDEN, INTERMEDIATE, NIBBLES_PER_INT32, ExpertSou
                   ffn_forward_sparse_axpy_f32_per_channel, ffn_sparse_axpy_workspace_bytes,
                   ffn_workspace_bytes, transpose_requantize_down, dequant_axpy_int4_active,
                   dequant_axpy_int4_active_auto, fill_bytes, fill_normal,
-                  fill_scales, gate_up_silu, gemm_int4_bf16, MoEExperts, moe_forward,
+                  fill_scales, gate_up_silu, gemm_int4_bf16, gemm_workspace_bytes, MoEExperts,
+                  moe_forward,
                   moe_workspace_bytes, ov_gemv, ov_to_crate, quantize_int4_group, tile_weights,
                   tiled_sizes)
 
@@ -45,7 +46,8 @@ __all__ = [
     "ffn_forward_sparse_axpy_f32", "ffn_forward_sparse_axpy_f32_mode",
     "ffn_forward_sparse_axpy_f32_per_channel", "ffn_sparse_axpy_workspace_bytes",
     "transpose_requantize_down", "dequant_axpy_int4_active", "dequant_axpy_int4_active_auto", "fill_bytes",
-    "fill_normal", "fill_scales", "gate_up_silu", "gemm_int4_bf16", "tile_weights",
+    "fill_normal", "fill_scales", "gate_up_silu", "gemm_int4_bf16",
+    "gemm_workspace_bytes", "tile_weights",
     "tiled_sizes", "TILING_CRATE", "TILING_MFMA", "MoEExperts", "moe_forward",
     "moe_workspace_bytes", "ov_gemv", "ov_to_crate", "quantize_int4_group", "ROUTE_IDS",
     "ROUTE_SIGMOID_BIAS",

@@ -87,6 +87,8 @@ SIGNATURES = {
     "cascadia_int4_dequant_gemm_multi": (_i32, [_LP, _vp, _vp, _vp, _u32, _vp, _vp]),
     "cascadia_int4_dequant_gemm_bf16in": (_i32, [_LP, _vp, _vp, _vp, _u32, _vp, _vp]),
     "cascadia_int4_gemm_bf16": (_i32, [_LP, _vp, _vp, _vp, _u32, _vp, _vp]),
+    "cascadia_int4_gemm_workspace_bytes": (_sz, [_LP, _u32, _u32]),
+    "cascadia_int4_gemm": (_i32, [_LP, _vp, _vp, _vp, _u32, _u32, _vp, _u32, _vp, _vp]),
     "cascadia_int4_tiled_sizes": (_i32, [_LP, C.POINTER(_sz), C.POINTER(_sz)]),
     "cascadia_int4_tile_weights": (_i32, [_LP, _vp, _vp, _vp, _vp, _vp]),
     "cascadia_int4_expert_bytes": (_sz, [_u32, _u32, _u32]),

@@ -304,11 +304,40 @@ def build_active_mask_per_channel(gate_out, thresholds):
     return build_active_mask_mode(gate_out, SparsityMode.PerChannel(thresholds))
 
 
+def gemm_workspace_bytes(n_rows, k_cols, seq, x_f32, group_size=GROUP_SIZE,
+                         tiling=TILING_CRATE) -> int:
+    """Workspace bytes of dequant_gemm_int4_multi_auto / gemm_int4_bf16 for up to
+    seq rows on the current device."""
+    return int(lib().cascadia_int4_gemm_workspace_bytes(
+        _layout(n_rows, k_cols, group_size, SCALE_BF16, tiling), int(x_f32), seq))
+
+
+@functools.lru_cache(maxsize=1024)
+def _gemm_need(tuning, device, *dims):
+    return gemm_workspace_bytes(*dims)
+
+
+def _gemm_ws(L, packed, scale_bits, xs, seq, ys, workspace, n_rows, k_cols, group_size, tiling):
+    """A GEMM over a caller's workspace."""
+    _dev(workspace, "workspace")
+    x_f32 = xs.dtype == torch.float32
+    need = _gemm_need(lib().cascadia_int4_tuning_generation(), torch.cuda.current_device(),
+                      *map(int, (n_rows, k_cols, seq, x_f32, group_size, tiling)))
+    if workspace.nbytes < need:
+        raise ValueError(f"workspace has {workspace.nbytes} bytes, the call needs {need}")
+    check("cascadia_int4_gemm", lib().cascadia_int4_gemm(
+        L, packed.data_ptr(), scale_bits.data_ptr(), xs.data_ptr(), int(x_f32), seq, ys.data_ptr(),
+        int(ys.dtype == torch.float32), workspace.data_ptr(), _stream()))
+    return ys
+
+
 def dequant_gemm_int4_multi_auto(packed, scale_bits, xs, n_rows, k_cols, seq, ys,
                                  group_size=GROUP_SIZE, scale_dtype=SCALE_BF16,
-                                 tiling=TILING_CRATE):
+                                 tiling=TILING_CRATE, workspace=None):
     """ys[t*n_rows + r] for t < seq (kernel_avx512_multi.rs:207-245).
-    xs f32 [seq, k_cols]; bf16 xs use the exact bf16 MFMA path."""
+    xs f32 [seq, k_cols]; bf16 xs use the exact bf16 MFMA path.  In a graph
+    capture give a workspace (gemm_workspace_bytes): without one the call is
+    recorded in a form that is slower from 17 rows on."""
     _check_weights(packed, scale_bits, n_rows, k_cols, group_size, tiling)
     _dev(xs, "xs"), _dev(ys, "ys")
     _expect(seq >= 1, "seq must be >= 1")
@@ -322,6 +351,9 @@ def dequant_gemm_int4_multi_auto(packed, scale_bits, xs, n_rows, k_cols, seq, ys
     else:
         _expect(_is_bf16_bits(xs), "xs must be f32 or bf16")
         fn = "cascadia_int4_dequant_gemm_bf16in"
+    if workspace is not None:
+        return _gemm_ws(L, packed, scale_bits, xs, seq, ys, workspace, n_rows, k_cols, group_size,
+                        tiling)
     check(fn, getattr(lib(), fn)(L, packed.data_ptr(), scale_bits.data_ptr(),
                                  xs.data_ptr(), seq, ys.data_ptr(), _stream()))
     return ys
@@ -331,13 +363,18 @@ dequant_gemm_int4_multi_blocked_auto = dequant_gemm_int4_multi_auto  # _blocked.
 
 
 def gemm_int4_bf16(packed, scale_bits, xs_bf16, n_rows, k_cols, seq, ys_bf16,
-                   group_size=GROUP_SIZE, scale_dtype=SCALE_BF16, tiling=TILING_CRATE):
-    """Prefill GEMM: bf16 [seq, k_cols] in, bf16 [seq, n_rows] out (f32 inside)."""
+                   group_size=GROUP_SIZE, scale_dtype=SCALE_BF16, tiling=TILING_CRATE,
+                   workspace=None):
+    """Prefill GEMM: bf16 [seq, k_cols] in, bf16 [seq, n_rows] out (f32 inside).
+    workspace: as dequant_gemm_int4_multi_auto's."""
     _check_weights(packed, scale_bits, n_rows, k_cols, group_size, tiling)
     _dev(xs_bf16, "xs_bf16"), _dev(ys_bf16, "ys_bf16")
     _expect(_is_bf16_bits(xs_bf16) and xs_bf16.numel() == seq * k_cols, "xs_bf16 [seq, k_cols] bf16")
     _expect(_is_bf16_bits(ys_bf16) and ys_bf16.numel() == seq * n_rows, "ys_bf16 [seq, n_rows] bf16")
     L = _layout(n_rows, k_cols, group_size, scale_dtype, tiling)
+    if workspace is not None:
+        return _gemm_ws(L, packed, scale_bits, xs_bf16, seq, ys_bf16, workspace, n_rows, k_cols,
+                        group_size, tiling)
     check("cascadia_int4_gemm_bf16", lib().cascadia_int4_gemm_bf16(
         L, packed.data_ptr(), scale_bits.data_ptr(), xs_bf16.data_ptr(), seq,
         ys_bf16.data_ptr(), _stream()))

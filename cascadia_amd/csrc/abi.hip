@@ -5,6 +5,7 @@
 // CASCADIA_INT4_ERR_ARG instead of panicking; nothing throws across the ABI.
 #include <stdlib.h>
 
+#include <atomic>
 #include <mutex>
 #include <new>
 
@@ -27,13 +28,26 @@ namespace {
 
 constexpr int kMaxDevices = 64;
 
+// A workspace of the library's own.  A call holds mu from before its first
+// launch over the buffer until after its last: two threads on one stream then
+// use it one call after the other, in the stream's order.
+struct Buffer {
+  std::mutex mu;
+  void *p = nullptr;
+  std::atomic<size_t> bytes{0};
+};
+
+constexpr int kStreamBuffers = 16;
+
 struct DeviceState {
   int num_cus = 0;
   size_t max_lds = 0;
-  void *ws = nullptr;  // library-owned workspace (grow-only)
-  size_t ws_bytes = 0;
-  void **retired = nullptr;  // earlier, smaller workspaces: held, never freed
-  size_t n_retired = 0;
+  Buffer streams[kStreamBuffers];  // one for each of the first streams seen
+  hipStream_t owner[kStreamBuffers] = {};
+  int n_owners = 0;
+  Buffer others;  // every further stream's, each use after the one before
+  hipEvent_t others_used = nullptr;
+  Buffer recorded;  // of the calls that graphs recorded
   hipStream_t side = nullptr;  // second stream for independent work (default priority)
   hipEvent_t fork = nullptr, join = nullptr;
 };
@@ -114,51 +128,118 @@ int side_stream(int dev, hipStream_t *side, hipEvent_t *fork, hipEvent_t *join) 
   return CASCADIA_INT4_OK;
 }
 
-// Library workspace of at least `bytes` on the current device.  Growing it
-// allocates a larger buffer (at least twice the old size) and RETIRES the old
-// one without freeing it: a graph captured while the old buffer was current
-// keeps its address in its kernel arguments and stays valid to replay.
-// Retired buffers are held until the process ends (their total stays below
-// the current buffer's size, since each growth at least doubles).  A growth
-// cannot be recorded by a stream capture: while `st` is capturing, a call that
-// would grow the workspace is refused with ERR_ARG (pass a workspace of the
-// *_workspace_bytes size instead).
-int lib_workspace(int dev, size_t bytes, void **out, hipStream_t st) {
-  std::lock_guard<std::mutex> lk(g_mu);
-  DeviceState &d = g_dev[dev];
-  if (d.ws_bytes < bytes) {
-    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(st, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone)
-      return CASCADIA_INT4_ERR_ARG;
-    size_t sz = bytes < (1u << 20) ? (1u << 20) : bytes;
-    if (sz < 2 * d.ws_bytes) sz = 2 * d.ws_bytes;
-    void *p = nullptr;
-    if (hipMalloc(&p, sz) != hipSuccess) {
+// Whether work on st is being recorded into a graph (or st cannot say).
+bool capturing(hipStream_t st) {
+  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+  return hipStreamIsCapturing(st, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone;
+}
+
+// A buffer's new memory: at least twice the old size, or `bytes`.
+int alloc_larger(size_t bytes, size_t old, void **p, size_t *size) {
+  size_t sz = bytes < (1u << 20) ? (1u << 20) : bytes;
+  if (sz < 2 * old) sz = 2 * old;
+  if (hipMalloc(p, sz) != hipSuccess) {
+    (void)hipGetLastError();
+    // the doubling is a preference, the request is the requirement
+    sz = bytes;
+    if (hipMalloc(p, sz) != hipSuccess) {
       (void)hipGetLastError();
-      // the doubling is a preference, the request is the requirement
-      p = nullptr;
-      sz = bytes;
-      if (hipMalloc(&p, sz) != hipSuccess) {
-        (void)hipGetLastError();
-        return CASCADIA_INT4_ERR_NOMEM;
-      }
+      return CASCADIA_INT4_ERR_NOMEM;
     }
-    if (d.ws) {
-      // kept alive, never reused: captured graphs may still address it
-      void **grown = static_cast<void **>(realloc(d.retired, (d.n_retired + 1) * sizeof(void *)));
-      if (!grown) {
-        (void)hipFree(p);
-        return CASCADIA_INT4_ERR_NOMEM;
-      }
-      d.retired = grown;
-      d.retired[d.n_retired++] = d.ws;
-    }
-    d.ws = p;
-    d.ws_bytes = sz;
   }
-  *out = d.ws;
+  *size = sz;
   return CASCADIA_INT4_OK;
 }
+
+// The library's workspace for one call on one stream, held until the object
+// goes (after the call's launches).  Each stream has its own, so that calls on
+// different streams run beside each other; streams past the first kStreamBuffers
+// (and the per-thread stream, one handle of many streams) share one, whose uses
+// an event orders.  A stream is known by its handle: one that is destroyed must
+// have finished its calls.
+//
+// A recorded call runs whenever its graph is replayed, beside whatever eager
+// calls there are then, so graphs have a buffer of their own, grown ahead by the
+// eager calls (a capture cannot record an allocation: a call that does not fit is
+// refused with ERR_ARG).  Growing it RETIRES the old memory without freeing it: a
+// graph recorded while it was current keeps its address in its kernel arguments
+// and stays valid to replay (the total held stays below the current size, since
+// each growth at least doubles).  Graphs that use it must not run at the same time.
+class Workspace {
+ public:
+  Workspace() = default;
+  Workspace(const Workspace &) = delete;
+  Workspace &operator=(const Workspace &) = delete;
+  ~Workspace() { release(); }
+
+  // recorded: what the call's recorded form needs of the graphs' buffer.
+  int get(int dev, size_t bytes, hipStream_t st, void **out) { return get(dev, bytes, st, out, bytes); }
+  int get(int dev, size_t bytes, hipStream_t st, void **out, size_t recorded) {
+    release();
+    DeviceState &d = g_dev[dev];
+    if (capturing(st)) {
+      lk_ = std::unique_lock<std::mutex>(d.recorded.mu);
+      if (d.recorded.bytes < bytes) return fail(CASCADIA_INT4_ERR_ARG);
+      *out = d.recorded.p;
+      return CASCADIA_INT4_OK;
+    }
+    Buffer *b = buffer_of(d, st);
+    lk_ = std::unique_lock<std::mutex>(b->mu);
+    if (b == &d.others) {
+      if (!d.others_used) {
+        if (hipEventCreateWithFlags(&d.others_used, hipEventDisableTiming) != hipSuccess) {
+          d.others_used = nullptr;
+          return fail(CASCADIA_INT4_ERR_DEVICE);
+        }
+      } else if (hipStreamWaitEvent(st, d.others_used, 0) != hipSuccess) {
+        return fail(CASCADIA_INT4_ERR_DEVICE);
+      }
+      after_ = d.others_used;
+      st_ = st;
+    }
+    void *p = nullptr;
+    size_t size = 0;
+    if (b->bytes < bytes) {
+      if (int rc = alloc_larger(bytes, b->bytes, &p, &size)) return fail(rc);
+      // the old memory's uses are all on st, or st waits for them
+      if (b->p && hipStreamSynchronize(st) == hipSuccess) (void)hipFree(b->p);
+      b->p = p;
+      b->bytes = size;
+    }
+    *out = b->p;
+    if (d.recorded.bytes < recorded) {  // (or not: a capture of the call is refused then)
+      std::lock_guard<std::mutex> lk(d.recorded.mu);
+      if (d.recorded.bytes < recorded && !alloc_larger(recorded, d.recorded.bytes, &p, &size)) {
+        d.recorded.p = p;  // (the old memory: retired)
+        d.recorded.bytes = size;
+      }
+    }
+    return CASCADIA_INT4_OK;
+  }
+
+ private:
+  static Buffer *buffer_of(DeviceState &d, hipStream_t st) {
+    if (st == hipStreamPerThread) return &d.others;
+    std::lock_guard<std::mutex> lk(g_mu);
+    for (int i = 0; i < d.n_owners; ++i)
+      if (d.owner[i] == st) return &d.streams[i];
+    if (d.n_owners == kStreamBuffers) return &d.others;
+    d.owner[d.n_owners] = st;
+    return &d.streams[d.n_owners++];
+  }
+  void release() {
+    if (after_ && hipEventRecord(after_, st_) != hipSuccess) (void)hipStreamSynchronize(st_);
+    after_ = nullptr;
+    if (lk_.owns_lock()) lk_.unlock();
+  }
+  int fail(int rc) {
+    release();
+    return rc;
+  }
+  std::unique_lock<std::mutex> lk_;
+  hipEvent_t after_ = nullptr;
+  hipStream_t st_ = nullptr;
+};
 
 inline bool aligned(const void *p, size_t a) { return ((uintptr_t)p % a) == 0; }
 
@@ -189,7 +270,8 @@ bool act_fits(int M, int K, int amode) {
 
 // One skinny GEMM (any M), f32 output or fused epilogue.  `partials` is
 // workspace for split-K partial sums (null: the library's own workspace,
-// unless `may_alloc` is false, when a plan that needs partials is an error).
+// unless `may_alloc` is false, when a plan that needs partials is an error: the
+// caller holds a workspace, the library's own or one it was given).
 int run_gemm(const uint8_t *w0, const uint8_t *s0, const uint8_t *w1, const uint8_t *s1,
              int N, int K, int G, int sdt, int tiled, const void *x, const void *x2, int amode,
              int M, void *out, void *out2, int epi, hipStream_t st, void *partials = nullptr,
@@ -218,9 +300,10 @@ int run_gemm(const uint8_t *w0, const uint8_t *s0, const uint8_t *w1, const uint
       return hip_status(cai4::gemv_launch(g, amode, epi, d.num_cus, 0, st));
   }
   const cai4::SkinnyPlan p = cai4::skinny_plan(N, K, G, M, amode, epi, d);
+  Workspace own;
   if (p.partial_bytes && !partials) {
     if (!may_alloc) return CASCADIA_INT4_ERR_ARG;
-    if (int rc = lib_workspace(dev, p.partial_bytes, &partials, st)) return rc;
+    if (int rc = own.get(dev, p.partial_bytes, st, &partials)) return rc;
   }
   cai4::SkinnyArgs a{};
   a.partials = partials;
@@ -568,13 +651,14 @@ int ffn_common(uint32_t hidden, uint32_t inter, uint32_t group, uint32_t sdt,
       !act_fits((int)n_tokens, (int)inter, cai4::A_HILO))
     return CASCADIA_INT4_ERR_ARG;
   const FfnWorkspace need = ffn_workspace(dev, hidden, inter, group, n_tokens, x_f32);
+  Workspace own;
   void *ws = workspace;
   bool lean = need.total() > workspace_bytes;
   if (!ws) {
     // a library workspace that cannot grow now (a capture, no memory) may still
     // hold what the call needs at least
-    if (lib_workspace(dev, need.total(), &ws, st)) {
-      if (int rc = lib_workspace(dev, need.least(), &ws, st)) return rc;
+    if (own.get(dev, need.total(), st, &ws)) {
+      if (int rc = own.get(dev, need.least(), st, &ws)) return rc;
       lean = true;
     }
   } else if (!aligned(ws, 16)) {
@@ -590,8 +674,8 @@ int ffn_common(uint32_t hidden, uint32_t inter, uint32_t group, uint32_t sdt,
   uint16_t *hi = reinterpret_cast<uint16_t *>(ws);
   uint16_t *lo = hi + (size_t)n_tokens * inter;
   void *part = need.partials ? static_cast<uint8_t *>(ws) + need.planes : nullptr;
-  // a caller's workspace (or the static scratch) is never supplemented by an allocation
-  const bool may_alloc = workspace == nullptr;
+  // the workspace, whoever's, has room for the partials: no second one
+  const bool may_alloc = false;
   int rc = run_gemm(e->gate_packed, e->gate_scale, e->up_packed, e->up_scale, (int)inter,
                     (int)hidden, (int)group, (int)sdt, (int)e->tiling, x, nullptr,
                     x_f32 ? cai4::A_XF32 : cai4::A_BF16, (int)n_tokens, hi, lo,
@@ -783,9 +867,10 @@ int sparse_common(uint32_t hidden, uint32_t inter, uint32_t group, uint32_t sdt,
       !act_fits((int)n_tokens, (int)inter, cai4::A_XF32))
     return CASCADIA_INT4_ERR_ARG;
   const SparseWorkspace w = sparse_workspace(dev, hidden, inter, group, n_tokens);
+  Workspace own;
   void *ws = workspace;
   if (!ws) {
-    if (int rc = lib_workspace(dev, w.total, &ws, st)) return rc;
+    if (int rc = own.get(dev, w.total, st, &ws)) return rc;
   }
   uint8_t *b = static_cast<uint8_t *>(ws);
   float *gate = reinterpret_cast<float *>(b);
@@ -800,7 +885,7 @@ int sparse_common(uint32_t hidden, uint32_t inter, uint32_t group, uint32_t sdt,
     // active lanes only (ffn_sparsity.rs:499-527), then the down in full
     (void)upv;
     int rc = sparse_gate(e->gate_packed, e->gate_scale, gd_tiling(e), hidden, inter, group, sdt,
-                         x, amode, n_tokens, gate, thr, true, slots, &n_slots, part, true, st);
+                         x, amode, n_tokens, gate, thr, true, slots, &n_slots, part, false, st);
     if (rc) return rc;
     cai4::SparseSubsetArgs a{};
     a.gate = gate;
@@ -823,10 +908,10 @@ int sparse_common(uint32_t hidden, uint32_t inter, uint32_t group, uint32_t sdt,
     return run_gemm(e->down_packed, e->down_scale, nullptr, nullptr, (int)hidden, (int)inter,
                     (int)group, (int)sdt, gd_tiling(e), mid, nullptr, cai4::A_XF32,
                     (int)n_tokens, out, nullptr, out_bf16 ? cai4::EPI_BF16 : cai4::EPI_F32, st,
-                    part);
+                    part, false);
   }
   int rc = sparse_gate_up(e, hidden, inter, group, sdt, x, amode, n_tokens, gate, upv, thr, true,
-                          slots, &n_slots, part, true, st);
+                          slots, &n_slots, part, false, st);
   if (rc) return rc;
   cai4::SparseMaskArgs m{};
   m.gate = gate;
@@ -846,7 +931,7 @@ int sparse_common(uint32_t hidden, uint32_t inter, uint32_t group, uint32_t sdt,
   return run_gemm(e->down_packed, e->down_scale, nullptr, nullptr, (int)hidden, (int)inter,
                   (int)group, (int)sdt, (int)e->tiling, mid, nullptr, cai4::A_XF32,
                   (int)n_tokens, out, nullptr, out_bf16 ? cai4::EPI_BF16 : cai4::EPI_F32, st,
-                  part);
+                  part, false);
 }
 
 // Workspace of the AXPY-form sparse FFN: gate and up ([n_tokens, inter] f32
@@ -911,9 +996,10 @@ int axpy_ffn(uint32_t hidden, uint32_t inter, uint32_t group, uint32_t sdt,
   int dev;
   if (int rc = current_device(&dev)) return rc;
   const AxpyFfnWorkspace w = axpy_ffn_workspace(dev, hidden, inter, group, n_tokens);
+  Workspace own;
   void *ws = workspace;
   if (!ws) {
-    if (int rc = lib_workspace(dev, w.total, &ws, st)) return rc;
+    if (int rc = own.get(dev, w.total, st, &ws)) return rc;
   }
   uint8_t *b = static_cast<uint8_t *>(ws);
   float *gate = reinterpret_cast<float *>(b);
@@ -934,7 +1020,7 @@ int axpy_ffn(uint32_t hidden, uint32_t inter, uint32_t group, uint32_t sdt,
     (void)upv;
     int rc = sparse_gate(e->gate_packed, e->gate_scale, gd_tiling(e), hidden, inter, group, sdt,
                          x, cai4::A_XF32, n_tokens, gate, thr, false, slots, &n_slots, part_gemm,
-                         workspace == nullptr, st);
+                         false, st);
     if (rc) return rc;
     cai4::SparseSubsetArgs a{};
     a.gate = gate;
@@ -961,7 +1047,7 @@ int axpy_ffn(uint32_t hidden, uint32_t inter, uint32_t group, uint32_t sdt,
     return hip_status(err);
   }
   int rc = sparse_gate_up(e, hidden, inter, group, sdt, x, cai4::A_XF32, n_tokens, gate, upv,
-                          thr, false, slots, &n_slots, part_gemm, workspace == nullptr, st);
+                          thr, false, slots, &n_slots, part_gemm, false, st);
   if (rc) return rc;
   cai4::SparseMaskArgs m{};
   m.gate = gate;
@@ -1017,23 +1103,31 @@ void expert_blob_sections(uint32_t hidden, uint32_t inter, uint32_t group, uint3
 }
 
 // Prefill GEMM (many tokens, MFMA-tiled weights): bf16 x, or f32 x as two planes.
+// workspace: the caller's (gemm_workspace bytes), or null for the library's;
+// recorded: see Workspace::get (no more than this call's own).
 int run_prefill(const cascadia_int4_layout *L, const uint8_t *packed, const uint8_t *scales,
-                const void *x, bool x_f32, uint32_t M, void *y, bool out_f32, hipStream_t st) {
+                const void *x, bool x_f32, uint32_t M, void *y, bool out_f32, void *workspace,
+                size_t recorded, hipStream_t st) {
   int dev;
   if (int rc = current_device(&dev)) return rc;
   if ((size_t)M * L->k_cols * 2 >= 0x7FFFFFFFu) return CASCADIA_INT4_ERR_ARG;
   const int cus = device_props(dev).num_cus;
   const int amode = x_f32 ? cai4::GG_A_F32 : cai4::GG_A_BF16;
   const int epi = out_f32 ? cai4::GG_F32 : cai4::GG_BF16;
-  void *ws = nullptr;
+  Workspace own;
+  void *ws = workspace;
   int slices = 8;
   auto bytes = [&] {
     return cai4::gg_dense_workspace((int)M, (int)L->n_rows, (int)L->k_cols, (int)L->group_size,
                                     amode, epi, cus, false, slices);
   };
-  if (lib_workspace(dev, bytes(), &ws, st)) {
+  auto get = [&] {
+    const size_t b = bytes();
+    return own.get(dev, b, st, &ws, recorded < b ? recorded : b);
+  };
+  if (!ws && get()) {
     slices = 1;  // a workspace that cannot grow now: no partials
-    if (int rc = lib_workspace(dev, bytes(), &ws, st)) return rc;
+    if (int rc = get()) return rc;
   }
   cai4::GgArgs a{};
   a.w0 = packed;
@@ -1066,6 +1160,57 @@ bool prefill_shape(const cascadia_int4_layout *L, uint32_t seq, bool x_f32) {
   const size_t bytes = (size_t)L->n_rows * L->k_cols / 2;
   if (x_f32) return tiles_pay(seq, 32, bytes, 17, (size_t)22 << 20);
   return seq >= 64 || tiles_pay(seq, 64, bytes, 33, (size_t)22 << 20);
+}
+
+// seq rows through the tile GEMM, the skinny kernel or the GEMV.  Without a
+// workspace, rows that the skinny kernel would take in no shared memory (f32, or
+// fewer than 64 of bf16) take the tiles only where the library's buffer is this
+// stream's alone: a recorded call runs beside others later.
+int gemm_common(const cascadia_int4_layout *L, const uint8_t *packed, const uint8_t *scales,
+                const void *x, bool x_f32, uint32_t seq, void *y, bool y_f32, void *workspace,
+                hipStream_t st) {
+  if (int rc = check_layout(L)) return rc;
+  if (int rc = check_weights(packed, scales)) return rc;
+  if (!x || !y) return CASCADIA_INT4_ERR_NULL;
+  if (seq == 0) return CASCADIA_INT4_ERR_ARG;  // the crate asserts seq >= 1
+  if (!aligned(x, 16) || !aligned(y, y_f32 ? 4 : 2) || (workspace && !aligned(workspace, 16)))
+    return CASCADIA_INT4_ERR_ARG;
+  const int amode = x_f32 ? cai4::A_XF32 : cai4::A_BF16;
+  const bool tiles_only = !x_f32 && seq >= 64;
+  if (prefill_shape(L, seq, x_f32) && (tiles_only || act_fits((int)seq, (int)L->k_cols, amode)) &&
+      (tiles_only || workspace || !capturing(st))) {
+    size_t recorded = ~(size_t)0;
+    if (!tiles_only && !workspace) {  // recorded, it is the skinny kernel's
+      int dev;
+      if (int rc = current_device(&dev)) return rc;
+      recorded = cai4::skinny_plan((int)L->n_rows, (int)L->k_cols, (int)L->group_size, (int)seq,
+                                   amode, cai4::EPI_F32, device_props(dev))
+                     .partial_bytes;
+    }
+    const int rc = run_prefill(L, packed, scales, x, x_f32, seq, y, y_f32, workspace, recorded, st);
+    if (tiles_only || !fall_back(rc)) return rc;
+  }
+  return run_gemm(packed, scales, nullptr, nullptr, (int)L->n_rows, (int)L->k_cols,
+                  (int)L->group_size, (int)L->scale_dtype, (int)L->tiling, x, nullptr, amode,
+                  (int)seq, y, nullptr, y_f32 ? cai4::EPI_F32 : cai4::EPI_BF16, st, workspace,
+                  workspace == nullptr);
+}
+
+// Its workspace, for every count of rows n_plan .. seq (as ffn_workspace's).
+size_t gemm_workspace(int dev, const cascadia_int4_layout *L, bool x_f32, uint32_t seq,
+                      uint32_t n_plan) {
+  const cai4::SkinnyDevice d = device_props(dev);
+  const int N = (int)L->n_rows, K = (int)L->k_cols, G = (int)L->group_size;
+  size_t b = cai4::skinny_plan(N, K, G, (int)n_plan, x_f32 ? cai4::A_XF32 : cai4::A_BF16,
+                               cai4::EPI_F32, d)
+                 .partial_bytes;
+  if (prefill_shape(L, seq, x_f32)) {
+    const size_t t =
+        cai4::gg_dense_workspace((int)n_plan, N, K, G, x_f32 ? cai4::GG_A_F32 : cai4::GG_A_BF16,
+                                 cai4::GG_F32, d.num_cus, false, 8, (int)seq);
+    b = t > b ? t : b;
+  }
+  return b;
 }
 
 // ov_gemv's: the activations as f32, the output as f32, the GEMVs' partials; for
@@ -1234,13 +1379,14 @@ int moe_forward(const cascadia_int4_moe_layer *L, const cascadia_int4_routing *R
   if (int rc = current_device(&dev)) return rc;
   const bool given = R->mode == CASCADIA_INT4_ROUTE_IDS;
   MoePlan m = moe_plan(dev, L, R->top_k, T, given);
+  Workspace own;
   void *ws = workspace;
   if (!ws) {
     // a library workspace that cannot grow now (a capture, no memory) may still
     // hold what the layer needs at least
-    if (lib_workspace(dev, m.ws.total, &ws, st)) {
+    if (own.get(dev, m.ws.total, st, &ws)) {
       m = moe_plan(dev, L, R->top_k, T, given, true);
-      if (int rc = lib_workspace(dev, m.ws.total, &ws, st)) return rc;
+      if (int rc = own.get(dev, m.ws.total, st, &ws)) return rc;
     }
   } else if (!aligned(ws, 256)) {
     return CASCADIA_INT4_ERR_ARG;
@@ -1336,7 +1482,8 @@ int moe_forward(const cascadia_int4_moe_layer *L, const cascadia_int4_routing *R
         return run_gemm(L->shared.gate_packed, L->shared.gate_scale, L->shared.up_packed,
                         L->shared.up_scale, I, H, (int)L->group_size, (int)L->scale_dtype,
                         (int)L->shared.tiling, x, nullptr, cai4::A_XF32, 1,
-                        hi + (size_t)k * I, lo + (size_t)k * I, cai4::EPI_SWIGLU_HILO, on);
+                        hi + (size_t)k * I, lo + (size_t)k * I, cai4::EPI_SWIGLU_HILO, on,
+                        nullptr, false);
       return ffn_common(L->hidden, L->shared_inter, L->group_size, L->scale_dtype, &L->shared,
                         x, true, T, sh, false, W + m.ws.shared_ws, on, m.shared_bytes);
     };
@@ -1681,59 +1828,39 @@ int cascadia_int4_bf16_to_f32(const uint16_t *x_bf16, size_t n, float *out, void
 int cascadia_int4_dequant_gemm_multi(const cascadia_int4_layout *L, const uint8_t *packed,
                                      const uint8_t *scale_bits, const float *xs, uint32_t seq,
                                      float *ys, void *stream) {
-  if (int rc = check_layout(L)) return rc;
-  if (int rc = check_weights(packed, scale_bits)) return rc;
-  if (!xs || !ys) return CASCADIA_INT4_ERR_NULL;
-  if (seq == 0) return CASCADIA_INT4_ERR_ARG;  // the crate asserts seq >= 1
-  if (!aligned(xs, 16) || !aligned(ys, 4)) return CASCADIA_INT4_ERR_ARG;
-  // many tokens over tiled weights: two planes through the tile GEMM, unless
-  // the library's workspace cannot grow to hold them (then, as for fewer
-  // tokens, the skinny kernel's passes)
-  if (prefill_shape(L, seq, true) && act_fits((int)seq, (int)L->k_cols, cai4::A_XF32)) {
-    const int rc = run_prefill(L, packed, scale_bits, xs, true, seq, ys, true, (hipStream_t)stream);
-    if (!fall_back(rc)) return rc;
-  }
-  return run_gemm(packed, scale_bits, nullptr, nullptr, (int)L->n_rows, (int)L->k_cols,
-                  (int)L->group_size, (int)L->scale_dtype, (int)L->tiling, xs, nullptr, cai4::A_XF32, (int)seq,
-                  ys, nullptr, cai4::EPI_F32, (hipStream_t)stream);
+  return gemm_common(L, packed, scale_bits, xs, true, seq, ys, true, nullptr, (hipStream_t)stream);
 }
 
 int cascadia_int4_dequant_gemm_bf16in(const cascadia_int4_layout *L, const uint8_t *packed,
                                       const uint8_t *scale_bits, const uint16_t *xs_bf16,
                                       uint32_t seq, float *ys, void *stream) {
-  if (int rc = check_layout(L)) return rc;
-  if (int rc = check_weights(packed, scale_bits)) return rc;
-  if (!xs_bf16 || !ys) return CASCADIA_INT4_ERR_NULL;
-  if (seq == 0) return CASCADIA_INT4_ERR_ARG;
-  if (!aligned(xs_bf16, 16) || !aligned(ys, 4)) return CASCADIA_INT4_ERR_ARG;
-  if (prefill_shape(L, seq, false)) {
-    const int rc =
-        run_prefill(L, packed, scale_bits, xs_bf16, false, seq, ys, true, (hipStream_t)stream);
-    if (seq >= 64 || !fall_back(rc)) return rc;
-  }
-  return run_gemm(packed, scale_bits, nullptr, nullptr, (int)L->n_rows, (int)L->k_cols,
-                  (int)L->group_size, (int)L->scale_dtype, (int)L->tiling, xs_bf16, nullptr,
-                  cai4::A_BF16,
-                  (int)seq, ys, nullptr, cai4::EPI_F32, (hipStream_t)stream);
+  return gemm_common(L, packed, scale_bits, xs_bf16, false, seq, ys, true, nullptr,
+                     (hipStream_t)stream);
 }
 
 int cascadia_int4_gemm_bf16(const cascadia_int4_layout *L, const uint8_t *packed,
                             const uint8_t *scale_bits, const uint16_t *xs_bf16, uint32_t seq,
                             uint16_t *ys_bf16, void *stream) {
-  if (int rc = check_layout(L)) return rc;
-  if (int rc = check_weights(packed, scale_bits)) return rc;
-  if (!xs_bf16 || !ys_bf16) return CASCADIA_INT4_ERR_NULL;
-  if (seq == 0) return CASCADIA_INT4_ERR_ARG;
-  if (!aligned(xs_bf16, 16) || !aligned(ys_bf16, 2)) return CASCADIA_INT4_ERR_ARG;
-  if (prefill_shape(L, seq, false)) {
-    const int rc = run_prefill(L, packed, scale_bits, xs_bf16, false, seq, ys_bf16, false,
-                               (hipStream_t)stream);
-    if (seq >= 64 || !fall_back(rc)) return rc;
-  }
-  return run_gemm(packed, scale_bits, nullptr, nullptr, (int)L->n_rows, (int)L->k_cols,
-                  (int)L->group_size, (int)L->scale_dtype, (int)L->tiling, xs_bf16, nullptr,
-                  cai4::A_BF16,
-                  (int)seq, ys_bf16, nullptr, cai4::EPI_BF16, (hipStream_t)stream);
+  return gemm_common(L, packed, scale_bits, xs_bf16, false, seq, ys_bf16, false, nullptr,
+                     (hipStream_t)stream);
+}
+
+size_t cascadia_int4_gemm_workspace_bytes(const cascadia_int4_layout *L, uint32_t x_is_f32,
+                                          uint32_t seq) {
+  int dev;
+  if (check_layout(L) || current_device(&dev)) return 0;
+  return rows_upto(seq, 0x7FFFFFFFu / ((x_is_f32 ? 4 : 2) * (size_t)L->k_cols),
+                   [&](uint32_t lo, uint32_t hi) {
+                     return gemm_workspace(dev, L, x_is_f32 != 0, hi, lo);
+                   });
+}
+
+int cascadia_int4_gemm(const cascadia_int4_layout *L, const uint8_t *packed,
+                       const uint8_t *scale_bits, const void *xs, uint32_t x_is_f32, uint32_t seq,
+                       void *ys, uint32_t y_is_f32, void *workspace, void *stream) {
+  if (x_is_f32 && !y_is_f32) return CASCADIA_INT4_ERR_ARG;
+  return gemm_common(L, packed, scale_bits, xs, x_is_f32 != 0, seq, ys, y_is_f32 != 0, workspace,
+                     (hipStream_t)stream);
 }
 
 size_t cascadia_int4_expert_bytes(uint32_t hidden, uint32_t inter, uint32_t group_size) {
@@ -1895,11 +2022,12 @@ int cascadia_int4_dequant_axpy_active(const uint8_t *packed_t, const uint8_t *sc
     return CASCADIA_INT4_ERR_ARG;
   if (n_active == 0) return CASCADIA_INT4_OK;
   const cai4::AxpyPlan p = cai4::axpy_plan((int)hidden, (int)n_active);
+  Workspace own;
   void *ws = workspace;
   if (!ws) {
     int dev;
     if (int rc = current_device(&dev)) return rc;
-    if (int rc = lib_workspace(dev, p.partial_bytes, &ws, (hipStream_t)stream)) return rc;
+    if (int rc = own.get(dev, p.partial_bytes, (hipStream_t)stream, &ws)) return rc;
   }
   return hip_status(cai4::axpy_active(packed_t, scale_t_bits, scalars, active, (int)n_active,
                                       (int)hidden, (int)inter, static_cast<float *>(ws), y,
@@ -1981,9 +2109,10 @@ int cascadia_int4_ov_gemv(const cascadia_int4_ov_segment *segs, uint32_t n_segs,
   if (int rc = current_device(&dev)) return rc;
   hipStream_t st = (hipStream_t)stream;
   const size_t need = ov_workspace(dev, segs, n_segs, k_cols, group_size, rows, rows);
+  Workspace own;
   void *ws = workspace;
   if (!ws) {
-    if (int rc = lib_workspace(dev, need, &ws, st)) return rc;
+    if (int rc = own.get(dev, need, st, &ws)) return rc;
   }
   uint8_t *b = static_cast<uint8_t *>(ws);
   const size_t act_b = align256((size_t)rows * k_cols * 4);

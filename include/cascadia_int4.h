@@ -24,18 +24,25 @@
  *     the seq-major GEMMs (seq >= 1, kernel_avx512_multi.rs:80) and
  *     cascadia_int4_moe_forward return CASCADIA_INT4_ERR_ARG for zero rows.
  *   - Outputs are fully overwritten, as in the crate.  Calls are reentrant
- *     for distinct output buffers; a shared workspace (workspace == NULL, the
- *     library's own) makes concurrent calls on different streams race.
- *   - HIP graph capture: the library's own workspace grows by an allocation,
- *     which a capture cannot record; a call on a capturing stream that would
- *     grow it returns CASCADIA_INT4_ERR_ARG.  Callers that capture pass a
- *     workspace of the matching *_workspace_bytes size, or use
- *     cascadia_int4_expert_forward_noalloc, or warm the library's workspace
- *     with an eager call of the same shape first.  A growth never frees the
- *     buffer it replaces (the library keeps it until the process ends), so a
- *     graph captured on the smaller buffer stays valid after a later, larger
- *     eager call; it still shares that buffer with any eager call, so replays
- *     and eager calls that use the library's workspace must not overlap.
+ *     for distinct output buffers, from any thread and on any streams: a call
+ *     without a workspace (workspace == NULL, or no such argument) uses the
+ *     library's buffer of its stream, one for each of the first 16 streams of
+ *     a device; further streams, and hipStreamPerThread, share one, whose uses
+ *     run one after another.  A stream that is destroyed must have finished
+ *     its calls.  A caller's workspace serves one call at a time.
+ *   - HIP graph capture: callers that capture pass a workspace of the matching
+ *     *_workspace_bytes size (the GEMMs: cascadia_int4_gemm), or use
+ *     cascadia_int4_expert_forward_noalloc.  Without one a recorded call uses
+ *     the library's buffer for graphs, apart from the eager calls' but one for
+ *     all graphs of a device: graphs that use it must not run at the same time.
+ *     It grows by an allocation, which a capture cannot record, so it is grown
+ *     by eager calls: a call on a capturing stream that does not fit takes a
+ *     form that needs less or returns CASCADIA_INT4_ERR_ARG; an eager call of
+ *     the same shape first makes it fit.  A growth never frees the memory it
+ *     replaces (kept until the process ends): a graph recorded on it stays
+ *     valid.  f32 rows, and fewer than 64 of bf16, of a GEMM without a
+ *     workspace are recorded in a form that shares no memory but the partials
+ *     of a split K, slower than the eager form from 17 rows on.
  */
 #ifndef CASCADIA_INT4_H
 #define CASCADIA_INT4_H
@@ -184,6 +191,17 @@ int cascadia_int4_gemm_bf16(const cascadia_int4_layout *layout, const uint8_t *p
                             const uint8_t *scale_bits, const uint16_t *xs_bf16, uint32_t seq,
                             uint16_t *ys_bf16, void *stream);
 
+/* The three GEMMs above with a caller's workspace (16-byte aligned, of at least
+ * cascadia_int4_gemm_workspace_bytes for seq rows or more; NULL: as above), for
+ * callers that capture: xs f32 (x_is_f32 1) or bf16 bits, ys f32 (y_is_f32 1)
+ * or, for bf16 xs, bf16 bits.  The same kernels and results as the eager calls
+ * above.  The size is 0 on bad arguments and where no workspace is needed. */
+size_t cascadia_int4_gemm_workspace_bytes(const cascadia_int4_layout *layout, uint32_t x_is_f32,
+                                          uint32_t seq);
+int cascadia_int4_gemm(const cascadia_int4_layout *layout, const uint8_t *packed,
+                       const uint8_t *scale_bits, const void *xs, uint32_t x_is_f32, uint32_t seq,
+                       void *ys, uint32_t y_is_f32, void *workspace, void *stream);
+
 /* One expert's six weight slices (device pointers), as expert_forward takes
  * them (src/kernel.rs:75-84): gate/up are [inter, hidden], down is
  * [hidden, inter], each packed u8 + scale u16 in the layout above.  Packed
@@ -231,7 +249,7 @@ size_t cascadia_int4_ffn_workspace_bytes(uint32_t hidden, uint32_t inter, uint32
  * rounding of the output (src/kernel.rs:75-136; ffn_sparsity.rs:756 at
  * tau = 0).  x_bf16, out_bf16: [n_tokens, hidden] bf16 bits.  workspace:
  * >= cascadia_int4_ffn_workspace_bytes bytes, 16-byte aligned, or NULL to use
- * the library's per-device buffer.  Named _device because the crate's C FFI
+ * the library's buffer.  Named _device because the crate's C FFI
  * already exports cascadia_int4_expert_forward for its safetensors-handle
  * call (c_ffi.rs:308-341, f32 in/out); that name stays reserved for it. */
 int cascadia_int4_expert_forward_device(uint32_t hidden, uint32_t inter, uint32_t group_size,

@@ -55,7 +55,7 @@ struct Options {
   Tiling tiling = Tiling::Crate;
   hipStream_t stream = nullptr;
   bool synchronize = true;     // the crate's calls return with the result written
-  void *workspace = nullptr;   // null: the library's per-device buffer
+  void *workspace = nullptr;   // null: the library's buffer
 };
 
 // A HIP or device-memory failure (the C ABI's -3 / -4).

@@ -10,7 +10,13 @@ tokens, and MoE layers at
 the shared expert forks onto the library's side stream) are enqueued on two
 streams, alternating, with no synchronisation between them, and every output
 is compared with the serial result.
+
+Calls without a workspace use the library's buffer of their stream: multi-row
+GEMMs and FFNs on two streams, on more streams than have a buffer of their own,
+from two threads on one stream, and beside the replays of a graph.
 """
+import threading
+
 import numpy as np
 import pytest
 import torch
@@ -100,3 +106,135 @@ def test_two_streams_equal_serial(cl, orc):
         for j, (_, outs) in enumerate(jobs):
             for t, w in zip(outs, want[j]):
                 assert torch.equal(t, w), f"{name}, job {j}: differs from the serial call"
+
+
+def gemm_jobs(cl, rows=(17, 100, 333), n=3072, k=4096, g=32):
+    """Calls without a workspace that need one: f32 and bf16 rows through the
+    tile GEMM, and an FFN; each (call, output)."""
+    packed = cl.fill_bytes(torch.empty(n * k // 2, dtype=torch.uint8, device="cuda"), 21, 1)
+    scales = cl.fill_scales(torch.empty(n * (k // g), dtype=torch.int16, device="cuda"), 21, 2)
+    pt, st = cl.tile_weights(packed, scales.view(torch.uint8), n, k, g)
+    opts = dict(group_size=g, scale_dtype=F16, tiling=cl.TILING_MFMA)
+    jobs = []
+    for M in rows:
+        for dt in (torch.float32, torch.bfloat16):
+            x = cl.fill_normal(torch.empty((M, k), dtype=dt, device="cuda"), 22, M)
+            y = torch.empty((M, n), dtype=torch.float32, device="cuda")
+            jobs.append((lambda x=x, y=y, M=M: cl.dequant_gemm_int4_multi_auto(
+                pt, st, x, n, k, M, y, **opts), y))
+    h, i, hg = 1024, 3072, 128
+    flat = cl.fill_bytes(torch.empty(cl.expert_bytes(h, i, hg), dtype=torch.uint8, device="cuda"),
+                         23, 1)
+    W = cl.ExpertWeights(flat, h, i, hg, F16)
+    for s in W.slices()[1::2]:
+        cl.fill_scales(s.view(torch.int16), 23, 2)
+    W = W.tiled()
+    x = cl.fill_normal(torch.empty((200, h), dtype=torch.bfloat16, device="cuda"), 24, 1)
+    out = torch.empty_like(x)
+    jobs.append((lambda: cl.expert_forward(x, *W.slices(), out, group_size=hg, scale_dtype=F16,
+                                           tiling=cl.TILING_MFMA), out))
+    return jobs
+
+
+def serial_results(jobs):
+    want = []
+    for fn, out in jobs:
+        fn()
+        torch.cuda.synchronize()
+        want.append(out.clone())
+        out.zero_()
+    torch.cuda.synchronize()
+    return want
+
+
+@pytest.mark.parametrize("n_streams", [2, 20])
+def test_library_workspace_on_streams(cl, n_streams):
+    """(20: more streams than the library keeps a buffer for)"""
+    print(f"{n_streams} streams without workspaces", flush=True)
+    sets = [gemm_jobs(cl, rows=(333,) if n_streams > 2 else (17, 100, 333))
+            for _ in range(n_streams)]
+    want = serial_results(sets[0])
+    streams = [torch.cuda.Stream() for _ in range(n_streams)]
+    torch.cuda.synchronize()
+    for rep in range(4):
+        for j in range(len(want)):
+            for s, jobs in zip(streams, sets):
+                with torch.cuda.stream(s):
+                    jobs[(j + rep) % len(jobs)][0]()
+    torch.cuda.synchronize()
+    for c, jobs in enumerate(sets):
+        for j, (_, out) in enumerate(jobs):
+            assert torch.equal(out, want[j]), f"stream {c}, job {j}: differs from the serial call"
+
+
+@pytest.mark.parametrize("one_stream", [True, False])
+def test_library_workspace_from_two_threads(cl, one_stream):
+    print(f"two threads, one stream: {one_stream}", flush=True)
+    sets = [gemm_jobs(cl), gemm_jobs(cl)]
+    want = serial_results(sets[0])
+    shared = torch.cuda.Stream()
+    streams = [shared, shared if one_stream else torch.cuda.Stream()]
+    errors = []
+
+    def work(jobs, stream):
+        try:
+            with torch.cuda.stream(stream):
+                for _ in range(6):
+                    for fn, _ in jobs:
+                        fn()
+        except Exception as e:  # noqa: BLE001 -- reported below
+            errors.append(e)
+
+    threads = [threading.Thread(target=work, args=a) for a in zip(sets, streams)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    torch.cuda.synchronize()
+    assert not errors, errors
+    for c, jobs in enumerate(sets):
+        for j, (_, out) in enumerate(jobs):
+            assert torch.equal(out, want[j]), f"thread {c}, job {j}: differs from the serial call"
+
+
+@pytest.mark.parametrize("own_workspace", [True, False])
+def test_graph_replays_beside_eager_calls(cl, own_workspace):
+    """A recorded f32 GEMM replayed while eager ones run on another stream; with a
+    workspace of its own it is the eager form, bit for bit."""
+    n, k, g, M = 3072, 4096, 32, 333
+    packed = cl.fill_bytes(torch.empty(n * k // 2, dtype=torch.uint8, device="cuda"), 31, 1)
+    scales = cl.fill_scales(torch.empty(n * (k // g), dtype=torch.int16, device="cuda"), 31, 2)
+    pt, st = cl.tile_weights(packed, scales.view(torch.uint8), n, k, g)
+    opts = dict(group_size=g, scale_dtype=F16, tiling=cl.TILING_MFMA)
+    xs = [cl.fill_normal(torch.empty((M, k), device="cuda"), 32, j) for j in range(2)]
+    ys = [torch.empty((M, n), device="cuda") for _ in range(2)]
+    call = lambda j, **kw: cl.dequant_gemm_int4_multi_auto(  # noqa: E731
+        pt, st, xs[j], n, k, M, ys[j], **opts, **kw)
+    want = serial_results([(lambda: call(0), ys[0]), (lambda: call(1), ys[1])])
+    kw = {}
+    if own_workspace:
+        kw["workspace"] = torch.empty(cl.gemm_workspace_bytes(n, k, M, True, g, cl.TILING_MFMA),
+                                      dtype=torch.uint8, device="cuda")
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        call(0, **kw)
+    graph.replay()
+    torch.cuda.synchronize()
+    recorded = ys[0].clone()
+    if own_workspace:
+        assert torch.equal(recorded, want[0])
+    else:  # the form that shares no memory: another order of the same sums
+        assert float((recorded - want[0]).norm() / want[0].norm()) <= 1e-5
+    sa, sb = torch.cuda.Stream(), torch.cuda.Stream()
+    torch.cuda.synchronize()
+    for rep in range(8):
+        ys[0].zero_(), ys[1].zero_()
+        torch.cuda.synchronize()
+        with torch.cuda.stream(sa):
+            graph.replay()
+        with torch.cuda.stream(sb):
+            call(1)
+            call(1)
+        torch.cuda.synchronize()
+        assert torch.equal(ys[0], recorded), f"replay {rep}"
+        assert torch.equal(ys[1], want[1]), f"eager call beside replay {rep}"
