@@ -243,6 +243,11 @@ class Workspace {
 
 inline bool aligned(const void *p, size_t a) { return ((uintptr_t)p % a) == 0; }
 
+// Whether the kernels that load scales straight into LDS, four bytes a lane
+// (grouped.hip, few.hip), take these: callers may align scales to two bytes
+// only, which the others' loads into registers allow for.
+bool lds_loads_ok(const uint8_t *scales) { return aligned(scales, 4); }
+
 int check_layout(const cascadia_int4_layout *L) {
   if (!L) return CASCADIA_INT4_ERR_NULL;
   if (L->n_rows == 0 || L->k_cols == 0 || L->group_size == 0) return CASCADIA_INT4_ERR_ARG;
@@ -664,10 +669,12 @@ int ffn_common(uint32_t hidden, uint32_t inter, uint32_t group, uint32_t sdt,
   } else if (!aligned(ws, 16)) {
     return CASCADIA_INT4_ERR_ARG;
   }
-  if (!lean && need.few && e->tiling == CASCADIA_INT4_TILING_MFMA)
+  const bool lds_loads =
+      lds_loads_ok(e->gate_scale) && lds_loads_ok(e->up_scale) && lds_loads_ok(e->down_scale);
+  if (!lean && need.few && lds_loads && e->tiling == CASCADIA_INT4_TILING_MFMA)
     return ffn_few(hidden, inter, group, sdt, e, x, n_tokens, out, out_bf16, ws,
                    device_props(dev).num_cus, st);
-  if ((lean ? need.lean : need.tile) && e->tiling == CASCADIA_INT4_TILING_MFMA)
+  if ((lean ? need.lean : need.tile) && lds_loads && e->tiling == CASCADIA_INT4_TILING_MFMA)
     return ffn_tiles(hidden, inter, group, sdt, e, x, x_f32, n_tokens, out, out_bf16, ws, lean,
                      device_props(dev).num_cus, st);
   // the SwiGLU intermediate as two bf16 planes (hi, lo): [n_tokens, inter] each
@@ -1176,8 +1183,9 @@ int gemm_common(const cascadia_int4_layout *L, const uint8_t *packed, const uint
   if (!aligned(x, 16) || !aligned(y, y_f32 ? 4 : 2) || (workspace && !aligned(workspace, 16)))
     return CASCADIA_INT4_ERR_ARG;
   const int amode = x_f32 ? cai4::A_XF32 : cai4::A_BF16;
-  const bool tiles_only = !x_f32 && seq >= 64;
-  if (prefill_shape(L, seq, x_f32) && (tiles_only || act_fits((int)seq, (int)L->k_cols, amode)) &&
+  const bool tiles = prefill_shape(L, seq, x_f32) && lds_loads_ok(scales);
+  const bool tiles_only = tiles && !x_f32 && seq >= 64;
+  if (tiles && (tiles_only || act_fits((int)seq, (int)L->k_cols, amode)) &&
       (tiles_only || workspace || !capturing(st))) {
     size_t recorded = ~(size_t)0;
     if (!tiles_only && !workspace) {  // recorded, it is the skinny kernel's

@@ -136,6 +136,46 @@ def test_gemm_f32_tiles_lose_no_precision(cl, tuning, g, mean):
     assert err["tiles"] <= err["skinny"], err
 
 
+def shifted(t):
+    """The same bytes two past a 16-byte boundary."""
+    s = torch.empty(t.numel() + 16, dtype=torch.uint8, device="cuda")[2:2 + t.numel()]
+    return s.copy_(t)
+
+
+@pytest.mark.parametrize("g", [32, 128])
+def test_scales_aligned_to_two_bytes(cl, tuning, g):
+    """Scales need two bytes' alignment only; the kernels that load them into LDS
+    four bytes at a time leave such calls to the skinny kernel."""
+    n, k, M = 1024, 2048, 100
+    packed = cl.fill_bytes(torch.empty(n * k // 2, dtype=torch.uint8, device="cuda"), 12, 1)
+    scales = cl.fill_scales(torch.empty(n * (k // g), dtype=torch.int16, device="cuda"), 12, 2, F16)
+    pt, st = cl.tile_weights(packed, scales.view(torch.uint8), n, k, g)
+    x = cl.fill_normal(torch.empty((M, k), dtype=torch.float32, device="cuda"), 12, 3)
+    opts = dict(group_size=g, scale_dtype=F16, tiling=cl.TILING_MFMA)
+    ys = [torch.empty((M, n), device="cuda") for _ in range(2)]
+    tuning("CASCADIA_INT4_F32_TILE_TOKENS", "17")
+    cl.dequant_gemm_int4_multi_auto(pt, shifted(st), x, n, k, M, ys[0], **opts)
+    tuning("CASCADIA_INT4_F32_TILE_TOKENS", "100000")
+    cl.dequant_gemm_int4_multi_auto(pt, st, x, n, k, M, ys[1], **opts)
+    assert torch.equal(ys[0], ys[1])
+    h, i = 1024, 512
+    flat = cl.fill_bytes(torch.empty(cl.expert_bytes(h, i, g), dtype=torch.uint8, device="cuda"),
+                         13, 1)
+    W = cl.ExpertWeights(flat, h, i, g, F16)
+    for t in W.slices()[1::2]:
+        cl.fill_scales(t.view(torch.int16), 13, 2)
+    W = W.tiled()
+    xb = x[:, :h].to(torch.bfloat16).contiguous()
+    for m, var in ((16, "CASCADIA_INT4_FEW_MIN_TOKENS"), (100, "CASCADIA_INT4_FFN_TILE_TOKENS")):
+        outs = [torch.empty((m, h), dtype=torch.bfloat16, device="cuda") for _ in range(2)]
+        tuning(var, "2")
+        cl.expert_forward(xb[:m], *[shifted(t) if j % 2 else t for j, t in enumerate(W.slices())],
+                          outs[0], **opts)
+        tuning(var, "100000")
+        cl.expert_forward(xb[:m], *W.slices(), outs[1], **opts)
+        assert torch.equal(outs[0], outs[1]), f"{m} rows"
+
+
 def test_gemm_f32_capture(cl, orc):
     """A stream capture cannot grow the library's workspace: the f32 GEMM of a
     shape not seen before is recorded all the same (without the tile route if
