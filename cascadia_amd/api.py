@@ -14,6 +14,7 @@ from __future__ import annotations
 
 import ctypes as C
 import functools
+from operator import index as _index
 
 import numpy as np
 import torch
@@ -83,7 +84,7 @@ def _is_bf16_bits(t: torch.Tensor) -> bool:
     return t.dtype in (torch.bfloat16, torch.int16, torch.uint16)
 
 
-@functools.lru_cache(maxsize=1024, typed=True)
+@functools.lru_cache(maxsize=1024)
 def _layout_of(n_rows, k_cols, group_size, scale_dtype, tiling):
     L = Layout(n_rows, k_cols, group_size, scale_dtype, tiling)
     return L, C.byref(L)  # (the struct is kept with its reference)
@@ -91,8 +92,10 @@ def _layout_of(n_rows, k_cols, group_size, scale_dtype, tiling):
 
 def _layout(n_rows, k_cols, group_size, scale_dtype, tiling=TILING_CRATE):
     """A reference to the layout struct of these values, made once per set of
-    values (the library only reads it)."""
-    return _layout_of(n_rows, k_cols, group_size, scale_dtype, tiling)[1]
+    values (the library only reads it): the values themselves, whatever integer
+    type carries them (an array or tensor hashes by identity, or not at all)."""
+    return _layout_of(_index(n_rows), _index(k_cols), _index(group_size), _index(scale_dtype),
+                      _index(tiling))[1]
 
 
 def tiled_sizes(n_rows, k_cols, group_size=GROUP_SIZE):

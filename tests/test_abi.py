@@ -41,6 +41,24 @@ def test_version(cl):
     assert b"gfx950" in cl.lib().cascadia_int4_version()
 
 
+def test_layout_struct_follows_the_values(cl):
+    """Sizes may come as any integer type, an array or tensor of one element
+    among them; the cached struct is of the values at the call."""
+    import numpy as np
+    import torch
+
+    from cascadia_amd import api
+
+    t = torch.tensor(4096)
+    for n in (4096, np.int64(4096), np.array(4096), t):
+        L = api._layout(n, np.array(512), 128, cl.SCALE_F16, True)._obj
+        assert (L.n_rows, L.k_cols, L.group_size, L.scale_dtype, L.tiling) == (4096, 512, 128, 1, 1)
+    t += 16
+    assert api._layout(t, 512, 128, cl.SCALE_F16)._obj.n_rows == 4112
+    with pytest.raises(TypeError):
+        api._layout(4096.0, 512, 128, 0)
+
+
 def test_expert_bytes_matches_oracle(cl, orc):
     for h, i, g in [(7168, 2048, 32), (3072, 1536, 128), (4096, 14336, 128), (64, 32, 32)]:
         assert cl.expert_bytes(h, i, g) == orc.expert_bytes(h, i, g)
