@@ -545,7 +545,6 @@ int ffn_tiles(uint32_t hidden, uint32_t inter, uint32_t group, uint32_t sdt,
   g.ldy = (int)inter;
   g.epi = cai4::GG_SWIGLU_HILO;
   g.seeds_out = seeds;
-  g.seeds_gw = cai4::gg_group_width((int)group);
   g.seeds_rp = cai4::gg_rows_pad((int)n_tokens);
   if (hipError_t err =
           cai4::gg_dense(g, x_f32 ? cai4::GG_A_F32 : cai4::GG_A_BF16, b, num_cus, st, slices))
@@ -568,11 +567,11 @@ int ffn_tiles(uint32_t hidden, uint32_t inter, uint32_t group, uint32_t sdt,
   return hip_status(cai4::gg_dense(dn, cai4::GG_A_PLANES, b, num_cus, st, slices));
 }
 
-// The expert FFN of a few bf16 rows: gate/up with the SwiGLU epilogue into
+// The expert FFN of a few bf16 rows (their output is bf16): gate/up with the SwiGLU epilogue into
 // hi / lo planes, then down over them (few.hip).
 int ffn_few(uint32_t hidden, uint32_t inter, uint32_t group, uint32_t sdt,
-            const cascadia_int4_expert *e, const void *x, uint32_t n_tokens, void *out,
-            bool out_bf16, void *ws, int num_cus, hipStream_t st) {
+            const cascadia_int4_expert *e, const void *x, uint32_t n_tokens, void *out, void *ws,
+            int num_cus, hipStream_t st) {
   const size_t plane = ffn_plane_bytes(inter, n_tokens);
   uint8_t *b = static_cast<uint8_t *>(ws);
   uint16_t *hi = reinterpret_cast<uint16_t *>(b);
@@ -607,7 +606,7 @@ int ffn_few(uint32_t hidden, uint32_t inter, uint32_t group, uint32_t sdt,
   dn.G = (int)group;
   dn.sdt = (int)sdt;
   dn.ldy = (int)hidden;
-  dn.epi = out_bf16 ? cai4::GG_BF16 : cai4::GG_F32;
+  dn.epi = cai4::GG_BF16;
   return hip_status(cai4::few_gemm(dn, b, num_cus, st));
 }
 
@@ -671,8 +670,8 @@ int ffn_common(uint32_t hidden, uint32_t inter, uint32_t group, uint32_t sdt,
   }
   const bool lds_loads =
       lds_loads_ok(e->gate_scale) && lds_loads_ok(e->up_scale) && lds_loads_ok(e->down_scale);
-  if (!lean && need.few && lds_loads && e->tiling == CASCADIA_INT4_TILING_MFMA)
-    return ffn_few(hidden, inter, group, sdt, e, x, n_tokens, out, out_bf16, ws,
+  if (!lean && need.few && out_bf16 && lds_loads && e->tiling == CASCADIA_INT4_TILING_MFMA)
+    return ffn_few(hidden, inter, group, sdt, e, x, n_tokens, out, ws,
                    device_props(dev).num_cus, st);
   if ((lean ? need.lean : need.tile) && lds_loads && e->tiling == CASCADIA_INT4_TILING_MFMA)
     return ffn_tiles(hidden, inter, group, sdt, e, x, x_f32, n_tokens, out, out_bf16, ws, lean,
@@ -1609,7 +1608,7 @@ int moe_forward(const cascadia_int4_moe_layer *L, const cascadia_int4_routing *R
     // gate/up reads its rows through the row map (no copy per assignment)
     const int Tp = cai4::gg_rows_pad((int)T);
     if (e == hipSuccess)
-      e = cai4::gg_prep(2, x, nullptr, nullptr, xg, nullptr, sx, (int)T, Tp, H, G, nullptr, st);
+      e = cai4::gg_prep(2, x, nullptr, xg, nullptr, sx, (int)T, Tp, H, G, st);
     cai4::GgArgs a{};
     a.estride = L->expert_stride;
     a.tiles = chunks;
@@ -1635,7 +1634,6 @@ int moe_forward(const cascadia_int4_moe_layer *L, const cascadia_int4_routing *R
       g.ldy = I;
       g.epi = cai4::GG_SWIGLU_HILO;
       g.seeds_out = si;  // the hot rows' down seeds, from the planes as they are written
-      g.seeds_gw = cai4::gg_group_width(G);
       g.seeds_rp = m.rows_pad;
       e = cai4::gg_grouped(g, m.ws.max_chunks, st);
     }

@@ -1,5 +1,5 @@
-// few.hip -- INT4 weight-only GEMM for 2 .. 32 token rows over MFMA-tiled
-// weights (gfx950): the FFN chain and the projections of a decode batch.
+// few.hip -- INT4 weight-only GEMM for up to 32 token rows over MFMA-tiled
+// weights (gfx950): the two GEMMs of a decode batch's FFN.
 //
 // y[t, r] = sum_g s[r, g] * sum_{c in g} (nibble[r, c] - 8) * x[t, c], the sum of
 // dequant_gemm_int4_multi_auto (kernel_avx512_multi.rs:66-245) and, with the
@@ -10,8 +10,8 @@
 // workgroup per CU, two k-blocks of weights per wave in flight meanwhile).
 // Here activations and weights arrive together: a stage holds two k-blocks of
 // the workgroup's eight weight tiles and of its rows, global -> LDS by buffer
-// loads with an LDS destination, as many stages ahead as LDS holds (64-80 KB of
-// weights in flight per CU from the first microsecond on), one barrier per
+// loads with an LDS destination, as many stages ahead as LDS holds (2 to 4: 32-64
+// KB of weights in flight per CU from the first microsecond on), one barrier per
 // stage.  Eight waves: four by columns (two tiles each: a gate and an up tile
 // with SwiGLU), two by k-block of the stage, added through LDS at the end.
 // K is cut into slices until the workgroups fill the CUs; the reduce kernels of
@@ -41,15 +41,13 @@ struct Few {
   static constexpr int AL = MT * PL;     // 1 KB activation loads per wave and stage
   static constexpr int LOADS = AL + 2 + 1;
   static constexpr int PIECES = 2 * GPK;  // 256-byte pieces of scales: [2 k-blocks][8 tiles][GPK][16]
-  static constexpr int ST = 155 * 1024 / BYTES > 6 ? 6 : 155 * 1024 / BYTES;  // stages
-  static_assert(ST >= 3 && (ST - 2) * LOADS <= 63 && PIECES <= W, "stage");
+  static constexpr int ST = 155 * 1024 / BYTES;  // stages: 3 .. 5
+  static_assert(ST >= 3 && ST <= 5 && (ST - 2) * LOADS <= 63 && PIECES <= W, "stage");
 };
 
 template <int N>
-CAI4_DEV void few_wait(int ahead) {  // uniform: stages that may still be in flight
-  if (ahead >= 4)
-    dma_wait_barrier<4 * N>();
-  else if (ahead == 3)
+CAI4_DEV void few_wait(int ahead) {  // uniform: stages that may still be in flight (ST - 2 at most)
+  if (ahead == 3)
     dma_wait_barrier<3 * N>();
   else if (ahead == 2)
     dma_wait_barrier<2 * N>();
@@ -260,8 +258,6 @@ __global__ __launch_bounds__(512, 2) void few_kernel(GgArgs a) {
           if (n >= a.N) continue;
           if (a.part)
             a.part[((size_t)slice * a.M + t) * a.N + n] = y[i][j][v];
-          else if (a.epi == GG_F32)
-            static_cast<float *>(a.y)[(size_t)t * a.ldy + n] = y[i][j][v];
           else
             static_cast<uint16_t *>(a.y)[(size_t)t * a.ldy + n] = (uint16_t)f32_to_bf16_rne(y[i][j][v]);
         }
@@ -275,11 +271,11 @@ struct FewPlan {
 
 // Slices of K: as many as fill the CUs once, each of at least four k-blocks (an
 // even number: a stage holds two).
-FewPlan few_plan(int N, int K, bool sw, int num_cus, int max_slices) {
+FewPlan few_plan(int N, int K, bool sw, int num_cus) {
   const int KB = K / 128, tiles = (N + (sw ? 63 : 127)) / (sw ? 64 : 128);
   int s = num_cus / tiles;
   if (s > KB / 4) s = KB / 4;
-  if (s > max_slices) s = max_slices;
+  if (s > 64) s = 64;
   if (s < 1 || N % 4) s = 1;
   int kper = (KB + s - 1) / s;
   kper += kper & 1;
@@ -311,24 +307,23 @@ bool few_supported(int M, int N, int K, int G, int tiled) {
   return M >= 1 && M <= kFewMaxRows && N >= 16 && gg_supported(K, G, tiled);
 }
 
-size_t few_workspace(int M, int N, int K, bool sw, int num_cus, int max_slices) {
-  const FewPlan p = few_plan(N, K, sw, num_cus, max_slices);
+size_t few_workspace(int M, int N, int K, bool sw, int num_cus) {
+  const FewPlan p = few_plan(N, K, sw, num_cus);
   return p.nsl > 1 ? (size_t)p.nsl * M * (sw ? 2 * (size_t)N : N) * 4 : 0;
 }
 
-hipError_t few_gemm(GgArgs a, void *ws, int num_cus, hipStream_t st, int max_slices) {
+hipError_t few_gemm(GgArgs a, void *ws, int num_cus, hipStream_t st) {
   const bool sw = a.epi == GG_SWIGLU_HILO;
-  if (a.M < 1 || a.M > kFewMaxRows || (sw && a.hilo)) return hipErrorInvalidValue;
-  const FewPlan p = few_plan(a.N, a.K, sw, num_cus, max_slices);
+  if (a.M < 1 || a.M > kFewMaxRows || sw == (a.hilo != 0) || (!sw && a.epi != GG_BF16))
+    return hipErrorInvalidValue;
+  const FewPlan p = few_plan(a.N, a.K, sw, num_cus);
   a.kper = p.kper;
   a.part = p.nsl > 1 ? static_cast<float *>(ws) : nullptr;
   hipError_t e;
   if (sw)
     e = a.M <= 16 ? few_launch<1, 1, true>(a, p.nsl, st) : few_launch<2, 1, true>(a, p.nsl, st);
-  else if (a.hilo)
-    e = a.M <= 16 ? few_launch<1, 2, false>(a, p.nsl, st) : few_launch<2, 2, false>(a, p.nsl, st);
   else
-    e = a.M <= 16 ? few_launch<1, 1, false>(a, p.nsl, st) : few_launch<2, 1, false>(a, p.nsl, st);
+    e = a.M <= 16 ? few_launch<1, 2, false>(a, p.nsl, st) : few_launch<2, 2, false>(a, p.nsl, st);
   if (e != hipSuccess || p.nsl == 1) return e;
   return gg_reduce_slices(a, p.nsl, st);
 }

@@ -721,18 +721,14 @@ constexpr int kGgPrepPasses = 2;
 
 template <int L>
 __global__ __launch_bounds__(256) void gg_prep_kernel(int mode, const void *src, const void *src2,
-                                                      const int32_t *row_map, uint16_t *out,
-                                                      uint16_t *out2, float *seeds, int rows,
-                                                      int rows_pad, int K,
-                                                      const int32_t *rows_dev) {
+                                                      uint16_t *out, uint16_t *out2, float *seeds,
+                                                      int rows, int rows_pad, int K) {
   constexpr int P = kGgPrepPasses;
   const int lane = threadIdx.x & 63;
   const int r = blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (rows_dev) rows = *rows_dev;
   if (r >= rows) return;  // whole waves; no barriers here
   const int gw = 8 * L;   // columns per seed group
-  size_t srow = (size_t)r;
-  if (mode == 2 && row_map) srow = (size_t)row_map[r];
+  const size_t srow = (size_t)r;
   const int c0 = blockIdx.y * P * 512 + 8 * lane;
   u32x4_t v[P], w[P];  // 8 columns a pass: bf16 hi (and lo), or two halves of f32
 #pragma unroll
@@ -857,21 +853,20 @@ bool gg_supported(int K, int G, int tiled) {
 
 int gg_rows_pad(int rows) { return (rows + 127) / 128 * 128; }
 
-hipError_t gg_prep(int mode, const void *src, const void *src2, const int32_t *row_map,
-                   uint16_t *out, uint16_t *out2, float *seeds, int rows, int rows_pad, int K,
-                   int G, const int32_t *rows_dev, hipStream_t st) {
+hipError_t gg_prep(int mode, const void *src, const void *src2, uint16_t *out, uint16_t *out2,
+                   float *seeds, int rows, int rows_pad, int K, int G, hipStream_t st) {
   if (rows <= 0) return hipSuccess;
   const dim3 grid((rows + 3) / 4, (K + 512 * kGgPrepPasses - 1) / (512 * kGgPrepPasses)), block(256);
   const int gw = gg_group_width(G);
   if (gw == 32)
-    hipLaunchKernelGGL(gg_prep_kernel<4>, grid, block, 0, st, mode, src, src2, row_map, out, out2,
-                       seeds, rows, rows_pad, K, rows_dev);
+    hipLaunchKernelGGL(gg_prep_kernel<4>, grid, block, 0, st, mode, src, src2, out, out2, seeds,
+                       rows, rows_pad, K);
   else if (gw == 64)
-    hipLaunchKernelGGL(gg_prep_kernel<8>, grid, block, 0, st, mode, src, src2, row_map, out, out2,
-                       seeds, rows, rows_pad, K, rows_dev);
+    hipLaunchKernelGGL(gg_prep_kernel<8>, grid, block, 0, st, mode, src, src2, out, out2, seeds,
+                       rows, rows_pad, K);
   else
-    hipLaunchKernelGGL(gg_prep_kernel<16>, grid, block, 0, st, mode, src, src2, row_map, out,
-                       out2, seeds, rows, rows_pad, K, rows_dev);
+    hipLaunchKernelGGL(gg_prep_kernel<16>, grid, block, 0, st, mode, src, src2, out, out2, seeds,
+                       rows, rows_pad, K);
   return hipGetLastError();
 }
 
@@ -937,12 +932,12 @@ hipError_t gg_dense(GgArgs a, int amode, void *ws, int num_cus, hipStream_t st, 
       w += al256((size_t)a.M * a.K * 2);
       uint16_t *lo = reinterpret_cast<uint16_t *>(w);
       w += al256((size_t)a.M * a.K * 2);
-      e = gg_prep(3, a.x, nullptr, nullptr, hi, lo, seeds, a.M, a.rows_pad, a.K, a.G, nullptr, st);
+      e = gg_prep(3, a.x, nullptr, hi, lo, seeds, a.M, a.rows_pad, a.K, a.G, st);
       a.x = hi;
       a.x2 = lo;
     } else {
-      e = gg_prep(a.hilo ? 1 : 0, a.x, a.x2, nullptr, nullptr, nullptr, seeds, a.M, a.rows_pad,
-                  a.K, a.G, nullptr, st);
+      e = gg_prep(a.hilo ? 1 : 0, a.x, a.x2, nullptr, nullptr, seeds, a.M, a.rows_pad, a.K, a.G,
+                  st);
     }
     if (e != hipSuccess) return e;
   } else if (amode == GG_A_F32) {
@@ -971,10 +966,7 @@ hipError_t gg_grouped(const GgArgs &a0, int max_tiles, hipStream_t st) {
   a.part = nullptr;
   if (max_tiles <= 0) return hipSuccess;
   const bool sw = a.epi == GG_SWIGLU_HILO;
-  // the epilogue's seeds: SwiGLU only, groups of one, two or four waves' 32 columns
-  if (a.seeds_out && (!sw || a.seeds_rp <= 0 ||
-                      (a.seeds_gw != 32 && a.seeds_gw != 64 && a.seeds_gw != 128)))
-    return hipErrorInvalidValue;
+  if (a.seeds_out && (!sw || a.seeds_rp <= 0)) return hipErrorInvalidValue;
   // rows through a row map: one bf16 plane, x rows addressable in 31 bits
   if (a.row_map && (a.hilo || a.x_rows <= 0 || (size_t)a.x_rows * a.K * 2 > 0x7FFFFFFFu))
     return hipErrorInvalidValue;

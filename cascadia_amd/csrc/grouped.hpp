@@ -32,10 +32,10 @@ struct GgArgs {
   float *part;   // dense split-K partials [ksplit][M][N] (f32), or null
   int kper;      // k-blocks per K slice (blockIdx.z)
   // SwiGLU only, or null: the seeds of the hi / lo planes the epilogue writes,
-  // for a GEMM that takes them as A: [N / seeds_gw][rows_pad], the zero point's
-  // share of hi + lo over each group of seeds_gw output columns (32, 64 or 128)
+  // for a GEMM that takes them as A: [N / gg_group_width(G)][seeds_rp], the zero
+  // point's share of hi + lo over each group of output columns
   float *seeds_out;
-  int seeds_gw, seeds_rp;  // group width, row stride of seeds_out
+  int seeds_rp;
   // grouped, one bf16 plane only, or null: A row r of the table is x row
   // row_map[r] (x: [x_rows, K], seeds [K / gw][rows_pad] per x row), so the
   // rows need no gathered copy
@@ -53,14 +53,10 @@ bool gg_supported(int K, int G, int tiled);
 // Seeds (and converted activations) of A, one wave per row:
 //   mode 0: bf16 rows x [rows, K] -> seeds;
 //   mode 1: bf16 hi/lo planes x, x2 -> seeds of hi + lo;
-//   mode 2: f32 rows src gathered through row_map (row r = src row row_map[r];
-//           src row r when row_map is null) -> bf16 (RNE) rows into out + seeds;
+//   mode 2: f32 rows src -> bf16 (RNE) rows out + seeds;
 //   mode 3: f32 rows src -> hi/lo planes out / out2 + seeds.
-// rows_dev (device, may be null): the row count, when only the device knows
-// it (rows is then an upper bound).
-hipError_t gg_prep(int mode, const void *src, const void *src2, const int32_t *row_map,
-                   uint16_t *out, uint16_t *out2, float *seeds, int rows, int rows_pad, int K,
-                   int G, const int32_t *rows_dev, hipStream_t st);
+hipError_t gg_prep(int mode, const void *src, const void *src2, uint16_t *out, uint16_t *out2,
+                   float *seeds, int rows, int rows_pad, int K, int G, hipStream_t st);
 
 // Rows of seeds to allocate for `rows` A rows.
 int gg_rows_pad(int rows);
