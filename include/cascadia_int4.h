@@ -264,7 +264,7 @@ int cascadia_int4_expert_forward_device(uint32_t hidden, uint32_t inter, uint32_
  * and split-K partials live in a file-scope device array of
  * CASCADIA_INT4_NOALLOC_SCRATCH_BYTES per GPU, held until the process ends;
  * a call that would need more in any form returns CASCADIA_INT4_ERR_ARG
- * (config 1's Llama-3-8B FFN fits up to 64 tokens), and one whose usual form
+ * (config 1's Llama-3-8B FFN fits up to 16 tokens), and one whose usual form
  * needs more but whose least form fits runs in that form (results within
  * rounding order of the _device entry point's).  Every call on one GPU shares
  * that array, so calls that overlap on one GPU (different streams, or threads)
