@@ -485,14 +485,14 @@ FfnWorkspace ffn_workspace(int dev, uint32_t hidden, uint32_t inter, uint32_t gr
 // a route that begins inside it), and K is cut into no more slices than for lo
 // (the slices' cost grows with the rows, their gain does not).  accepted: more
 // rows than that no call takes.
+uint32_t step_end(uint32_t lo) { return lo <= 64 ? lo : (lo + 31) / 32 * 32; }
+
 template <class Need>
-size_t rows_upto(uint32_t n, size_t accepted, Need need) {
+size_t rows_upto(uint32_t n, size_t accepted, Need need, uint32_t from = 1, size_t most = 0) {
   if (n > accepted) n = (uint32_t)accepted;
-  size_t most = 0;
-  for (size_t lo = 1, hi; lo <= n; lo = hi + 1) {
-    hi = lo <= 64 ? lo : (lo + 31) / 32 * 32;
-    if (hi > n) hi = n;
-    const size_t b = need((uint32_t)lo, (uint32_t)hi);
+  for (uint32_t lo = from, hi; lo <= n; lo = hi + 1) {
+    hi = step_end(lo) < n ? step_end(lo) : n;
+    const size_t b = need(lo, hi);
     if (b > most) most = b;
   }
   return most;
@@ -503,13 +503,54 @@ size_t accepted_rows(uint32_t hidden, uint32_t inter) {
   return 0x7FFFFFFFu / (2 * (size_t)(hidden > inter ? hidden : inter));
 }
 
-// Enough for an FFN of any number of rows up to n, f32 or bf16.
+// Enough for an FFN of any number of rows up to n, f32 or bf16.  The maxima of
+// the whole steps of the last shapes asked for are kept: a program asks once
+// per batch size, 70 us of planning each for 200 rows.
 size_t ffn_workspace_upto(int dev, uint32_t hidden, uint32_t inter, uint32_t group, uint32_t n) {
-  return rows_upto(n, accepted_rows(hidden, inter), [&](uint32_t lo, uint32_t hi) {
+  constexpr int kShapes = 8, kSteps = 64 + 256;
+  struct Shape {
+    int dev;
+    uint32_t hidden, inter, group, tuning, steps, rows;  // steps kept, the last one's rows
+    size_t most[kSteps];
+  };
+  static std::mutex mu;
+  static Shape shapes[kShapes];
+  static int n_shapes = 0;
+  static unsigned oldest = 0;
+  auto need = [&](uint32_t lo, uint32_t hi) {
     const size_t f = ffn_workspace(dev, hidden, inter, group, hi, true, lo).total();
     const size_t b = ffn_workspace(dev, hidden, inter, group, hi, false, lo).total();
     return f > b ? f : b;
-  });
+  };
+  const size_t accepted = accepted_rows(hidden, inter);
+  if (n > accepted) n = (uint32_t)accepted;
+  const uint32_t tuning = cascadia_int4_tuning_generation();
+  std::lock_guard<std::mutex> lk(mu);
+  Shape *s = nullptr;
+  for (int i = 0; i < n_shapes && !s; ++i)
+    if (shapes[i].dev == dev && shapes[i].hidden == hidden && shapes[i].inter == inter &&
+        shapes[i].group == group && shapes[i].tuning == tuning)
+      s = &shapes[i];
+  if (!s) {
+    s = n_shapes < kShapes ? &shapes[n_shapes++] : &shapes[oldest++ % kShapes];
+    s->dev = dev;
+    s->hidden = hidden;
+    s->inter = inter;
+    s->group = group;
+    s->tuning = tuning;
+    s->steps = s->rows = 0;
+  }
+  while (s->steps < kSteps && step_end(s->rows + 1) <= n) {
+    const uint32_t lo = s->rows + 1;
+    s->rows = step_end(lo);
+    const size_t b = need(lo, s->rows), m = s->steps ? s->most[s->steps - 1] : 0;
+    s->most[s->steps++] = b > m ? b : m;
+  }
+  // the whole steps up to n that are kept, then the others
+  uint32_t k = n <= 64 ? n : 64 + (n - 64) / 32;
+  if (k > s->steps) k = s->steps;
+  const uint32_t rows = k <= 64 ? k : 64 + (k - 64) * 32;
+  return rows_upto(n, accepted, need, rows + 1, k ? s->most[k - 1] : 0);
 }
 
 // The expert FFN on the MFMA-tile GEMMs: gate/up with the SwiGLU epilogue
