@@ -276,7 +276,7 @@ FewPlan few_plan(int N, int K, bool sw, int num_cus) {
   int s = num_cus / tiles;
   if (s > KB / 4) s = KB / 4;
   if (s > 64) s = 64;
-  if (s < 1 || N % 4) s = 1;
+  if (s < 1 || N % 4) s = 1;  // (the partials' rows are N apart here)
   int kper = (KB + s - 1) / s;
   kper += kper & 1;
   return FewPlan{(KB + kper - 1) / kper, kper};

@@ -567,8 +567,8 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gg_kernel(GgArgs a) {
       }
     }
   } else if (a.part || a.epi == GG_F32) {
-    float *y = a.part ? a.part + (size_t)blockIdx.z * a.M * a.N : reinterpret_cast<float *>(a.y);
-    const size_t ld = a.part ? a.N : a.ldy;
+    const size_t ld = a.part ? gg_part_ld(a.N) : a.ldy;
+    float *y = a.part ? a.part + (size_t)blockIdx.z * a.M * ld : reinterpret_cast<float *>(a.y);
     if (live) {
 #pragma unroll
       for (int i = 0; i < MT; ++i)
@@ -628,38 +628,40 @@ CAI4_DEV f32x4_t sum_slices(const float *part, size_t stride, size_t i, int nsl)
   return nsl <= 4 ? sum_slices_by<4>(part, stride, i, nsl) : sum_slices_by<8>(part, stride, i, nsl);
 }
 
-// y = sum over the K slices' partials, in slice order; bf16 (RNE) or f32.
+// y = sum over the K slices' partials, in slice order; bf16 (RNE) or f32.  The
+// partials' rows are gg_part_ld(N) apart: a thread's four columns are aligned
+// and in one row whatever N is (those past N are read and not used).
 __global__ __launch_bounds__(256) void gg_reduce_kernel(const float *part, void *y, int M, int N,
                                                         int ldy, int nsl, int out_f32) {
   const size_t i = ((size_t)blockIdx.x * blockDim.x + threadIdx.x) * 4;
-  const size_t n = (size_t)M * N;
+  const uint32_t ld = gg_part_ld(N);
+  const size_t n = (size_t)M * ld;
   if (i >= n) return;  // n is a multiple of 4
   const f32x4_t s = sum_slices(part, n, i, nsl);
-  // N % 4 == 0: the four stay in one row
-  const size_t r = n >> 32 ? i / N : (uint32_t)i / (uint32_t)N, c = i - r * N;
+  const size_t r = n >> 32 ? i / ld : (uint32_t)i / ld;
+  const int c = (int)(i - r * ld);
+  const bool four = c + 4 <= N;
   const size_t o = r * ldy + c;
   if (out_f32) {
     float *yf = reinterpret_cast<float *>(y) + o;
-    if (((uintptr_t)yf & 15) == 0) {
+    if (four && ((uintptr_t)yf & 15) == 0) {
       *reinterpret_cast<f32x4_t *>(yf) = s;
     } else {
-      yf[0] = s.x;
-      yf[1] = s.y;
-      yf[2] = s.z;
-      yf[3] = s.w;
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (c + e < N) yf[e] = s[e];
     }
   } else {
     uint16_t *yb = reinterpret_cast<uint16_t *>(y) + o;
     u32x2_t b;
     b.x = f32_to_bf16_rne(s.x) | (f32_to_bf16_rne(s.y) << 16);
     b.y = f32_to_bf16_rne(s.z) | (f32_to_bf16_rne(s.w) << 16);
-    if (((uintptr_t)yb & 7) == 0) {
+    if (four && ((uintptr_t)yb & 7) == 0) {
       *reinterpret_cast<u32x2_t *>(yb) = b;
     } else {
-      yb[0] = (uint16_t)b.x;
-      yb[1] = (uint16_t)(b.x >> 16);
-      yb[2] = (uint16_t)b.y;
-      yb[3] = (uint16_t)(b.y >> 16);
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (c + e < N) yb[e] = (uint16_t)(b[e >> 1] >> (16 * (e & 1)));
     }
   }
 }
@@ -831,7 +833,7 @@ GgPlan gg_plan(int M, int N, int K, int G, bool two, bool sw, int num_cus, int m
     const long slots = small ? 2L * num_cus : num_cus;
     const double tkb = small ? tkb_small : two ? tkb64x2 : tkb128;
     for (int s = 1; s <= max_slices && s <= 8; ++s) {
-      if (s > 1 && (KB / s < 4 || N % 4)) break;
+      if (s > 1 && KB / s < 4) break;
       const int kper = (KB + s - 1) / s, nsl = (KB + kper - 1) / kper;
       const long rounds = (tiles * nsl + slots - 1) / slots;
       double t = rounds * (kper * tkb + kTile);
@@ -895,7 +897,7 @@ hipError_t gg_reduce_slices(const GgArgs &a, int nsl, hipStream_t st) {
     }
     return hipGetLastError();
   }
-  const size_t n = (size_t)a.M * a.N;
+  const size_t n = (size_t)a.M * gg_part_ld(a.N);
   // small outputs: one wave per workgroup, so that every CU has one
   const unsigned bs = n / 4 >= 1u << 17 ? 256 : 64;
   hipLaunchKernelGGL(gg_reduce_kernel, dim3((unsigned)((n / 4 + bs - 1) / bs)), dim3(bs), 0, st,
@@ -910,7 +912,7 @@ size_t gg_dense_workspace(int M, int N, int K, int G, int amode, int epi, int nu
   size_t b = have_seeds ? 0 : al256((size_t)(K / gg_group_width(G)) * gg_rows_pad(rows) * 4);
   if (amode == GG_A_F32) b += 2 * al256((size_t)rows * K * 2);  // the A planes
   const GgPlan p = gg_plan(M, N, K, G, amode != GG_A_BF16, sw, num_cus, max_slices);
-  return b + (p.nsl > 1 ? (size_t)p.nsl * rows * (sw ? 2 * (size_t)N : N) * 4 : 0);
+  return b + (p.nsl > 1 ? (size_t)p.nsl * rows * (sw ? 2 * (size_t)N : gg_part_ld(N)) * 4 : 0);
 }
 
 hipError_t gg_dense(GgArgs a, int amode, void *ws, int num_cus, hipStream_t st, int max_slices) {

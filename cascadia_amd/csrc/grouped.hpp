@@ -10,6 +10,9 @@
 
 namespace cai4 {
 
+// Columns between two rows of the slices' partials: N up to the next multiple of four.
+__host__ __device__ constexpr int gg_part_ld(int N) { return (N + 3) / 4 * 4; }
+
 // Output of a GEMM: f32, bf16 (RNE), or -- for a gate/up pair -- SwiGLU as the
 // two bf16 planes hi = bf16(h), lo = bf16(h - hi) of h = silu(gate) * up.
 enum GgEpi { GG_F32 = 0, GG_BF16 = 1, GG_SWIGLU_HILO = 2 };
@@ -29,7 +32,7 @@ struct GgArgs {
   int N, K, G, sdt, ldy, rows_pad;
   int hilo;      // A has two bf16 planes (x + x2)
   int epi;       // GgEpi
-  float *part;   // dense split-K partials [ksplit][M][N] (f32), or null
+  float *part;   // dense split-K partials [ksplit][M][gg_part_ld(N)] (f32), or null
   int kper;      // k-blocks per K slice (blockIdx.z)
   // SwiGLU only, or null: the seeds of the hi / lo planes the epilogue writes,
   // for a GEMM that takes them as A: [N / gg_group_width(G)][seeds_rp], the zero

@@ -136,6 +136,37 @@ def test_gemm_f32_tiles_lose_no_precision(cl, tuning, g, mean):
     assert err["tiles"] <= err["skinny"], err
 
 
+@pytest.mark.parametrize("n", [1001, 1002, 1003, 4097])
+@pytest.mark.parametrize("M,g", [(64, 128), (77, 32)])
+def test_gemm_split_any_columns(cl, tuning, n, M, g):
+    """K is cut into slices whatever the columns (few tiles, long K): f32 and
+    bf16 rows, f32 and bf16 outputs, nothing written past the last column."""
+    k = 8192
+    tuning("CASCADIA_INT4_F32_TILE_TOKENS", "17")
+    packed = cl.fill_bytes(torch.empty(n * k // 2, dtype=torch.uint8, device="cuda"), 17, 1)
+    scales = cl.fill_scales(torch.empty(n * (k // g), dtype=torch.int16, device="cuda"), 17, 2)
+    scales = scales.view(torch.uint8)
+    pt, st = cl.tile_weights(packed, scales, n, k, g)
+    x = cl.fill_normal(torch.empty((M, k), device="cuda"), 17, 3)
+    W = cl.debug_dequant(packed, scales, n, k, g, F16).double()
+    # the partials of at least two slices, beside the f32 rows' planes
+    assert cl.gemm_workspace_bytes(n, k, M, True, g, cl.TILING_MFMA) >= 4 * M * k + 8 * M * n
+    for dt in (torch.float32, torch.bfloat16):
+        xd = x.to(dt)
+        want = (xd.double() @ W.T).cpu().numpy()
+        opts = dict(group_size=g, scale_dtype=F16, tiling=cl.TILING_MFMA)
+        buf = torch.full((M * n + 8,), 7.0, device="cuda")
+        cl.dequant_gemm_int4_multi_auto(pt, st, xd, n, k, M, buf[:M * n], **opts)
+        assert rel_l2(host(buf[:M * n]).reshape(M, n), want) <= 1e-5
+        assert bool((buf[M * n:] == 7.0).all())
+        if dt == torch.bfloat16:
+            out = torch.full((M * n + 8,), 7.0, dtype=dt, device="cuda")
+            cl.gemm_int4_bf16(pt, st, xd, n, k, M, out[:M * n], **opts)
+            # one rounding to 8 bits: at most 2^-9 of each value
+            assert rel_l2(host(out[:M * n].float()).reshape(M, n), want) <= 2 ** -9
+            assert bool((out[M * n:] == 7.0).all())
+
+
 def shifted(t):
     """The same bytes two past a 16-byte boundary."""
     s = torch.empty(t.numel() + 16, dtype=torch.uint8, device="cuda")[2:2 + t.numel()]
