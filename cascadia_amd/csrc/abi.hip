@@ -1196,7 +1196,7 @@ int run_prefill(const cascadia_int4_layout *L, const uint8_t *packed, const uint
 bool fall_back(int rc) { return rc == CASCADIA_INT4_ERR_ARG || rc == CASCADIA_INT4_ERR_NOMEM; }
 
 // Many rows over MFMA-tiled weights: the tile GEMM (grouped.hip), for bf16 rows
-// from 64 on, else where it pays (tiles_pay).
+// from 64 on, else where it pays (tiles_pay, and not skinny_streams).
 bool prefill_shape(const cascadia_int4_layout *L, uint32_t seq, bool x_f32) {
   if (!L->tiling || L->n_rows < 16 ||
       !cai4::gg_supported((int)L->k_cols, (int)L->group_size, 1))
@@ -1207,6 +1207,41 @@ bool prefill_shape(const cascadia_int4_layout *L, uint32_t seq, bool x_f32) {
   const size_t bytes = (size_t)L->n_rows * L->k_cols / 2;
   if (x_f32) return tiles_pay(seq, 32, bytes, 17, (size_t)22 << 20);
   return seq >= 64 || tiles_pay(seq, 64, bytes, 33, (size_t)22 << 20);
+}
+
+// Whether the skinny kernel is the faster one all the same, where its plan runs
+// one round of workgroups over the CUs, each with its whole k-range in LDS: a
+// stream of the weights with little beside it.  Measured (us, tiles / skinny):
+//   f32  G128  4096 x 14336 17 rows 28.4 / 22.0, 20 (no such plan): 28.9 / 36.7
+//              4096 x 11264 24 rows 25.6 / 19.7, 32 (none): 26.4 / 34.3
+//              5000 x 10240 17: 24.4 / 21.7; 6144 x 8192 20: 21.6 / 21.0
+//              14336 x 1792 33: 18.2 / 19.9, 40: 21.2 / 20.0, 64: 23.8 / 20.8
+//              8192 x 4096  33: 19.2 / 21.0, 40: 19.9 / 20.9, 64: 24.0 / 22.6
+//              4096 x 4096  97: 21.2 / 22.4, 128: 24.1 / 23.0
+//              32768 x 1536 17: 20.2 / 15.5; 65536 x 768 17: 16.7 / 14.5
+//        G32   4096 x 14336 17: 31.9 / 26.6; 4096 x 11264 24: 28.2 / 22.6
+//              6144 x 8192  17: 23.3 / 25.0; 7168 x 7168 17: 22.4 / 25.9
+//              32768 x 1536 17: 21.6 / 19.2, 24: 22.3 / 22.8
+//   bf16 G128  32768 x 1536 33: 20.0 / 16.2, 40: 20.1 / 17.3, 48: 20.8 / 20.5
+//              65536 x 768  33: 15.0 / 15.0; 4096 x 11264 33: 18.4 / 19.0
+// So: groups of 128 and more, in the upper half of a pass's rows (f32), or over
+// short rows, up to 40 (bf16); smaller groups, whose scales cost the skinny
+// kernel more, where one f32 pass splits K not at all or six ways and more.
+bool skinny_streams(const cascadia_int4_layout *L, uint32_t seq, bool x_f32, int dev) {
+  if (seq >= (x_f32 ? 129u : 64u)) return false;
+  const int env = cai4::tuning_env(
+      x_f32 ? "CASCADIA_INT4_F32_TILE_TOKENS" : "CASCADIA_INT4_BF16_TILE_TOKENS", 0);
+  if (env > 0) return false;
+  const cai4::SkinnyDevice d = device_props(dev);
+  const cai4::SkinnyPlan p =
+      cai4::skinny_plan((int)L->n_rows, (int)L->k_cols, (int)L->group_size, (int)seq,
+                        x_f32 ? cai4::A_XF32 : cai4::A_BF16, cai4::EPI_F32, d);
+  const long wgs = (long)p.row_blocks * p.m_chunks * p.ksplit;
+  if (p.kslice < p.kper || wgs > d.num_cus || wgs < (long)d.num_cus * 7 / 8) return false;
+  const bool wide = L->group_size % 128 == 0;
+  if (!x_f32) return wide && p.ksplit <= 2 && seq <= 40;
+  if (wide) return (seq - 1) % 32 >= 15;
+  return seq <= 32 && (p.ksplit == 1 || p.ksplit >= 6);
 }
 
 // seq rows through the tile GEMM, the skinny kernel or the GEMV.  Without a
@@ -1223,14 +1258,17 @@ int gemm_common(const cascadia_int4_layout *L, const uint8_t *packed, const uint
   if (!aligned(x, 16) || !aligned(y, y_f32 ? 4 : 2) || (workspace && !aligned(workspace, 16)))
     return CASCADIA_INT4_ERR_ARG;
   const int amode = x_f32 ? cai4::A_XF32 : cai4::A_BF16;
-  const bool tiles = prefill_shape(L, seq, x_f32) && lds_loads_ok(scales);
+  int dev = 0;
+  bool tiles = prefill_shape(L, seq, x_f32) && lds_loads_ok(scales);
+  if (tiles) {
+    if (int rc = current_device(&dev)) return rc;
+    tiles = !skinny_streams(L, seq, x_f32, dev);
+  }
   const bool tiles_only = tiles && !x_f32 && seq >= 64;
   if (tiles && (tiles_only || act_fits((int)seq, (int)L->k_cols, amode)) &&
       (tiles_only || workspace || !capturing(st))) {
     size_t recorded = ~(size_t)0;
     if (!tiles_only && !workspace) {  // recorded, it is the skinny kernel's
-      int dev;
-      if (int rc = current_device(&dev)) return rc;
       recorded = cai4::skinny_plan((int)L->n_rows, (int)L->k_cols, (int)L->group_size, (int)seq,
                                    amode, cai4::EPI_F32, device_props(dev))
                      .partial_bytes;

@@ -60,6 +60,34 @@ def test_ffn_few_rows_by_default(cl, orc, tuning, M, few):
     assert_bf16_close(outs[0], orc.cpu_expert_forward(xb, M, flat, h, i, g, F16), f"few M{M}")
 
 
+@pytest.mark.parametrize("x_f32,M,n,k,g,tiles", [
+    # where the skinny kernel's plan is one round of workgroups with all of K in
+    # LDS, and the next rows or shapes, where it is not or the tiles are faster
+    (True, 24, 4096, 11264, 128, False), (True, 32, 4096, 11264, 128, True),
+    (True, 17, 4096, 11264, 32, False), (True, 17, 6144, 8192, 32, True),
+    (True, 16, 7168, 8192, 128, False), (True, 17, 7168, 8192, 128, True),
+    (True, 40, 8192, 4096, 128, True), (True, 64, 8192, 4096, 128, False),
+    (False, 40, 32768, 1536, 128, False), (False, 48, 32768, 1536, 128, True)])
+def test_gemm_route_by_default(cl, tuning, x_f32, M, n, k, g, tiles):
+    """The route that a GEMM of few rows takes without a variable: the forced
+    route's result, bit for bit, and not the other's."""
+    packed = cl.fill_bytes(torch.empty(n * k // 2, dtype=torch.uint8, device="cuda"), 16, 1)
+    scales = cl.fill_scales(torch.empty(n * (k // g), dtype=torch.int16, device="cuda"), 16, 2)
+    pt, st = cl.tile_weights(packed, scales.view(torch.uint8), n, k, g)
+    x = cl.fill_normal(torch.empty((M, k), dtype=torch.float32 if x_f32 else torch.bfloat16,
+                                   device="cuda"), 16, 3)
+    var = "CASCADIA_INT4_F32_TILE_TOKENS" if x_f32 else "CASCADIA_INT4_BF16_TILE_TOKENS"
+    ys = {}
+    for route, rows in (("default", None), ("tiles", "2"), ("skinny", "100000")):
+        if rows:
+            tuning(var, rows)
+        y = ys[route] = torch.empty((M, n), device="cuda")
+        cl.dequant_gemm_int4_multi_auto(pt, st, x, n, k, M, y, group_size=g, scale_dtype=F16,
+                                        tiling=cl.TILING_MFMA)
+    assert not torch.equal(ys["tiles"], ys["skinny"])
+    assert torch.equal(ys["default"], ys["tiles" if tiles else "skinny"])
+
+
 @pytest.mark.parametrize("h,i,g,M,form", [(1536, 10240, 32, 70, "skinny"),
                                           (1024, 1024, 32, 512, "tiles")])
 def test_noalloc_least_form(cl, orc, tuning, h, i, g, M, form):
