@@ -820,24 +820,32 @@ struct GgPlan {
 // prologue and epilogue, and the reduce launch with its partials written and
 // read.  Slices of at least four k-blocks (the pipeline's depth), at most
 // eight.  max_slices 1: no partials (a workspace that cannot grow).
+// A small tile alone on its CU takes 0.6 of the time per k-block of two, and a
+// split of two planes 1.5 us more than its reduce: without the two, short K was
+// split to its loss (163 x 10703 x 1536, G 32: 26.5 us in three slices of large
+// tiles, 21.0 in one of small ones; 384 x 2431 x 1152 of f32 rows 24.8 / 22.7).
+// Over 92 shapes of 64-2048 bf16 rows with every plan measured, the one chosen
+// is 2.4 % behind the best on average; of 33-500 f32 rows, 36 shapes, 1.1 %.
 GgPlan gg_plan(int M, int N, int K, int G, bool two, bool sw, int num_cus, int max_slices) {
   const int KB = K / 128, ncol = sw ? 2 * N : N;
   const double tkb128 = G == 32 ? 2.4 : G == 64 ? 1.9 : 1.5;
   const double tkb64x2 = G == 32 ? 1.6 : 1.4, tkb_small = G == 32 ? 1.8 : 1.25;
-  constexpr double kTile = 6.0, kReduce = 3.0, kBytesPerUs = 1.2e7;
+  constexpr double kTile = 6.0, kTileSmall = 4.5, kAlone = 0.6, kBytesPerUs = 1.2e7;
+  const double reduce = two && !sw ? 4.5 : 3.0;
   GgPlan best{false, 1, KB};
   double best_t = -1.0;
   for (int small = 0; small < (two || sw ? 1 : 2); ++small) {
     const int bm = small || two ? 64 : 128, bn = small ? 128 : sw ? 128 : 256;
     const long tiles = (long)((N + bn - 1) / bn) * ((M + bm - 1) / bm);
     const long slots = small ? 2L * num_cus : num_cus;
-    const double tkb = small ? tkb_small : two ? tkb64x2 : tkb128;
     for (int s = 1; s <= max_slices && s <= 8; ++s) {
       if (s > 1 && KB / s < 4) break;
       const int kper = (KB + s - 1) / s, nsl = (KB + kper - 1) / kper;
       const long rounds = (tiles * nsl + slots - 1) / slots;
-      double t = rounds * (kper * tkb + kTile);
-      if (nsl > 1) t += kReduce + (double)nsl * M * ncol * 8.0 / kBytesPerUs;
+      const double tkb = !small ? (two ? tkb64x2 : tkb128)
+                         : tiles * nsl <= num_cus ? kAlone * tkb_small : tkb_small;
+      double t = rounds * (kper * tkb + (small ? kTileSmall : kTile));
+      if (nsl > 1) t += reduce + (double)nsl * M * ncol * 8.0 / kBytesPerUs;
       if (best_t < 0 || t < best_t) {
         best_t = t;
         best = GgPlan{small != 0, nsl, kper};
