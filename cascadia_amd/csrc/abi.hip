@@ -1419,20 +1419,32 @@ size_t moe_workspace_upto(int dev, const cascadia_int4_moe_layer *L, uint32_t to
   const int k = (int)top_k;
   const bool mfma = L->tiling == CASCADIA_INT4_TILING_MFMA;
   size_t part = 0;
-  int seen[2][2] = {{-1, -1}, {-1, -1}};  // the last chunk rows and chunks planned for
-  for (uint32_t t = 1; t <= T; ++t)
-    for (int given = 0; given < 2; ++given) {
-      const int C = moe_tiles(L, top_k, t, false)
+  auto plan = [&](int C, int maxc) {
+    for (const cai4::SkinnyPlan &p :
+         {cai4::skinny_plan_grouped(I, H, G, C, maxc, cai4::A_GATHER, cai4::EPI_SWIGLU_HILO, d),
+          cai4::skinny_plan_grouped(H, I, G, C, maxc, cai4::A_HILO, cai4::EPI_BF16, d)})
+      if (p.partial_bytes > part) part = p.partial_bytes;
+  };
+  // up to 32 tokens the chunk size each count takes, from there on the largest
+  // (moe_chunk_rows) or, beside tiles, 16 rows
+  for (int given = 0; given < 2; ++given) {
+    int C = 0, last = 0;
+    for (uint32_t t = 1; t <= T && t <= 32; ++t) {
+      const int c = moe_tiles(L, top_k, t, false)
                         ? 16
                         : cai4::moe_chunk_rows((int)t, given ? (int)t * k : (int)t, mfma);
-      const int maxc = cai4::moe_max_chunks((int)t, E, k, C);
-      if (seen[given][0] == C && seen[given][1] == maxc) continue;
-      seen[given][0] = C;
-      seen[given][1] = maxc;
-      for (const cai4::SkinnyPlan &p :
-           {cai4::skinny_plan_grouped(I, H, G, C, maxc, cai4::A_GATHER, cai4::EPI_SWIGLU_HILO, d),
-            cai4::skinny_plan_grouped(H, I, G, C, maxc, cai4::A_HILO, cai4::EPI_BF16, d)})
-        if (p.partial_bytes > part) part = p.partial_bytes;
+      const int m = cai4::moe_max_chunks((int)t, E, k, c);
+      if (c != C || m != last) plan(c, m);
+      C = c;
+      last = m;
+    }
+  }
+  for (const int C : {cai4::moe_chunk_rows(64, 64, mfma), 16})
+    for (uint32_t t = 33, last = 0; t <= T; ++t) {
+      const uint32_t m = (uint32_t)cai4::moe_max_chunks((int)t, E, k, C);
+      // (from a chunk per CU on, K is split the same way: the last is the most)
+      if (m != last && (m < (uint32_t)d.num_cus || t == T)) plan(C, (int)m);
+      last = m < (uint32_t)d.num_cus ? m : 0;
     }
   size_t sh = 0, sh_ws = 0;
   if (has_shared(L)) {
