@@ -54,7 +54,8 @@
 // Measured (M 2048, N 14336, K 4096, G 128): 264 -> 230 us against the
 // 16x16x32 kernel with block phases (3600 -> 2900 cycles per k-block; the tile
 // through LDS in 16-byte stores, 14.5k cycles of 2-byte stores before); 1024
-// tokens over 384 experts, G 32: 2.50 -> 2.07 ms a layer.
+// tokens over 384 experts, G 32: 2.39 -> 1.98 ms a layer (with the other changes
+// to its tiles' rules).
 #include "grouped.hpp"
 #include "int4_common.hpp"
 #include "lds_dma.hpp"
@@ -621,9 +622,11 @@ CAI4_DEV f32x4_t sum_slices_by(const float *part, size_t stride, size_t i, int n
   }
   return s;
 }
-// Loads past the last slice repeat it, so few slices take the narrow form: with
-// eight-wide loads and 64-thread blocks, four slices of 512 x 4096 took 7.04 us,
-// so 6.60; eight slices of 16 x 4096 4.56 -> 3.7-4.6.
+// Loads past the last slice repeat it, so few slices take the narrow form.  Back
+// to back (us, four / eight wide, bf16 out): 3 slices of 333 x 4096 2.9 / 3.5, 4 of
+// 200 x 7168 2.9 / 3.6, 4 of 512 x 4096 4.1 / 4.8, 2 of 1024 x 4096 6.3 / 7.3; up to
+// 100 x 4096 both at the launch floor (2.4); eight slices 2.40 / 2.44 (16 x 4096),
+// 11.8 / 12.6 (512 x 4096): there the order of the loads matters little.
 CAI4_DEV f32x4_t sum_slices(const float *part, size_t stride, size_t i, int nsl) {
   return nsl <= 4 ? sum_slices_by<4>(part, stride, i, nsl) : sum_slices_by<8>(part, stride, i, nsl);
 }
@@ -906,7 +909,9 @@ hipError_t gg_reduce_slices(const GgArgs &a, int nsl, hipStream_t st) {
     return hipGetLastError();
   }
   const size_t n = (size_t)a.M * gg_part_ld(a.N);
-  // small outputs: one wave per workgroup, so that every CU has one
+  // small outputs: one wave per workgroup, so that every CU has one (16 x 4096 is
+  // 64 workgroups of 256).  Back to back the two sizes are within 1 % up to 100 x
+  // 4096, 4 % at 1024 x 7168 either way: the line is not sharp.
   const unsigned bs = n / 4 >= 1u << 17 ? 256 : 64;
   hipLaunchKernelGGL(gg_reduce_kernel, dim3((unsigned)((n / 4 + bs - 1) / bs)), dim3(bs), 0, st,
                      a.part, a.y, a.M, a.N, a.ldy, nsl, a.epi == GG_F32 ? 1 : 0);

@@ -15,8 +15,9 @@
 // 2b (low) and 2b+1 (high); the tiled byte b holds columns b (low) and b+4
 // (high), so that the MFMA decode (two masks, one shift, four byte permutes)
 // yields the dword's 8 columns in natural order and the activations need no
-// re-ordering.  The nibble codes and scale bits are moved, never changed, so
-// every kernel computes bit-identical results from either layout.
+// re-ordering.  The nibble codes and scale bits are moved, never changed: a
+// kernel that takes both layouts computes bit-identical results from either
+// (grouped.hip, few.hip and the one-token GEMV take the tiled one only).
 //
 // Groups of fewer than 128 columns (G not a multiple of 128): every 32-column
 // MFMA step must cover whole groups, so its lanes' dwords must be the block's

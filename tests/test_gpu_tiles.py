@@ -208,9 +208,10 @@ def test_scales_aligned_to_two_bytes(cl, tuning, g):
 
 
 def test_gemm_f32_capture(cl, orc):
-    """A stream capture cannot grow the library's workspace: the f32 GEMM of a
-    shape not seen before is recorded all the same (without the tile route if
-    need be), and every replay gives the eager result."""
+    """An f32 GEMM without a workspace, of a shape not seen before, is recorded in
+    the skinny kernel's form (a process whose first call is recorded:
+    test_recorded_forms_in_a_fresh_process); replays and eager calls between
+    them, on the tile route, are both within the bar."""
     n, k, g, M = 3000, 4096, 128, 333
     packed = orc.fill_bytes(5, 5, n * k // 2)
     scales = orc.fill_scales(5, 6, n * (k // g), F16).view(np.uint8).copy()
