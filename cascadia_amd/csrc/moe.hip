@@ -50,19 +50,24 @@ int moe_chunk_rows(int T, int per_expert_max, bool gemv_rows) {
   return per_expert_max < c ? per_expert_max : c;
 }
 
-// From 512 tokens on, or where the experts' mean is 36 rows and more.  Measured
+// From 512 tokens on, or from 192 where the experts' mean is 40 rows and more.
+// Measured
 // (us per layer: skinny chunks only / tiles; hidden 3,584, inter 1,408, top 8):
 //   60 experts G128   200 tokens even 228 / 245, Zipf 246 / 218; 256: 297 / 264,
 //                     284 / 243; 300: 326 / 266, 317 / 285; 400: 422 / 291, 407 / 285
 //   60 experts G32    256 tokens 364 / 367, 350 / 320; 400: 508 / 355, 490 / 358
 //   16 experts G128   128 tokens 143 / 105, 139 / 152; 192: 198 / 109, 195 / 110
 //   128 experts G128  400 tokens 470 / 528, 424 / 336; 512: 547 / 522, 529 / 374
+// Of 2,259 drawn layers of 192-511 tokens with a mean of 40 and more, one is over
+// 4 % slower on tiles and the mean is 0.69 of the time; of 69 with even routing
+// and a mean of 36-39, where about half the experts fall short of a tile's rows,
+// 12 % were (60 experts, 287 tokens, 3200 x 768, G128: 173 / 204).
 // (128-256 tokens over 384 experts, Zipf-skewed, would gain 15 %, but the same
 // sizes with even routing lose 5 % to the second set of launches.)
 bool moe_tiles_pay(int T, int E, int top_k, bool lean) {
   const int n = tuning_env("CASCADIA_INT4_MOE_TILE_TOKENS", 0);
   if (n > 0) return T >= n;
-  return T >= 512 || (!lean && T >= 192 && (int64_t)T * top_k >= (int64_t)36 * E);
+  return T >= 512 || (!lean && T >= 192 && (int64_t)T * top_k >= (int64_t)40 * E);
 }
 
 // Rows from which an expert is worth a 128-row tile rather than 16-row chunks:

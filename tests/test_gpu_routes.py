@@ -112,6 +112,30 @@ def test_noalloc_least_form(cl, orc, tuning, h, i, g, M, form):
         assert np.array_equal(host(out).view(np.uint16).reshape(M, h), got)
 
 
+@pytest.mark.parametrize("T,tiles", [(191, False), (199, False), (200, True)])
+def test_moe_route_by_default(cl, tuning, T, tiles):
+    """From 192 tokens a layer runs on tiles where the experts' mean is 40 rows
+    and more: the forced route's result, bit for bit, and not the other's."""
+    E, top, h, i, g = 40, 8, 512, 256, 128
+    stride = (cl.expert_bytes(h, i, g) + 255) // 256 * 256
+    blobs = cl.fill_bytes(torch.empty(stride * E, dtype=torch.uint8, device="cuda"), 18, 1)
+    for e in range(E):
+        W = cl.ExpertWeights(blobs[e * stride:e * stride + cl.expert_bytes(h, i, g)], h, i, g, F16)
+        for t in W.slices()[1::2]:
+            cl.fill_scales(t.view(torch.int16), 18, 2)
+    ex = cl.MoEExperts.from_crate(blobs, E, h, i, g, F16, stride)
+    x = cl.fill_normal(torch.empty((T, h), device="cuda"), 18, 3)
+    logits = cl.fill_normal(torch.empty((T, E), device="cuda"), 18, 4)
+    out = {}
+    for route, tokens in (("default", None), ("tiles", "2"), ("skinny", "100000")):
+        if tokens:
+            tuning("CASCADIA_INT4_MOE_TILE_TOKENS", tokens)
+        out[route] = torch.empty_like(x)
+        cl.moe_forward(ex, x, out[route], top_k=top, logits=logits)
+    assert not torch.equal(out["tiles"], out["skinny"])
+    assert torch.equal(out["default"], out["tiles" if tiles else "skinny"])
+
+
 SPECIAL = {3: float("nan"), 20: float("inf"), 40: float("-inf"), 63: 3.4028234663852886e38}
 
 
