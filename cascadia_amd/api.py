@@ -43,6 +43,11 @@ def _stream() -> int:
     return _raw_stream(_cur_device())
 
 
+def _device() -> int:
+    """The current device's index (where a device tensor is at hand)."""
+    return torch.cuda.current_device() if _cur_device is None else _cur_device()
+
+
 def _nbytes(t: torch.Tensor) -> int:
     return t.nbytes
 
@@ -68,7 +73,7 @@ def _workspace_ptr(workspace, fn, *dims) -> int:
     if workspace is None:
         return 0
     _dev(workspace, "workspace")
-    need = _need(fn, lib().cascadia_int4_tuning_generation(), torch.cuda.current_device(),
+    need = _need(fn, lib().cascadia_int4_tuning_generation(), _device(),
                  *map(int, dims))
     if workspace.nbytes < need:
         raise ValueError(f"workspace has {workspace.nbytes} bytes, the call needs {need}")
@@ -324,7 +329,7 @@ def _gemm_ws(L, packed, scale_bits, xs, seq, ys, workspace, n_rows, k_cols, grou
     """A GEMM over a caller's workspace."""
     _dev(workspace, "workspace")
     x_f32 = xs.dtype == torch.float32
-    need = _gemm_need(lib().cascadia_int4_tuning_generation(), torch.cuda.current_device(),
+    need = _gemm_need(lib().cascadia_int4_tuning_generation(), _device(),
                       *map(int, (n_rows, k_cols, seq, x_f32, group_size, tiling)))
     if workspace.nbytes < need:
         raise ValueError(f"workspace has {workspace.nbytes} bytes, the call needs {need}")
@@ -956,7 +961,7 @@ def moe_forward(experts: MoEExperts, x, out, *, top_k: int, logits=None, bias=No
     ws = 0
     if workspace is not None:
         ws = _dev(workspace, "workspace").data_ptr()
-        need = _moe_need(lib().cascadia_int4_tuning_generation(), torch.cuda.current_device(),
+        need = _moe_need(lib().cascadia_int4_tuning_generation(), _device(),
                          H, experts.inter, experts.group_size, experts.scale_dtype, experts.tiling,
                          experts.n_experts, experts.shared and experts.shared.inter,
                          experts.shared and experts.shared.tiling, top_k, T)
